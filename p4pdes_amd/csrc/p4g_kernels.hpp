@@ -2829,334 +2829,6 @@ k_ilu27_plane(SorOp o, const double* __restrict__ u, int p, int backward, const 
     z[q] = T(s / uq);
 }
 
-// One directional sweep of PETSc's SOR (omega 1, zero initial guess) on a
-// 2D 27-plane level (planes 9..17), as strips of 64 rows, one wave each.
-// Lane r owns row j of its strip and at step t takes the point c = t - 2r
-// along its row (sweep order), so the row below (forward) or above
-// (backward) is one lane over and two steps ahead: its three values reach
-// lane r by shuffles of each lane's last three results.  Lane 0 takes that
-// row from the previous strip through global memory, after that strip's
-// last lane has published (release) how many points of its row are done;
-// a strip starts SOR9_SLACK points behind, so in steady state it rarely
-// polls.  The arithmetic is k_sor_plane's: forward x = (b - sum over
-// c = 9..12 of a_c x_c) / a_13; backward the same over c = 9..12, 14..17,
-// the lower neighbours holding forward values; a null row stays zero.
-// flag: per strip, base + points done (bases grow from sweep to sweep); a
-// wait longer than spin_limit polls sets *err and ends the waiting (no
-// hang), and a launch that finds *err already set waits for nothing: after
-// a stall every later sweep runs through at once until the host, which
-// checks *err after each linear solve, stops the solve.  need_extra is added
-// to every wait's target (0; the host's stall test sets a target no strip
-// reaches, so that every wait gives up after spin_limit polls).
-constexpr int SOR9_SLACK = 64;
-
-// lane i receives lane i-1's value (DPP wave_shr:1; lane 0 keeps its own)
-__device__ __forceinline__ double wave_shr1(double v) {
-    const long long b = __double_as_longlong(v);
-    const int lo = (int)(b & 0xffffffffLL), hi = (int)(b >> 32);
-    const int rlo = __builtin_amdgcn_update_dpp(lo, lo, 0x138, 0xf, 0xf, false);
-    const int rhi = __builtin_amdgcn_update_dpp(hi, hi, 0x138, 0xf, 0xf, false);
-    return __longlong_as_double(((long long)rhi << 32) | (unsigned int)rlo);
-}
-
-__device__ __forceinline__ double ld_agent(const double* p) {
-    const unsigned long long v =
-        __hip_atomic_load((const unsigned long long*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return __longlong_as_double((long long)v);
-}
-
-// the per-point record of k_sor9_strips: the 2D planes c = 9..17 with the
-// diagonal replaced by its reciprocal (0 for a null row), and a pad
-__global__ void __launch_bounds__(256)
-k_sor9_pack(long n, const double* __restrict__ g, double* __restrict__ pk) {
-    for (long q = blockIdx.x * 256L + threadIdx.x; q < n; q += (long)gridDim.x * 256L) {
-        double* o = pk + q * 10;
-#pragma unroll
-        for (int c = 0; c < 9; ++c) o[c] = g[(long)(9 + c) * n + q];
-        const double dq = g[13 * n + q];
-        o[4] = dq != 0.0 ? 1.0 / dq : 0.0;
-        o[9] = dq;
-    }
-}
-
-// the operands of one step of k_sor9_strips, loaded SOR9_AHEAD steps early
-struct Sor9Ops {
-    double b, a[10], x[4];
-};
-constexpr int SOR9_AHEAD = 4;
-
-__global__ void __launch_bounds__(64)
-k_sor9_strips(int mx, int my, const double* __restrict__ pk, const double* __restrict__ b, double* x,
-              unsigned long long* flag, unsigned long long base, int backward, int* err, long spin_limit,
-              unsigned long long need_extra) {
-    const int s = blockIdx.x, r = threadIdx.x;
-    const int row0 = 64 * s;
-    const int rows = min(64, my - row0);
-    const int j = backward ? my - 1 - (row0 + r) : row0 + r;
-    const bool live = r < rows;
-    const bool hs = j > 0, hn = j + 1 < my;
-    const int nsteps = mx + 2 * (rows - 1);
-    // the previous strip's last row, copied into an LDS ring by the wave in
-    // coalesced batches once that strip has published it (lane 0's row
-    // neighbour); positions are along the sweep: p -> column p or mx-1-p
-    __shared__ double ring[256];
-    const int jn = backward ? my - row0 : row0 - 1;   // lane 0's neighbour row (s > 0), the same for all lanes
-    int copied = 0;                                    // positions in the ring (wave-uniform)
-    bool dead = __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
-    double h1 = 0.0, h2 = 0.0, h3 = 0.0, xo = 0.0;
-    Sor9Ops pf[SOR9_AHEAD];   // a ring of prefetched operands, indexed by step mod SOR9_AHEAD
-    auto fetch = [&](int t, Sor9Ops& o) {
-        const int c = t - 2 * r;
-        if (!(live && c >= 0 && c < mx)) return;
-        const int i = backward ? mx - 1 - c : c;
-        const long q = (long)j * mx + i;
-        o.b = b[q];
-        const double* rec = pk + q * 10;
-#pragma unroll
-        for (int k = 0; k < 10; ++k) o.a[k] = rec[k];
-        if (backward) {   // forward values below and to the left
-            o.x[0] = (hs && i > 0) ? x[q - mx - 1] : 0.0;
-            o.x[1] = hs ? x[q - mx] : 0.0;
-            o.x[2] = (hs && i + 1 < mx) ? x[q - mx + 1] : 0.0;
-            o.x[3] = i > 0 ? x[q - 1] : 0.0;
-        }
-    };
-    auto step = [&](int t, Sor9Ops& cur) {
-        // lane 0 is at position t: it needs positions t-1..t+1 of the neighbour row
-        if (s > 0 && t < mx && copied < min(t + 2, mx)) {   // uniform
-            unsigned long long kn = 0;
-            if (r == 0) {
-                const unsigned long long need =
-                    base + (unsigned long long)min(t == 0 ? SOR9_SLACK : t + 2, mx) + need_extra;
-                long spins = 0;
-                // relaxed polls (an acquire per poll would invalidate the
-                // cache every time), one acquire fence once the count is there
-                while (!dead && (kn = __hip_atomic_load(flag + s - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) < need) {
-                    if (++spins > spin_limit) {
-                        atomicExch(err, 1);
-                        dead = true;
-                    } else if ((spins & 63) == 0 &&
-                               __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
-                        dead = true;   // another workgroup gave up: stop waiting too
-                    }
-                    __builtin_amdgcn_s_sleep(1);
-                }
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-                if (dead) kn = base + (unsigned long long)mx;
-            }
-            kn = __shfl(kn, 0, 64);
-            const int avail = (int)min((unsigned long long)mx, kn - base);
-            const int upto = min(avail, t + 130);
-            for (int p = copied + r; p < upto; p += 64) {
-                const int col = backward ? mx - 1 - p : p;
-                ring[p & 255] = ld_agent(x + (long)jn * mx + col);
-            }
-            __syncthreads();
-            copied = upto;
-        }
-        const double u1 = wave_shr1(h1), u2 = wave_shr1(h2), u3 = wave_shr1(h3);
-        const int c = t - 2 * r;
-        double res = 0.0;
-        if (live && c >= 0 && c < mx) {
-            const double* a = cur.a;
-            const int i = backward ? mx - 1 - c : c;
-            const long q = (long)j * mx + i;
-            const bool hv = backward ? hn : hs;   // the row toward the sweep's origin
-            double v_im1 = 0.0, v_i = 0.0, v_ip1 = 0.0;
-            if (hv) {
-                if (r > 0) {
-                    if (!backward) { v_im1 = u3; v_i = u2; v_ip1 = u1; }
-                    else { v_im1 = u1; v_i = u2; v_ip1 = u3; }
-                } else {   // positions c-1, c, c+1 of the ring
-                    const double pm = c > 0 ? ring[(c - 1) & 255] : 0.0;
-                    const double pp = c + 1 < mx ? ring[(c + 1) & 255] : 0.0;
-                    v_i = ring[c & 255];
-                    if (!backward) { v_im1 = pm; v_ip1 = pp; }
-                    else { v_im1 = pp; v_ip1 = pm; }
-                }
-            }
-            const bool hw = i > 0, he = i + 1 < mx;
-            double sum = cur.b;
-            if (!backward) {
-                if (hs && hw && a[0] != 0.0) sum -= a[0] * v_im1;
-                if (hs && a[1] != 0.0) sum -= a[1] * v_i;
-                if (hs && he && a[2] != 0.0) sum -= a[2] * v_ip1;
-                if (hw && a[3] != 0.0) sum -= a[3] * xo;
-            } else {
-                if (hs && hw && a[0] != 0.0) sum -= a[0] * cur.x[0];
-                if (hs && a[1] != 0.0) sum -= a[1] * cur.x[1];
-                if (hs && he && a[2] != 0.0) sum -= a[2] * cur.x[2];
-                if (hw && a[3] != 0.0) sum -= a[3] * cur.x[3];
-                if (he && a[5] != 0.0) sum -= a[5] * xo;
-                if (hn && hw && a[6] != 0.0) sum -= a[6] * v_im1;
-                if (hn && a[7] != 0.0) sum -= a[7] * v_i;
-                if (hn && he && a[8] != 0.0) sum -= a[8] * v_ip1;
-            }
-            res = a[9] != 0.0 ? sum * a[4] : 0.0;
-            x[q] = res;
-            xo = res;
-            // a full strip publishes its last row's progress every 32 points
-            // (the consumer reads this lane's row only: its own release store)
-            if (r == 63 && ((c & 31) == 31 || c == mx - 1))
-                __hip_atomic_store(flag + s, base + (unsigned long long)(c + 1), __ATOMIC_RELEASE,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-        }
-        fetch(t + SOR9_AHEAD, cur);   // this slot now holds step t + SOR9_AHEAD
-        h3 = h2;
-        h2 = h1;
-        h1 = res;
-    };
-#pragma unroll
-    for (int k = 0; k < SOR9_AHEAD; ++k) fetch(k, pf[k]);
-    for (int t0 = 0; t0 < nsteps; t0 += SOR9_AHEAD) {
-#pragma unroll
-        for (int k = 0; k < SOR9_AHEAD; ++k)
-            if (t0 + k < nsteps) step(t0 + k, pf[k]);
-    }
-}
-
-// One direction of a symmetric SOR sweep (omega 1, zero initial guess) of a
-// 3D constant-coefficient 7-point level in lexicographic order, pipelined:
-// a 64-lane workgroup owns a strip of 64 rows of one plane (rows in sweep
-// order: j = 64 s + r forward, my - 1 - 64 s - r backward), lane r its row,
-// and marches along the row one point per step, lane r one step behind lane
-// r-1, so the neighbour toward the sweep's origin in the same plane is lane
-// r-1's result of the previous step (a DPP shift) and the one in the same
-// row the lane's own.  Workgroup g = nstrips k' + s (k' = k forward, mz-1-k
-// backward) needs the strip before it in its plane (lane 0's neighbour row)
-// and the same strip in the plane before it (every lane's neighbour plane):
-// both have lower indices.  Steps run in batches of SOR7_BATCH: before a
-// batch the first lane waits (relaxed polls, then an agent-scope acquire
-// fence) until those two have
-// published enough steps, then every lane loads the batch's operands (b,
-// the neighbour plane's new values, lane 0's neighbour row; backward also
-// the three lower neighbours, which still hold forward values: the points
-// after a point in the backward order run later), computes the batch, fences
-// its stores (one agent-scope release fence), and the last lane publishes
-// the steps done.
-// Forward: x = (b + sz x_{k-1} + sy x_{j-1} + sx x_{i-1}) / d over interior
-// neighbours, in k_sor_plane's order; backward: (b + sz x_{k-1} + sy
-// x_{j-1} + sx x_{i-1} + sx x_{i+1} + sy x_{j+1} + sz x_{k+1}) / d; a
-// boundary row b / db.  flag: per workgroup, base + steps done (bases grow
-// from sweep to sweep); a wait longer than spin_limit polls sets *err and
-// gives up, and a launch that finds *err set (at entry, or every 64 polls
-// of a wait) waits for nothing (the host checks *err after the solve); need_extra is added to every wait's target
-// (0; the host's stall test sets one no workgroup reaches).  Grid nstrips *
-// mz, block 64.
-constexpr int SOR7_BATCH = 8;
-template <typename T>
-__global__ void __launch_bounds__(64)
-k_sor7_strips(int mx, int my, int mz, double d, double db, double sx, double sy, double sz,
-              const T* __restrict__ b, T* x, unsigned long long* flag, unsigned long long base, int backward,
-              int* err, long spin_limit, unsigned long long need_extra) {
-    static_assert(sizeof(T) == 8, "FP64 sweeps (the neighbours' new values are read as 8-byte atomics)");
-    constexpr int B = SOR7_BATCH;
-    const int nstrips = (my + 63) / 64;
-    const int g = blockIdx.x, r = threadIdx.x;
-    const int s = g % nstrips, kk = g / nstrips;        // strip and plane in sweep order
-    const int k = backward ? mz - 1 - kk : kk;
-    const int jr = 64 * s + r;                          // row in sweep order
-    const int j = backward ? my - 1 - jr : jr;
-    const bool live = jr < my;
-    const int jn = backward ? j + 1 : j - 1;            // neighbour row toward the origin
-    const int kn = backward ? k + 1 : k - 1;            // neighbour plane toward the origin
-    const long dy = backward ? (long)mx : -(long)mx, dz = backward ? (long)mx * my : -((long)mx * my);
-    const long sy_ = mx, sz_ = (long)mx * my;
-    const bool bndjk = j == 0 || j == my - 1 || k == 0 || k == mz - 1;
-    auto inner = [&](int ii, int jj, int kq) {
-        return ii > 0 && ii < mx - 1 && jj > 0 && jj < my - 1 && kq > 0 && kq < mz - 1;
-    };
-    const int nsteps = mx + 63;
-    bool dead = __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
-    const unsigned long long* fs = s > 0 ? flag + (g - 1) : nullptr;          // previous strip, same plane
-    const unsigned long long* fk = kk > 0 ? flag + (g - nstrips) : nullptr;   // same strip, previous plane
-    double prev = 0.0;                                  // the lane's result of the previous step
-    for (int t0 = 0; t0 < nsteps; t0 += B) {
-        const int t1 = min(t0 + B, nsteps);
-        // the batch needs the previous strip through its step t1 - 1 + 64 (its
-        // last lane at this strip's lane-0 columns) and the previous plane's
-        // strip through its step t1 - 1
-        if (r == 0) {
-            const unsigned long long need_s = base + (unsigned long long)min(t1 + 64, nsteps) + need_extra;
-            const unsigned long long need_k = base + (unsigned long long)t1 + need_extra;
-            long spins = 0;
-            // relaxed polls, then one acquire fence (an acquire per poll would
-            // invalidate the cache every time)
-            while (!dead && ((fs && __hip_atomic_load(fs, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < need_s) ||
-                             (fk && __hip_atomic_load(fk, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < need_k))) {
-                if (++spins > spin_limit) {
-                    atomicExch(err, 1);
-                    dead = true;
-                } else if ((spins & 63) == 0 &&
-                           __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
-                    dead = true;   // another workgroup gave up: stop waiting too
-                }
-                __builtin_amdgcn_s_sleep(1);
-            }
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-        }
-        __syncthreads();
-        // the batch's operands
-        double bq[B], vk[B], vj[B], lk[B], lj[B], li[B];
-#pragma unroll
-        for (int e = 0; e < B; ++e) {
-            bq[e] = vk[e] = vj[e] = lk[e] = lj[e] = li[e] = 0.0;
-            const int c = t0 + e - r;
-            if (!(t0 + e < t1 && live && c >= 0 && c < mx)) continue;
-            const int i = backward ? mx - 1 - c : c;
-            const long q = ((long)k * my + j) * mx + i;
-            bq[e] = double(b[q]);
-            if (bndjk || i == 0 || i == mx - 1) continue;
-            if (inner(i, j, kn)) vk[e] = ld_agent((const double*)(x + q + dz));
-            if (r == 0 && inner(i, jn, k)) vj[e] = ld_agent((const double*)(x + q + dy));
-            if (backward) {
-                if (inner(i, j, k - 1)) lk[e] = double(x[q - sz_]);
-                if (inner(i, j - 1, k)) lj[e] = double(x[q - sy_]);
-                if (inner(i - 1, j, k)) li[e] = double(x[q - 1]);
-            }
-        }
-#pragma unroll
-        for (int e = 0; e < B; ++e) {
-            const int t = t0 + e;
-            const double nbv = wave_shr1(prev);         // lane r-1's result of step t-1: (i, jn)
-            const int c = t - r;
-            double res = prev;
-            if (t < t1 && live && c >= 0 && c < mx) {
-                const int i = backward ? mx - 1 - c : c;
-                const int in_ = backward ? i + 1 : i - 1;
-                const long q = ((long)k * my + j) * mx + i;
-                double sum = bq[e];
-                if (bndjk || i == 0 || i == mx - 1) {
-                    res = sum * (1.0 / db);
-                } else {
-                    const bool hk = inner(i, j, kn), hj = inner(i, jn, k), hi = inner(in_, j, k);
-                    const double xj = r > 0 ? nbv : vj[e];
-                    if (!backward) {
-                        if (hk) sum += sz * vk[e];
-                        if (hj) sum += sy * xj;
-                        if (hi) sum += sx * prev;
-                    } else {
-                        if (inner(i, j, k - 1)) sum += sz * lk[e];
-                        if (inner(i, j - 1, k)) sum += sy * lj[e];
-                        if (inner(i - 1, j, k)) sum += sx * li[e];
-                        if (hi) sum += sx * prev;
-                        if (hj) sum += sy * xj;
-                        if (hk) sum += sz * vk[e];
-                    }
-                    res = sum * (1.0 / d);
-                }
-                x[q] = T(res);
-            }
-            prev = res;
-        }
-        // every lane's stores of the batch before the published count: one
-        // release fence for the wave, then the count
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        if (r == 63)
-            __hip_atomic_store(flag + g, base + (unsigned long long)t1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-}
-
 // The dense inverse of a band LU factor (unit lower L and upper U in band
 // storage, row i at B[i * w + (col - i + bw)], w = 2 bw + 1): thread c
 // solves L U z = e_c by band substitution and writes column c of the

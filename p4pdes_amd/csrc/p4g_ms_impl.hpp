@@ -118,7 +118,7 @@ static int ms_fdjac_level(p4g_solver_s* s, MsRun& R, int l, const double* x, con
     const double unorm = std::sqrt(s->cx.hS[16 + S_TMP1]);
     const double d = 1.0 / (std::sqrt(1.0 + unorm) * 1.490116119384766e-08);   // "wp": PETSC_SQRT_MACHINE_EPSILON
     k_ms_fdjac<<<nb, 256, 0, R.st>>>(g, x, R.gb[l], F, d, 1.0 / d, s->g27[l]);
-    if (s->lv[l].pipe) k_sor9_pack<<<nb, 256, 0, R.st>>>(g.n, s->g27[l], s->lv[l].pipe->pk);
+    if (s->lv[l].pipe) sor9_pack(s->lv[l], s->g27[l], R.st);
     LAUNCH_CHECK();
     return 0;
 }
@@ -130,7 +130,7 @@ static int ms_const_level(p4g_solver_s* s, MsRun& R, int l) {
     const LevelInfo& Lv = s->lv[l];
     const int nb = vblocks(Lv.n);
     k_const5_to_g27<<<nb, 256, 0, R.st>>>(Lv.mx, Lv.my, Lv.d, Lv.db, Lv.sx, Lv.sy, s->g27[l]);
-    if (Lv.pipe) k_sor9_pack<<<nb, 256, 0, R.st>>>(Lv.n, s->g27[l], Lv.pipe->pk);
+    if (Lv.pipe) sor9_pack(Lv, s->g27[l], R.st);
     LAUNCH_CHECK();
     return 0;
 }
@@ -339,16 +339,7 @@ static int ms_solve(p4g_solver_s* s, double q, const double* gb, double* x, p4g_
         }
         if (s->sor && s->pctype == PCT_MG) {   // pipelined strip sweeps on every level
             s->ms_pipes.resize(s->nlev);
-            for (int l = l0; l <= L; ++l) {
-                if (s->lv[l].mx >= (1 << 22)) continue;
-                const int ns = (s->lv[l].my + 63) / 64;
-                SorPipe& P = s->ms_pipes[l];
-                P4G_TRY(dalloc(s, (void**)&P.flags, (ns + 1) * sizeof(unsigned long long) + sizeof(int)));
-                HIP_TRY(hipMemset(P.flags, 0, (ns + 1) * sizeof(unsigned long long) + sizeof(int)));
-                P.err = (int*)(P.flags + ns + 1);
-                P4G_TRY(dalloc(s, (void**)&P.pk, 10 * s->lv[l].n * sizeof(double)));
-                s->lv[l].pipe = &P;
-            }
+            for (int l = l0; l <= L; ++l) P4G_TRY(sor_pipe_alloc(s, l, SOR_9PT));
         }
         if (s->pctype == PCT_ILU) {
             P4G_TRY(dalloc(s, (void**)&s->ms_ilu9, 9 * n * sizeof(double)));

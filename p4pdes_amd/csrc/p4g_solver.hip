@@ -32,6 +32,7 @@
 
 #include "p4g_internal.hpp"
 #include "p4g_kernels.hpp"
+#include "p4g_sor_kernels.hpp"
 
 using namespace p4g;
 
@@ -74,15 +75,19 @@ static double now_ms() {
 }
 
 // precision-independent description of one multigrid level
-// the progress flags of a level's pipelined 2D SOR sweeps (k_sor9_strips):
-// one word per 64-row strip, a stall word, and the host's sweep counter
+// a level's pipelined SOR sweeps (k_sor2, k_sor7): their working arrays
+enum SorKind { SOR_5PT, SOR_9PT, SOR_7PT };
 struct SorPipe {
-    double* pk = nullptr;                 // the operator as k_sor9_pack records (refreshed with it)
-    unsigned long long* flags = nullptr;
-    int* err = nullptr;
-    unsigned long long epoch = 0;
+    SorKind kind = SOR_5PT;
+    int Tp = 0, ns = 0, ng = 0;           // steps, strips, plane groups
+    T2<double>* S = nullptr;              // the sweep's sums, in its order
+    T2<double>* pk = nullptr;             // 9-point: the operator as k_sor9_pack records (refreshed with it)
+    T2<double>* inv = nullptr;            //   and its reciprocal diagonal
+    u64* yh = nullptr;                    // handed-over rows and planes
+    u64* zh = nullptr;
+    unsigned* ctl = nullptr;              // stall word, sweeps done
     long spin_limit = 1L << 24;           // polls before a wait gives up
-    unsigned long long need_extra = 0;    // -p4g_sor_test_stall: a target no strip reaches
+    unsigned extra = 0;                   // -p4g_sor_test_stall: a tag no workgroup writes
 };
 
 struct LevelInfo {
@@ -98,36 +103,59 @@ struct LevelInfo {
     bool gal = false;                                // Galerkin operator P^T A P in 27-point form
     int sor_nblk = 1;                                // SOR local sweeps: blocks of the slowest dimension
     int sor_blk[17] = {0};                           //   and their first indices
-    SorPipe* pipe = nullptr;                         // 2D 27-plane SOR by pipelined strips, when set
+    SorPipe* pipe = nullptr;                         // SOR by pipelined strips, when set
 };
 
+// the pipelined sweeps of a level with working arrays, if they apply to it now
+static SorPipe* sor_pipe_of(const LevelInfo& L) {
+    if (!L.pipe || L.var || L.sor_nblk > 1 || L.gal != (L.pipe->kind == SOR_9PT)) return nullptr;
+    return L.pipe;
+}
+
+// the packed operator of a 9-point level's sweeps, from its coefficients
+static void sor9_pack(const LevelInfo& L, const double* g27, hipStream_t st) {
+    const SorPipe& P = *L.pipe;
+    k_sor9_pack<<<dim3(P.Tp / 32, P.ns), 256, 0, st>>>(L.mx, L.my, P.Tp, g27, P.pk, P.inv);
+}
+
+// one symmetric sweep by pipelined strips, a launch per direction: 2D into z
+// (natural order), 3D into P->S (sweep order)
+static void sor_pipe_run(const LevelInfo& L, SorPipe* P, const double* r, double* z, hipStream_t st) {
+    const SorCtl c{P->ctl, P->spin_limit, P->extra};
+    if (P->kind == SOR_7PT) {
+        k_sor7_pack<<<dim3(P->Tp / 64, P->ns * P->ng), 256, 0, st>>>(L.mx, L.my, L.mz, P->Tp, P->ns, r, P->S);
+        const Sor7Args A{L.mx, L.my, L.mz, P->Tp, P->ns, P->ng, L.d, L.sx, L.sy, L.sz, P->S, P->yh, P->zh, c};
+        k_sor7<false><<<P->ns * P->ng, 64, 0, st>>>(A);
+        k_sor7<true><<<P->ns * P->ng, 64, 0, st>>>(A);
+        return;
+    }
+    const Sor2Args A{L.mx, L.my, P->Tp, P->ns, L.d, L.db, L.sx, L.sy, P->pk, P->inv, r, P->S, z, P->yh, c};
+    if (P->kind == SOR_9PT) {
+        k_sor2<true, false><<<P->ns, 64, 0, st>>>(A);
+        k_sor2<true, true><<<P->ns, 64, 0, st>>>(A);
+    } else {
+        const int nb = (2 * (L.mx + L.my) + 255) / 256;      // boundary rows, four points a lane
+        k_sor2<false, false><<<P->ns + nb, 64, 0, st>>>(A);
+        k_sor2<false, true><<<P->ns, 64, 0, st>>>(A);
+    }
+}
+
+// y = a p + c q + e SSOR(r) from the sweep's order (3D)
+static void sor7_unpack(const LevelInfo& L, const SorPipe* P, const double* r, double a, const double* p, double c,
+                        const double* q, double e, double* y, hipStream_t st) {
+    k_sor7_unpack<<<dim3(P->Tp / 64 + 1, P->ns * P->ng), 256, 0, st>>>(L.mx, L.my, L.mz, P->Tp, P->ns, P->S, r, L.db,
+                                                                     a, p, c, q, e, y);
+}
+
 // one symmetric SOR sweep z = SSOR(r) on a level (omega 1, zero initial
-// guess): the hyperplanes forward then backward (k_sor_plane)
+// guess): by pipelined strips, or the hyperplanes forward then backward
+// (k_sor_plane): 1D levels, 3D Galerkin levels, several ranks' local sweeps
 template <typename T>
 static int sor_run(const LevelInfo& L, const double* g27, const T* r, T* z, hipStream_t st) {
     if constexpr (std::is_same<T, double>::value) {
-        if (L.dim == 3 && !L.gal && !L.var && L.pipe && L.pipe->flags && !L.pipe->pk && L.sor_nblk <= 1) {
-            // 3D 7-point level: pipelined strips, one launch per sweep direction
-            SorPipe* P = L.pipe;
-            const unsigned nwg = (unsigned)(((L.my + 63) / 64) * L.mz);
-            const unsigned long long b0 = (++P->epoch) << 22;
-            k_sor7_strips<double><<<nwg, 64, 0, st>>>(L.mx, L.my, L.mz, L.d, L.db, L.sx, L.sy, L.sz, r, z, P->flags,
-                                                       b0, 0, P->err, P->spin_limit, P->need_extra);
-            const unsigned long long b1 = (++P->epoch) << 22;
-            k_sor7_strips<double><<<nwg, 64, 0, st>>>(L.mx, L.my, L.mz, L.d, L.db, L.sx, L.sy, L.sz, r, z, P->flags,
-                                                       b1, 1, P->err, P->spin_limit, P->need_extra);
-            LAUNCH_CHECK();
-            return 0;
-        }
-        if (L.gal && L.dim == 2 && L.pipe && L.pipe->pk && L.sor_nblk <= 1 && g27) {   // one launch per direction
-            const int ns = (L.my + 63) / 64;
-            SorPipe* P = L.pipe;
-            const unsigned long long b0 = (++P->epoch) << 22;
-            k_sor9_strips<<<ns, 64, 0, st>>>(L.mx, L.my, P->pk, r, z, P->flags, b0, 0, P->err, P->spin_limit,
-                                             P->need_extra);
-            const unsigned long long b1 = (++P->epoch) << 22;
-            k_sor9_strips<<<ns, 64, 0, st>>>(L.mx, L.my, P->pk, r, z, P->flags, b1, 1, P->err, P->spin_limit,
-                                             P->need_extra);
+        if (SorPipe* P = sor_pipe_of(L)) {
+            sor_pipe_run(L, P, r, z, st);
+            if (P->kind == SOR_7PT) sor7_unpack(L, P, r, 0.0, nullptr, 0.0, nullptr, 1.0, z, st);
             LAUNCH_CHECK();
             return 0;
         }
@@ -941,8 +969,9 @@ struct Engine {
                 P4G_TRY(e);
                 rr = r;
             }
+            SorPipe* const P3 = sor_pipe_of(L) && L.pipe->kind == SOR_7PT && !lilu ? L.pipe : nullptr;
             if (lilu) P4G_TRY(ilu_run<T>(L, ilu_u.size() > (size_t)l ? ilu_u[l] : nullptr, rr, z, st));
-            else P4G_TRY(sor_run<T>(L, g27.size() > (size_t)l ? g27[l] : nullptr, rr, z, st));
+            else if (!P3) P4G_TRY(sor_run<T>(L, g27.size() > (size_t)l ? g27[l] : nullptr, rr, z, st));
             T* dst = out;
             if (m < nu)
                 for (int q = 1; q < 4; ++q)
@@ -956,7 +985,11 @@ struct Engine {
                 ca = 1.0 - omega; cb = omega; cc = omega * s;
             }
             const T* pa = (smoother == SM_CHEB && m >= 2) ? pm2 : nullptr;
+            if constexpr (std::is_same<T, double>::value)
+                if (P3) sor_pipe_run(L, P3, rr, nullptr, st);
             P4G_TRY(cx->launch(P4G_K_SMOOTH, l == nlev - 1, 3.0 * n * sizeof(T), [&] {
+                if constexpr (std::is_same<T, double>::value)
+                    if (P3) return sor7_unpack(L, P3, rr, ca, pa, cb, pm1, cc, dst, st);
                 k_comb3<T><<<gb, 256, 0, st>>>(n, ca, pa, cb, pm1, cc, z, dst);
             }));
             pm2 = pm1;
@@ -2572,25 +2605,57 @@ static void sor_splits(p4g_solver_s* s) {
     }
 }
 
+// the working arrays of level l's pipelined SOR sweeps (1D levels, and grids
+// without interior points, have none)
+static int sor_pipe_alloc(p4g_solver_s* s, int l, SorKind kind) {
+    LevelInfo& L = s->lv[l];
+    if (L.dim < 2 || L.var) return 0;
+    const bool nine = kind == SOR_9PT;
+    if (!nine && (L.mx < 3 || L.my < 3 || (L.dim == 3 && L.mz < 3))) return 0;
+    SorPipe& P = s->ms_pipes[l];
+    P.kind = kind;
+    P.ng = 1;
+    size_t nS, ny, nz = 0;
+    if (kind == SOR_7PT) {
+        P.Tp = Sor7::steps(L.mx);
+        P.ns = Sor7::strips(L.my);
+        P.ng = Sor7::groups(L.mz);
+        nS = (size_t)P.ns * P.ng * P.Tp * (Sor7::K / 2) * 64;
+        ny = (size_t)P.ns * P.ng * (L.mx - 2) * Sor7::K * 2;
+        nz = (size_t)P.ns * P.ng * (P.Tp + Sor7::K - 1) * 128;
+    } else {
+        P.Tp = nine ? Sor2<true>::steps(L.mx) : Sor2<false>::steps(L.mx);
+        P.ns = nine ? Sor2<true>::strips(L.my) : Sor2<false>::strips(L.my);
+        nS = (size_t)P.ns * (P.Tp / 2) * 64;
+        ny = (size_t)P.ns * L.mx * 2;
+    }
+    auto zeroed = [&](void** p, size_t bytes) -> int {
+        P4G_TRY(dalloc(s, p, bytes));
+        HIP_TRY(hipMemset(*p, 0, bytes));
+        return 0;
+    };
+    P4G_TRY(zeroed((void**)&P.S, nS * sizeof(T2<double>)));
+    P4G_TRY(zeroed((void**)&P.yh, ny * sizeof(u64)));
+    if (nz) P4G_TRY(zeroed((void**)&P.zh, nz * sizeof(u64)));
+    P4G_TRY(zeroed((void**)&P.ctl, 2 * sizeof(unsigned)));
+    if (nine) {
+        P4G_TRY(dalloc(s, (void**)&P.pk, (size_t)P.ns * P.Tp * 256 * sizeof(T2<double>)));
+        P4G_TRY(dalloc(s, (void**)&P.inv, nS * sizeof(T2<double>)));
+    }
+    L.pipe = &P;
+    return 0;
+}
+
 int solver_setup(p4g_solver_s* s) {
     if (s->ready) return 0;
     const double t0 = now_ms();
     P4G_TRY(build_levels(s));
     sor_splits(s);
-    // pipelined 3D SOR sweeps (k_sor7_strips): progress flags per level
     if (s->pctype == PCT_MG && s->sor && !s->lilu && s->sor_pipeline && !s->vi_mode && !s->ms_mode) {
-        s->ms_pipes.resize(s->nlev);
-        for (int l = 1; l < s->nlev; ++l) {
-            LevelInfo& L = s->lv[l];
-            if (L.dim != 3 || L.sor_nblk > 1) continue;
-            const long nf = (long)((L.my + 63) / 64) * L.mz;
-            SorPipe& P = s->ms_pipes[l];
-            const size_t bytes = (nf + 1) * sizeof(unsigned long long) + sizeof(int);
-            P4G_TRY(dalloc(s, (void**)&P.flags, bytes));
-            HIP_TRY(hipMemset(P.flags, 0, bytes));
-            P.err = (int*)(P.flags + nf + 1);
-            L.pipe = &P;
-        }
+        s->ms_pipes.resize(s->nlev);   // pipelined SOR sweeps on the smoothing levels
+        for (int l = s->nlev > 1 ? 1 : 0; l < s->nlev; ++l)
+            if (s->lv[l].sor_nblk <= 1 && !(s->galerkin && l < s->nlev - 1))
+                P4G_TRY(sor_pipe_alloc(s, l, s->lv[l].dim == 3 ? SOR_7PT : SOR_5PT));
     }
     // ILU(0) pivots: the finest level for -pc_type ilu, the smoothing levels
     // for -mg_levels_pc_type ilu (computed once on the host, in the factor's
@@ -3577,25 +3642,25 @@ const char* p4g_version(void) { return "p4g 0.1 (gfx950)"; }
 
 // continuous-batching server (uses the types above)
 namespace p4g {
-// The stall words of the pipelined SOR sweeps (k_sor9_strips): cleared at the
+// The stall words of the pipelined SOR sweeps: cleared at the
 // start of a solve, read after each linear solve, where the solve has just
 // synchronized its stream, so a stall stops the solve at the Newton step it
 // happened in.
 static int sor_pipes_reset(p4g_solver_s* s) {
     for (SorPipe& P : s->ms_pipes) {
-        if (!P.err) continue;
+        if (!P.ctl) continue;
         P.spin_limit = s->sor_test_stall ? 64 : (1L << 24);
-        P.need_extra = s->sor_test_stall ? (1ull << 21) : 0;
-        HIP_TRY(hipMemsetAsync(P.err, 0, sizeof(int), s->cx.stream));
+        P.extra = s->sor_test_stall ? 1u << 21 : 0;
+        HIP_TRY(hipMemsetAsync(P.ctl, 0, sizeof(unsigned), s->cx.stream));
     }
     return 0;
 }
 
 static int sor_pipes_check(p4g_solver_s* s, const char* who) {
     for (const SorPipe& P : s->ms_pipes) {
-        if (!P.err) continue;
+        if (!P.ctl) continue;
         int e = 0;
-        HIP_TRY(hipMemcpyAsync(&e, P.err, sizeof(int), hipMemcpyDeviceToHost, s->cx.stream));
+        HIP_TRY(hipMemcpyAsync(&e, P.ctl, sizeof(int), hipMemcpyDeviceToHost, s->cx.stream));
         HIP_TRY(hipStreamSynchronize(s->cx.stream));
         if (e) return set_error(PETSC_ERR_LIB, "%s: a pipelined SOR sweep stalled", who);
     }

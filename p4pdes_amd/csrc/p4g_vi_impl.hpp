@@ -99,8 +99,7 @@ static int vi_operator(p4g_solver_s* s, ViRun& R) {
     P4G_TRY(galerkin_levels(s));
     for (int l = 0; l < L; ++l) e.g27[l] = s->g27[l];
     for (int l = 0; l <= L; ++l)   // the pipelined SOR sweeps read the operator as packed records
-        if (s->lv[l].pipe)
-            k_sor9_pack<<<vblocks(s->lv[l].n), 256, 0, R.st>>>(s->lv[l].n, s->g27[l], s->lv[l].pipe->pk);
+        if (s->lv[l].pipe) sor9_pack(s->lv[l], s->g27[l], R.st);
     LAUNCH_CHECK();
     if (L > 0) {
         std::vector<double> Ainv;
@@ -421,16 +420,7 @@ static int vi_solve(p4g_solver_s* s, const double* xl, const double* xu, double*
         // vectors (6 of the finest size) instead of allocating per level
         if (s->sor && s->pctype == PCT_MG && s->lv[L].dim == 2) {   // pipelined strip sweeps on every level
             s->ms_pipes.resize(s->nlev);
-            for (int l = 0; l <= L; ++l) {
-                if (s->lv[l].mx >= (1 << 22)) continue;
-                const int ns = (s->lv[l].my + 63) / 64;
-                SorPipe& P = s->ms_pipes[l];
-                P4G_TRY(dalloc(s, (void**)&P.flags, (ns + 1) * sizeof(unsigned long long) + sizeof(int)));
-                HIP_TRY(hipMemset(P.flags, 0, (ns + 1) * sizeof(unsigned long long) + sizeof(int)));
-                P.err = (int*)(P.flags + ns + 1);
-                P4G_TRY(dalloc(s, (void**)&P.pk, 10 * s->lv[l].n * sizeof(double)));
-                s->lv[l].pipe = &P;
-            }
+            for (int l = 0; l <= L; ++l) P4G_TRY(sor_pipe_alloc(s, l, SOR_9PT));
         }
         if (s->pctype == PCT_MG && s->smoother == SM_CHEB) {
             s->est_cap = 6 * n;

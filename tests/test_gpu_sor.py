@@ -1,0 +1,61 @@
+"""Pipelined SOR sweeps (k_sor2, k_sor7) against the hyperplane sweeps
+(k_sor_plane): every point is updated from the same values in the same order,
+so one preconditioner application agrees bit for bit.  One-level grids take
+any size (the smoother is the preconditioner): the edges of a strip's 64 rows,
+of the operand ring's rounds of 32 steps and of the plane groups, single
+interior points, and boxes longer in each direction."""
+import numpy as np
+import pytest
+
+from p4pdes_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+GRIDS_2D = [(3, 3), (4, 3), (3, 70), (35, 5), (66, 66), (67, 65), (34, 131), (130, 67), (260, 130), (97, 200)]
+GRIDS_3D = [(3, 3, 3), (4, 5, 6), (66, 5, 3), (5, 66, 7), (6, 67, 8), (7, 4, 70), (33, 34, 35), (67, 130, 9), (65, 65, 65)]
+
+
+def _apply(args, b):
+    with capi.Session(args) as s:
+        assert s.n == b.size
+        A = capi.Solver(s)
+        return A.pc_apply(b), A.pc_apply(b)
+
+
+def _pair(args, n, seed):
+    b = np.random.default_rng(seed).standard_normal(n)
+    print("sor pair", args, flush=True)
+    z0, _ = _apply(args + " -p4g_sor_pipeline 0", b)
+    z1, z2 = _apply(args, b)
+    assert np.isfinite(z0).all()
+    assert np.array_equal(z0, z1), np.max(np.abs(z1 - z0))
+    assert np.array_equal(z1, z2)          # the tags of the next sweeps
+
+
+@pytest.mark.parametrize("grid", GRIDS_2D, ids=lambda g: "x".join(map(str, g)))
+def test_sor2_matches_hyperplanes(grid):
+    mx, my = grid
+    _pair("-fsh_dim 2 -fsh_problem zero -fsh_cx 1.7 -da_grid_x %d -da_grid_y %d -pc_type mg -pc_mg_levels 1 "
+          "-mg_levels_ksp_max_it 2" % (mx, my), mx * my, mx + my)
+
+
+@pytest.mark.parametrize("grid", GRIDS_3D, ids=lambda g: "x".join(map(str, g)))
+def test_sor7_matches_hyperplanes(grid):
+    mx, my, mz = grid
+    _pair("-fsh_dim 3 -fsh_problem zero -fsh_cx 1.7 -fsh_cz 0.6 -da_grid_x %d -da_grid_y %d -da_grid_z %d "
+          "-pc_type mg -pc_mg_levels 1 -mg_levels_ksp_max_it 3" % (mx, my, mz), mx * my * mz, mx + my + mz)
+
+
+def test_sor2_multigrid_matches_hyperplanes():
+    _pair("-fsh_dim 2 -fsh_problem zero -da_refine 8 -pc_type mg -pc_mg_cycle_type w", 513 * 513, 5)
+
+
+def test_sor2_stall_stops_the_solve():
+    # a 2D sweep of two strips whose waits cannot succeed: every kernel ends
+    # and the solve reports it; a fresh solve then runs normally
+    args = "-fsh_dim 2 -fsh_problem manupoly -da_refine 6 -pc_type mg -ksp_rtol 1e-8"
+    rc, text, _, _ = capi.fish_run(args + " -p4g_sor_test_stall 1")
+    assert rc == 76, text
+    assert "pipelined SOR sweep stalled" in text
+    rc, text, _, _ = capi.fish_run(args)
+    assert rc == 0, text
