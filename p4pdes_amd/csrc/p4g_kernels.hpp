@@ -80,6 +80,12 @@ __device__ __forceinline__ void stv(T* __restrict__ p, const TV<T, V>& a) {
     __builtin_memcpy(p, &t, sizeof(vec));
 }
 
+// LDS traffic between the lanes of one wave: the hardware keeps its order, this keeps the compiler's
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // points per lane of the stencil kernels: one 16-byte access
 template <typename T>
 struct VecOf {

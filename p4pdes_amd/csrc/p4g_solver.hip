@@ -131,12 +131,12 @@ static void sor_pipe_run(const LevelInfo& L, SorPipe* P, const double* r, double
     }
     const Sor2Args A{L.mx, L.my, P->Tp, P->ns, L.d, L.db, L.sx, L.sy, P->pk, P->inv, r, P->S, z, P->yh, c};
     if (P->kind == SOR_9PT) {
-        k_sor2<true, false><<<P->ns, 64, 0, st>>>(A);
-        k_sor2<true, true><<<P->ns, 64, 0, st>>>(A);
+        k_sor2<true, false><<<P->ns * kXcds, 64, 0, st>>>(A);
+        k_sor2<true, true><<<P->ns * kXcds, 64, 0, st>>>(A);
     } else {
         const int nb = (2 * (L.mx + L.my) + 255) / 256;      // boundary rows, four points a lane
-        k_sor2<false, false><<<P->ns + nb, 64, 0, st>>>(A);
-        k_sor2<false, true><<<P->ns, 64, 0, st>>>(A);
+        k_sor2<false, false><<<P->ns * kXcds + nb, 64, 0, st>>>(A);
+        k_sor2<false, true><<<P->ns * kXcds, 64, 0, st>>>(A);
     }
 }
 
@@ -2609,7 +2609,7 @@ static void sor_splits(p4g_solver_s* s) {
 // without interior points, have none)
 static int sor_pipe_alloc(p4g_solver_s* s, int l, SorKind kind) {
     LevelInfo& L = s->lv[l];
-    if (L.dim < 2 || L.var) return 0;
+    if (L.dim < 2 || L.var || L.mx >= 1 << 20) return 0;      // (a strip's rows are addressed in 32 bits)
     const bool nine = kind == SOR_9PT;
     if (!nine && (L.mx < 3 || L.my < 3 || (L.dim == 3 && L.mz < 3))) return 0;
     SorPipe& P = s->ms_pipes[l];
@@ -2627,7 +2627,7 @@ static int sor_pipe_alloc(p4g_solver_s* s, int l, SorKind kind) {
         P.Tp = nine ? Sor2<true>::steps(L.mx) : Sor2<false>::steps(L.mx);
         P.ns = nine ? Sor2<true>::strips(L.my) : Sor2<false>::strips(L.my);
         nS = (size_t)P.ns * (P.Tp / 2) * 64;
-        ny = (size_t)P.ns * L.mx * 2;
+        ny = (size_t)P.ns * (nine ? Sor2<true>::slots(P.Tp) : Sor2<false>::slots(P.Tp)) * 2;
     }
     auto zeroed = [&](void** p, size_t bytes) -> int {
         P4G_TRY(dalloc(s, p, bytes));
