@@ -2835,12 +2835,181 @@ k_ilu27_plane(SorOp o, const double* __restrict__ u, int p, int backward, const 
     z[q] = T(s / uq);
 }
 
-// The dense inverse of a band LU factor (unit lower L and upper U in band
-// storage, row i at B[i * w + (col - i + bw)], w = 2 bw + 1): thread c
-// solves L U z = e_c by band substitution and writes column c of the
-// row-major inverse, which is also its workspace (coalesced across c).
+// The coarsest operator of a 27-plane level in band storage: row i at
+// B[i w + (col - i + bw)], w = 2 bw + 1.  unit_null: a null row (an active
+// vertex of a reduced-space step) becomes a unit row, so that x_q = b_q.
 __global__ void __launch_bounds__(256)
+k_band_fill(int mx, int my, int n, int bw, const double* __restrict__ g, int unit_null, double* __restrict__ B) {
+    const int w = 2 * bw + 1;
+    for (long t = blockIdx.x * 256L + threadIdx.x; t < (long)n * w; t += (long)gridDim.x * 256L) {
+        const int q = (int)(t / w), p = q + (int)(t % w) - bw;
+        double v = 0.0;
+        if (p >= 0 && p < n) {
+            const int ox = p % mx - q % mx, oy = p / mx % my - q / mx % my, oz = p / mx / my - q / mx / my;
+            if (ox >= -1 && ox <= 1 && oy >= -1 && oy <= 1 && oz >= -1 && oz <= 1)
+                v = g[(long)((oz + 1) * 9 + (oy + 1) * 3 + ox + 1) * n + q];
+            if (p == q && unit_null && v == 0.0) v = 1.0;
+        }
+        B[t] = v;
+    }
+}
+
+// Band LU without pivoting, in place, by one workgroup (bw < 64).  Bound by
+// its n dependent steps, so the window of a step (rows and columns k ..
+// k + bw, at most 64 x 64) stays in registers, four entries a thread, at
+// places that its indices modulo bw + 1 give: a step publishes row and column
+// k through LDS, everyone updates, and row and column k + bw + 1 take the
+// free places.  The entering rows and columns are read kLuChunk steps ahead.
+// One barrier per step; 1089 points with bw 34: 0.26 ms, where the host took
+// 1.5 ms and two copies.  info: the first row whose pivot is zero (spd: not
+// positive), + 1, or 0.
+constexpr int kLuChunk = 8;
+__global__ void __launch_bounds__(1024)
+k_band_lu(int n, int bw, double* __restrict__ B, int spd, int* __restrict__ info) {
+    const int w = 2 * bw + 1, W = bw + 1, tid = threadIdx.x;
+    const int a = tid >> 4, b0 = tid & 15;               // place (a, b0 + 16 m)
+    __shared__ double row[2][64], col[2][64];
+    __shared__ double in[2][kLuChunk][128];              // entering row (0..63) and column (64..127), by place
+    double v[4];
+    auto entry = [&](int i, int j) {
+        return i < n && j < n && i - j <= bw && j - i <= bw ? B[(long)i * w + (j - i + bw)] : 0.0;
+    };
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        const int b = b0 + 16 * m;
+        v[m] = a < W && b < W ? entry(a, b) : 0.0;
+    }
+    // what enters after step k: row and column e = k + W; place p holds the
+    // column (row) in k + 1 .. k + W congruent to p
+    const int ls = tid >> 7, lp = tid & 127, lq = lp & 63;
+    auto enter = [&](int k) {
+        if (lq >= W) return 0.0;
+        const int e = k + W, base = k + 1, other = base + (lq - base % W + W) % W;
+        return lp < 64 ? entry(e, other) : entry(other, e);
+    };
+    in[0][ls][lp] = enter(ls);
+    int bad = 0;
+    __syncthreads();
+    int kw = 0;
+    for (int k0 = 0; k0 < n; k0 += kLuChunk) {
+        const int buf = (k0 / kLuChunk) & 1;
+        const double next = enter(k0 + kLuChunk + ls);
+#pragma unroll 1
+        for (int s = 0; s < kLuChunk && k0 + s < n; ++s) {
+            const int k = k0 + s, par = k & 1;
+            if (a == kw) {
+#pragma unroll
+                for (int m = 0; m < 4; ++m) row[par][b0 + 16 * m] = v[m];
+            }
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+                if (b0 + 16 * m == kw) col[par][a] = v[m];
+            if (s == kLuChunk - 1) in[buf ^ 1][ls][lp] = next;
+            __syncthreads();
+            const double piv = row[par][kw];
+            if (!bad && (spd ? !(piv > 0.0) : piv == 0.0)) bad = k + 1;
+            const double l = col[par][a] / piv;
+            const int i = k + (a - kw + W) % W;          // the row at place a
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                const int b = b0 + 16 * m, j = k + (b - kw + W) % W;
+                if (a >= W || b >= W) continue;
+                if (a == kw || b == kw) {                // final: U's row and L's column
+                    if (i < n && j < n) B[(long)i * w + (j - i + bw)] = b == kw && a != kw ? l : v[m];
+                    v[m] = a == kw ? in[buf][s][b] : in[buf][s][64 + a];
+                } else {
+                    v[m] -= l * row[par][b];
+                }
+            }
+            kw = kw + 1 == W ? 0 : kw + 1;
+        }
+        __syncthreads();
+    }
+    if (tid == 0) *info = bad;
+}
+
+// The dense inverse of a band LU factor (bw < 64): a wave takes 16 columns of
+// the identity through both substitutions, four lanes a column, each a
+// quarter of a row's sum; the last rows of the solution stay in LDS and the
+// factor's rows come through LDS a chunk ahead.  Bound by the 2 n dependent
+// rows: 1089 points with bw 34 took 9.1 ms with a thread per column and its
+// column read back from memory.
+constexpr int kInvRows = 8;
+__global__ void __launch_bounds__(64)
 k_band_inverse(int n, int bw, const double* __restrict__ B, double* __restrict__ Ainv) {
+    const int w = 2 * bw + 1, r = threadIdx.x, c = r >> 2, p = r & 3;
+    const int c0 = blockIdx.x * 16, cc = c0 + c;
+    __shared__ double win[128][16];                      // the last solution rows, by row modulo 128
+    __shared__ double Bs[2][kInvRows][136];              // factor rows, four zeros on either side
+    constexpr int PF = kInvRows * 136 / 64;
+    double pf[PF];
+    // forward rows r0 .. r0 + 7, or backward rows r0 .. r0 - 7
+    auto fetch = [&](int r0, int dir) {
+#pragma unroll
+        for (int e = 0; e < PF; ++e) {
+            const int t = e * 64 + r, i = r0 + dir * (t / 136), x = t % 136 - 4;
+            pf[e] = i >= 0 && i < n && x >= 0 && x < w ? B[(long)i * w + x] : 0.0;
+        }
+    };
+    auto stage = [&](int buf) {
+#pragma unroll
+        for (int e = 0; e < PF; ++e) {
+            const int t = e * 64 + r;
+            Bs[buf][t / 136][t % 136] = pf[e];
+        }
+        wave_lds_order();
+    };
+    auto quad = [&](double s) {                          // the sum over the column's four lanes
+        s += __shfl_xor(s, 1, 4);
+        return s + __shfl_xor(s, 2, 4);
+    };
+    const int terms = (bw + 3) / 4;
+    for (int dir = 1; dir >= -1; dir -= 2) {
+        const int first = dir > 0 ? c0 : n - 1, count = dir > 0 ? n - c0 : n;
+        for (int e = r; e < 128 * 16; e += 64) win[e >> 4][e & 15] = 0.0;
+        fetch(first, dir);
+        stage(0);
+        double z = dir < 0 && first >= c0 && cc < n ? Ainv[(long)first * n + cc] : 0.0;
+        for (int h = 0; h < count; h += kInvRows) {
+            const int buf = (h / kInvRows) & 1;
+            fetch(first + dir * (h + kInvRows), dir);
+            for (int s = 0; s < kInvRows && h + s < count; ++s) {
+                const int i = first + dir * (h + s);
+                const double* const br = Bs[buf][s] + 4 + bw;
+                double s0 = 0.0, s1 = 0.0;
+                int m = 0;
+                for (; m + 1 < terms; m += 2) {
+                    const int t0 = dir * (p + 1 + 4 * m), t1 = dir * (p + 5 + 4 * m);
+                    s0 += br[-t0] * win[(i - t0) & 127][c];
+                    s1 += br[-t1] * win[(i - t1) & 127][c];
+                }
+                if (m < terms) {
+                    const int t0 = dir * (p + 1 + 4 * m);
+                    s0 += br[-t0] * win[(i - t0) & 127][c];
+                }
+                const double base = dir > 0 ? (i == cc ? 1.0 : 0.0) : z;
+                if (dir < 0) {                           // the row after: asked for a row ahead
+                    const int in = i - 1;
+                    z = in >= c0 && cc < n ? Ainv[(long)in * n + cc] : 0.0;
+                }
+                double v = base - quad(s0 + s1);
+                if (dir < 0) v /= br[0];
+                if (p == 0) {
+                    win[i & 127][c] = v;
+                    if (cc < n) Ainv[(long)i * n + cc] = v;
+                }
+                wave_lds_order();
+            }
+            stage(buf ^ 1);
+        }
+        __syncthreads();                                 // the forward solution, read back by the column's lanes
+    }
+}
+
+// The same for wider bands: thread c solves L U z = e_c and writes column c of
+// the row-major inverse, which is also its workspace (coalesced across c).
+__global__ void __launch_bounds__(256)
+k_band_inverse_wide(int n, int bw, const double* __restrict__ B, double* __restrict__ Ainv) {
     const int c = blockIdx.x * 256 + threadIdx.x;
     if (c >= n) return;
     const int w = 2 * bw + 1;

@@ -11,57 +11,6 @@
 
 namespace p4g {
 
-// The coarsest level of a nonsymmetric 27-plane operator: band LU without
-// pivoting on the host (PETSc's serial coarse LU factors these diagonally
-// dominant Jacobians without row exchanges), then the engine's dense
-// inverse on the device, a column per thread (k_band_inverse).
-static int coarse_factor_lu(p4g_solver_s* s, const LevelInfo& L, const double* g27, Engine<double>& e,
-                            hipStream_t st) {
-    const int n = (int)L.n;
-    if (n > MAX_COARSE)
-        return set_error(PETSC_ERR_SUP, "coarsest grid has %d points (> %d); use more multigrid levels", n,
-                         MAX_COARSE);
-    if (!e.Ainv || e.n0 != n) return set_error(PETSC_ERR_LIB, "internal: coarse inverse of a different size");
-    const int mx = L.mx, my = L.my;
-    const int bw = L.dim == 3 ? mx * my + mx + 1 : (L.dim == 2 ? mx + 1 : 1);
-    const int w = 2 * bw + 1;
-    std::vector<double> g((size_t)27 * n);
-    HIP_TRY(hipMemcpy(g.data(), g27, g.size() * sizeof(double), hipMemcpyDeviceToHost));
-    std::vector<double> B((size_t)n * w, 0.0);
-    auto at = [&](long r, long c) -> double& { return B[(size_t)r * w + (c - r + bw)]; };
-    for (int k = 0; k < L.mz; ++k)
-        for (int j = 0; j < my; ++j)
-            for (int i = 0; i < mx; ++i) {
-                const long q = ((long)k * my + j) * mx + i;
-                for (int c = 0; c < 27; ++c) {
-                    const int oz = c / 9 - 1, oy = (c / 3) % 3 - 1, ox = c % 3 - 1;
-                    if (i + ox < 0 || i + ox >= mx || j + oy < 0 || j + oy >= my || k + oz < 0 || k + oz >= L.mz)
-                        continue;
-                    at(q, q + ((long)oz * my + oy) * mx + ox) = g[(size_t)c * n + q];
-                }
-            }
-    for (long kk = 0; kk < n; ++kk) {
-        const double piv = at(kk, kk);
-        if (piv == 0.0) return set_error(PETSC_ERR_LIB, "coarse LU: zero pivot in row %ld", kk);
-        const long iend = std::min<long>(kk + bw, n - 1);
-        for (long i = kk + 1; i <= iend; ++i) {
-            const double l = at(i, kk) / piv;
-            if (l == 0.0) continue;
-            at(i, kk) = l;
-            for (long j = kk + 1; j <= iend; ++j) at(i, j) -= l * at(kk, j);
-        }
-    }
-    if (!s->ms_band || s->ms_band_cap < (long)B.size()) {
-        P4G_TRY(dalloc(s, (void**)&s->ms_band, B.size() * sizeof(double)));
-        s->ms_band_cap = (long)B.size();
-    }
-    HIP_TRY(hipMemcpyAsync(s->ms_band, B.data(), B.size() * sizeof(double), hipMemcpyHostToDevice, st));
-    k_band_inverse<<<(n + 255) / 256, 256, 0, st>>>(n, bw, s->ms_band, e.Ainv);
-    LAUNCH_CHECK();
-    HIP_TRY(hipStreamSynchronize(st));   // B lives on the host stack
-    return 0;
-}
-
 struct MsRun {
     p4g_solver_s* s = nullptr;
     long n = 0;
@@ -179,10 +128,7 @@ static int ms_operator(p4g_solver_s* s, MsRun& R, bool fd) {
         P4G_TRY(R.fun(l, R.xl[l], R.fl[l]));
         P4G_TRY(ms_fdjac_level(s, R, l, R.xl[l], R.fl[l]));
     }
-    if (L > 0) {
-        HIP_TRY(hipStreamSynchronize(R.st));
-        P4G_TRY(coarse_factor_lu(s, s->lv[0], s->g27[0], e, R.st));
-    }
+    if (L > 0) P4G_TRY(coarse_factor_band(s, s->lv[0], s->g27[0], false, e, R.st));
     if (s->smoother == SM_CHEB)   // one level: the level smoother is the preconditioner
         for (int l = L > 0 ? 1 : 0; l <= L; ++l) P4G_TRY(estimate_level(s, l));
     return 0;

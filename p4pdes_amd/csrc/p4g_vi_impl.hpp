@@ -79,6 +79,69 @@ struct ViRun {
 
 static int asm_setup(p4g_solver_s* s, ViRun& R);
 
+// The coarsest level of a 27-plane operator, refactored at every Newton step:
+// band LU without pivoting (PETSc's serial coarse LU factors the diagonally
+// dominant Jacobians without row exchanges; of a symmetric positive definite
+// operator, spd, it is the Cholesky factor up to scaling), then the engine's
+// dense inverse.  Bands of 64 and more (long sides across x, 3D) are factored
+// as the set-up factors them, on the host.
+static int coarse_factor_band(p4g_solver_s* s, const LevelInfo& L, const double* g27, bool spd, Engine<double>& e,
+                              hipStream_t st) {
+    const int n = (int)L.n;
+    if (n > MAX_COARSE)
+        return set_error(PETSC_ERR_SUP, "coarsest grid has %d points (> %d); use more multigrid levels", n,
+                         MAX_COARSE);
+    if (!e.Ainv || e.n0 != n) return set_error(PETSC_ERR_LIB, "internal: coarse inverse of a different size");
+    const int mx = L.mx, my = L.my;
+    const int bw = L.dim == 3 ? mx * my + mx + 1 : (L.dim == 2 ? mx + 1 : 1);
+    const int w = 2 * bw + 1;
+    if (spd && bw >= 64) {
+        HIP_TRY(hipStreamSynchronize(st));
+        std::vector<double> Ainv;
+        P4G_TRY(coarse_factor(L, g27, Ainv));
+        return e.set_coarse_inverse(Ainv);
+    }
+    const size_t cap = (size_t)n * w + 1;               // and the pivot word
+    if (!s->ms_band || s->ms_band_cap < (long)cap) {
+        P4G_TRY(dalloc(s, (void**)&s->ms_band, cap * sizeof(double)));
+        s->ms_band_cap = (long)cap;
+    }
+    int* const info = (int*)(s->ms_band + (size_t)n * w);
+    k_band_fill<<<vblocks((long)n * w), 256, 0, st>>>(mx, my, n, bw, g27, spd ? 1 : 0, s->ms_band);
+    LAUNCH_CHECK();
+    int bad = 0;
+    if (bw < 64) {
+        k_band_lu<<<1, 1024, 0, st>>>(n, bw, s->ms_band, spd ? 1 : 0, info);
+        k_band_inverse<<<(n + 15) / 16, 64, 0, st>>>(n, bw, s->ms_band, e.Ainv);
+        LAUNCH_CHECK();
+        HIP_TRY(hipMemcpyAsync(&bad, info, sizeof(int), hipMemcpyDeviceToHost, st));
+        HIP_TRY(hipStreamSynchronize(st));
+    } else {
+        std::vector<double> B((size_t)n * w);
+        HIP_TRY(hipMemcpyAsync(B.data(), s->ms_band, B.size() * sizeof(double), hipMemcpyDeviceToHost, st));
+        HIP_TRY(hipStreamSynchronize(st));
+        auto at = [&](long r, long c) -> double& { return B[(size_t)r * w + (c - r + bw)]; };
+        for (long kk = 0; kk < n && !bad; ++kk) {
+            const double piv = at(kk, kk);
+            if (piv == 0.0) bad = (int)kk + 1;
+            const long iend = std::min<long>(kk + bw, n - 1);
+            for (long i = kk + 1; i <= iend; ++i) {
+                const double l = at(i, kk) / piv;
+                if (l == 0.0) continue;
+                at(i, kk) = l;
+                for (long j = kk + 1; j <= iend; ++j) at(i, j) -= l * at(kk, j);
+            }
+        }
+        HIP_TRY(hipMemcpyAsync(s->ms_band, B.data(), B.size() * sizeof(double), hipMemcpyHostToDevice, st));
+        k_band_inverse_wide<<<(n + 255) / 256, 256, 0, st>>>(n, bw, s->ms_band, e.Ainv);
+        LAUNCH_CHECK();
+        HIP_TRY(hipStreamSynchronize(st));   // B lives on the host stack
+    }
+    if (bad && spd) return set_error(PETSC_ERR_LIB, "coarse Cholesky: matrix not positive definite");
+    if (bad) return set_error(PETSC_ERR_LIB, "coarse LU: zero pivot in row %d", bad - 1);
+    return 0;
+}
+
 // the finest operator of the current active set and, under -pc_type mg, its
 // Galerkin coarse levels, coarse factor and Chebyshev bounds
 static int vi_operator(p4g_solver_s* s, ViRun& R) {
@@ -101,11 +164,7 @@ static int vi_operator(p4g_solver_s* s, ViRun& R) {
     for (int l = 0; l <= L; ++l)   // the pipelined SOR sweeps read the operator as packed records
         if (s->lv[l].pipe) sor9_pack(s->lv[l], s->g27[l], R.st);
     LAUNCH_CHECK();
-    if (L > 0) {
-        std::vector<double> Ainv;
-        P4G_TRY(coarse_factor(s->lv[0], s->g27[0], Ainv));
-        P4G_TRY(e.set_coarse_inverse(Ainv));
-    }
+    if (L > 0) P4G_TRY(coarse_factor_band(s, s->lv[0], s->g27[0], true, e, R.st));
     if (s->smoother == SM_CHEB)   // one level: the level smoother is the preconditioner
         for (int l = L > 0 ? 1 : 0; l <= L; ++l) P4G_TRY(estimate_level(s, l));
     return 0;
