@@ -155,6 +155,8 @@ int p4g_da_destroy(p4g_DA *da);
  *   -p4g_post_fuse auto|1|0 (auto and 1: levels where -p4g_lds applies,
  *       with two or more Chebyshev steps): the prolongation fused with the
  *       first post-smoothing step,
+ *   -p4g_tail 1|0 (default 1): the coarse levels of a V-cycle (65^2 or 17^3
+ *       points and below, constant coefficients, Jacobi) in one launch,
  *   -p4g_sor_pipeline 1|0 (default 1): SOR levels swept by pipelined
  *       strips, one launch per direction (else one per hyperplane).
  * Options and combinations the device path does not implement are rejected

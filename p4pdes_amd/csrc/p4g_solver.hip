@@ -33,6 +33,7 @@
 #include "p4g_internal.hpp"
 #include "p4g_kernels.hpp"
 #include "p4g_sor_kernels.hpp"
+#include "p4g_tail_kernels.hpp"
 
 using namespace p4g;
 
@@ -466,6 +467,8 @@ struct Engine {
     // steps the prolonged iterate would have to be stored for the Chebyshev
     // recurrence, and the fused kernel then loses to the separate passes)
     bool fuse_post = true;
+    bool tail_mode = true;     // -p4g_tail 1|0: the coarse end of a V-cycle in one launch (k_vtail)
+    bool tail_ready = false;   // its dynamic LDS size set
     // CG updates fused into stencil passes: the residual update into the
     // first kernel of the cycle (fuse_r), the direction update with the
     // operator apply (fuse_dir)
@@ -1161,6 +1164,80 @@ struct Engine {
         return stencil(nlev - 1, SrcArr<T>{pnew}, OutApplyDot<T>{w}, P4G_K_STENCIL_DOT, 2, nbs, false);
     }
 
+    // the largest level below the finest that k_vtail can take with all levels
+    // under it, or -1: vertex-nested constant-coefficient levels, V-cycles, up
+    // to kTailSteps smoothing steps, a direct coarse solve of few points, and
+    // three vectors a level within one compute unit's LDS.  Measured per
+    // cycle: 65^2 and below 69 us in 16 launches against 17 us in one; 17^3
+    // and below 45 us in 10 against 18 us.
+    int tail_level() const {
+        if (!tail_mode || sor || vi || vidiag || mf_op || cycles != 1 || coarse_its > 0 || nu > kTailSteps) return -1;
+        if (pctype != PCT_MG || nlev < 3 || !fuse_post || n0 > kTailCoarse) return -1;
+        size_t bytes = 0;
+        int top = -1;
+        for (int l = 0; l < nlev - 1 && l < kTailLevels; ++l) {
+            const LevelInfo& L = (*lv)[l];
+            if (L.dim < 2 || !zg_fusable(L)) break;
+            if (l > 0) {
+                const LevelInfo& C = (*lv)[l - 1];
+                if (L.mx != 2 * C.mx - 1 || L.my != 2 * C.my - 1 || (L.dim == 3 && L.mz != 2 * C.mz - 1)) break;
+            }
+            bytes += 3 * (size_t)L.n * sizeof(T);
+            if (bytes > kTailLds) break;
+            top = l;
+        }
+        return top > 0 ? top : -1;
+    }
+    // x = the V-cycle's correction for b on level `top`, from zero
+    int vtail(int top, const T* b, T* x) {
+        TailArgs<T> a;
+        a.nl = top + 1;
+        a.nu = nu;
+        a.n0 = n0;
+        a.Ainv = Ainv;
+        a.b = b;
+        a.x = x;
+        int off = 0;
+        for (int l = 0; l <= top; ++l) {
+            const LevelInfo& L = (*lv)[l];
+            TailLevel<T>& t = a.lv[l];
+            const OpConst<T> o = opc(L, jacobi != 0);
+            t.mx = L.mx; t.my = L.my; t.mz = L.dim == 3 ? L.mz : 1; t.n = (int)L.n; t.off = off;
+            off += 3 * (int)L.n;
+            t.d = o.d; t.sx = o.sx; t.sy = o.sy; t.sz = o.sz; t.idg = o.id; t.diff = o.diff;
+            // smooth()'s recurrence coefficients
+            double sc = rich_scale, mu = 0.0, op = 0.0, c0 = 1.0, c1 = 0.0;
+            if (l > 0 && smoother == SM_CHEB) {
+                sc = 2.0 / (L.emax + L.emin);
+                const double alpha = 1.0 - sc * L.emin;
+                mu = 1.0 / alpha;
+                op = 2.0 / alpha;
+                c1 = mu;
+            }
+            for (int m = 0; m < kTailSteps; ++m) {
+                t.c0[m] = T(0); t.c1[m] = T(1); t.c2[m] = T(sc);
+                if (m > 0 && smoother == SM_CHEB) {
+                    const double ckp1 = 2.0 * mu * c1 - c0, omega = op * c1 / ckp1;
+                    c0 = c1;
+                    c1 = ckp1;
+                    t.c0[m] = T(1.0 - omega); t.c1[m] = T(omega); t.c2[m] = T(omega * sc);
+                }
+            }
+        }
+        const size_t lds = (size_t)off * sizeof(T);
+        hipStream_t s = cx->stream;
+        const bool d3 = (*lv)[0].dim == 3;
+        const void* f = d3 ? (const void*)&k_vtail<T, 3> : (const void*)&k_vtail<T, 2>;
+        if (!tail_ready) {
+            HIP_TRY(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTailLds));
+            tail_ready = true;
+        }
+        return cx->launch(P4G_K_COARSE, false, 2.0 * (*lv)[top].n * sizeof(T) + 8.0 * n0 * n0, [&] {
+            if (d3) k_vtail<T, 3><<<1, kTailThreads, lds, s>>>(a);
+            else k_vtail<T, 2><<<1, kTailThreads, lds, s>>>(a);
+        });
+    }
+
     // PCMGMCycle: b, x of level l (x zero on entry when xzero).  On the
     // finest level with dots, the last kernel fuses (x,b) and (x,x).
     int mcycle(int l, const T* b, T* x, bool xzero, bool dots, long* nb) {
@@ -1176,6 +1253,7 @@ struct Engine {
             }
             return 0;
         }
+        if (l < nlev - 1 && xzero && l == tail_level()) return vtail(l, b, x);
         const LevelInfo& L = (*lv)[l];
         Dev& d = dv[l];
         const bool jac = jacobi != 0;
@@ -1938,6 +2016,7 @@ struct p4g_solver_s {
     long* asm_row = nullptr;          // per owned row: [inverse row offset, index offset, count, vertex]
     long asm_nrows = 0;
     size_t asm_cap_idx = 0, asm_cap_inv = 0, asm_cap_row = 0;
+    bool tail = true;                 // -p4g_tail 1|0: the coarse end of a V-cycle in one launch
     int post_fuse = -1;               // -p4g_post_fuse auto|1|0: prolongation + first of several post steps
     bool sor_test_stall = false;      // -p4g_sor_test_stall: every pipelined-SOR wait gives up at once
     bool sor_pipeline = true;         // -p4g_sor_pipeline 1|0: 3D SOR by pipelined strips (else hyperplanes)
@@ -2424,6 +2503,7 @@ static int configure(p4g_solver_s* s) {
         s->rr_planes = o.geti("p4g_rr_planes", 0);
         if (s->rr_planes < 0 || s->rr_planes > 64)
             return set_error(PETSC_ERR_ARG_OUTOFRANGE, "-p4g_rr_planes must be in 0..64");
+        s->tail = o.getb("p4g_tail", true);
         P4G_TRY(tri(o.gets("p4g_post_fuse", "auto"), "p4g_post_fuse", s->post_fuse));
         const std::string both = o.gets("p4g_fuse_cg", "auto");
         P4G_TRY(tri(both, "p4g_fuse_cg", s->fuse_r));
@@ -2723,6 +2803,7 @@ int solver_setup(p4g_solver_s* s) {
         e->rr_rows = s->rr_rows;
         e->rr_planes = s->rr_planes;
         e->post2_mode = s->post_fuse;
+        e->tail_mode = s->tail;
     };
     if (F.var) {
         const size_t nc = F.kcell.size();
