@@ -59,12 +59,15 @@ enum { PCT_MG = 0, PCT_JACOBI, PCT_NONE, PCT_ILU, PCT_ASM };
 enum { SM_CHEB = 0, SM_RICH };
 enum { NT_PRECOND = 0, NT_UNPRECOND, NT_NATURAL };
 
-// planes per marching chunk: short chunks on small grids (latency-bound),
-// longer ones on large grids (fewer re-read halo planes)
-// marching chunk: one plane per thread on small grids (latency-bound, want
-// parallelism), longer chunks on large ones (fewer halo re-reads)
+// marching chunk: one plane (row in 2D) per thread on small grids
+// (latency-bound, want parallelism), longer chunks on large ones (fewer halo
+// re-reads).  A 2D row is one wave per 128 points, so a 2D grid fills the
+// chip's 1024 SIMDs from about 400^2 on and takes the short chunks to 800^2
+// (129^2: direction pass 8.2 us with four rows a thread, prolongation and
+// smoothing 15.1 us with eight).
 static inline int kchf(int dim, int my, int mz) {
-    const int slow = dim == 3 ? mz : (dim == 2 ? my : 1);
+    if (dim == 2) return my >= 1600 ? 8 : (my >= 800 ? 4 : (my >= 400 ? 2 : 1));
+    const int slow = dim == 3 ? mz : 1;
     return slow >= 400 ? 8 : (slow >= 100 ? 4 : 1);
 }
 constexpr int VBLOCKS = 2048;      // blocks of the grid-stride vector kernels
@@ -381,7 +384,8 @@ static dim3 stencil_grid_v(int dim, int mx, int my, int mz, int V) {
 // chunks are longer than those of the stencil passes (3D, 6-row blocks:
 // 257^3 120 us at 16 planes, 134 us at 8; 513^3 855 us at 16, 939 us at 8)
 static inline int kch_fused(int dim, int my, int mz) {
-    const int slow = dim == 3 ? mz : my;
+    if (dim == 2) return 2 * kchf(dim, my, mz);
+    const int slow = dim == 3 ? mz : 1;
     return slow >= 200 ? 16 : std::min(16, 2 * kchf(dim, my, mz));
 }
 template <typename T>
@@ -416,7 +420,8 @@ static dim3 transfer_grid(int dim, int mxc, int my, int mz, int kch) {
 // coarse grid (my, mz): each is two fine planes read (fine 257^3: 45 us at
 // 1-2, 48 us at 4; fine 513^3: 293 us at 4, 303 us at 2 or 8)
 static inline int kch_restrict(int dim, int my, int mz) {
-    const int slow = dim == 3 ? mz : (dim == 2 ? my : 1);
+    if (dim == 2) return my >= 800 ? 4 : (my >= 400 ? 2 : 1);
+    const int slow = dim == 3 ? mz : 1;
     return slow >= 200 ? 4 : (slow >= 100 ? 2 : 1);
 }
 
