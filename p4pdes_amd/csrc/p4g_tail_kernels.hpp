@@ -17,7 +17,10 @@ namespace p4g {
 
 constexpr int kTailLevels = 8, kTailSteps = 4, kTailThreads = 1024;
 constexpr size_t kTailLds = 156 * 1024;   // of the compute unit's 160 KiB
-constexpr int kTailCoarse = 512;          // coarsest points: their inverse is read by this one workgroup
+// coarsest points: their inverse is read by this one workgroup, n^2 words at
+// one compute unit's rate (a tail over 13x11x9 and 210 coarsest points took
+// 29 us, the 7 launches that it stood for 20)
+constexpr int kTailCoarse = 128;
 
 template <typename T>
 struct TailLevel {
@@ -126,16 +129,24 @@ __global__ void __launch_bounds__(kTailThreads) k_vtail(TailArgs<T> A) {
         }
         __syncthreads();
     }
-    {   // the coarsest level: x = A^-1 b, a wave per row, in FP64
+    {   // the coarsest level: x = A^-1 b in FP64, a wave per row, four rows in flight
         const TailLevel<T>& L = A.lv[0];
         const T* const b = lds + L.off;
         T* const x = top == 0 ? A.x : lds + L.off + L.n;
         const int lane = tid & 63;
-        for (int row = tid >> 6; row < A.n0; row += kTailThreads / 64) {
-            double s = 0.0;
-            for (int c = lane; c < A.n0; c += 64) s += A.Ainv[(long)row * A.n0 + c] * double(b[c]);
-            s = wave_sum(s);
-            if (lane == 0) x[row] = T(s);
+        constexpr int WV = kTailThreads / 64, RW = 4;
+        for (int row = tid >> 6; row < A.n0; row += RW * WV) {
+            double s[RW] = {};
+            for (int c = lane; c < A.n0; c += 64) {
+                const double bc = double(b[c]);
+#pragma unroll
+                for (int h = 0; h < RW; ++h) s[h] += A.Ainv[(long)min(row + h * WV, A.n0 - 1) * A.n0 + c] * bc;
+            }
+#pragma unroll
+            for (int h = 0; h < RW; ++h) {
+                const double t = wave_sum(s[h]);
+                if (lane == 0 && row + h * WV < A.n0) x[row + h * WV] = T(t);
+            }
         }
     }
     __syncthreads();
