@@ -102,6 +102,9 @@ struct VecOf {
 // differences of close values are exact, where d uc - sum cancels.
 template <typename T>
 struct OpConst {
+    static constexpr bool CELLS = false;
+    template <int V>
+    struct Cells {};
     T d, db, sx, sy, sz;   // interior diagonal, boundary diagonal, couplings
     T id, idb;             // Jacobi: 1/d, 1/db (or 1 when no Jacobi scaling)
     int diff = 0;          // 1: difference form (requires d = 2(sx+sy+sz))
@@ -125,10 +128,42 @@ struct OpVar {
     int cx, cy, cz;             // cell counts
     T ax, ay, az;               // dvol/h^2 per direction
     int jac;                    // 1: Jacobi scaling, 0: identity
+    const T* __restrict__ idg = nullptr;   // reciprocal diagonal per point, for passes that take it from memory
+    static constexpr bool CELLS = true;
     __device__ __forceinline__ T cell(int i, int j, int k) const {
         return kc[((long)k * cy + j) * cx + i];
     }
-    __device__ __forceinline__ void bnd(int i, int j, int k, T u, T& Au, T& idg) const {
+    // One cell layer's values around V consecutive points i0.. of row j: cell
+    // rows j-1 and j, cell columns i0-1 .. i0+V-1.  A marching pass loads each
+    // layer once and uses it for the planes below and above it, where a point
+    // read its eight cells one by one.  What bounds these passes is registers:
+    // loading a layer a plane ahead took 141-145 and left one block of eight
+    // waves a compute unit (257^3: the CG operator pass 305 us against 254
+    // with single cells); without, and held to 128 (4 waves a SIMD, a few
+    // spills), it is 243, and the post-smoothing pass 353 against 386.
+    template <int V>
+    struct Cells {
+        T v[2][V + 1];
+    };
+    template <int V>
+    __device__ __forceinline__ Cells<V> cells(int i0, int j, int k) const {
+        Cells<V> r;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const T* const p = kc + ((long)k * cy + (j - 1 + h)) * cx + (i0 - 1);
+            if (i0 + V - 1 < cx) {
+                const TV<T, V> t = ldv<T, V>(p);
+#pragma unroll
+                for (int e = 0; e < V; ++e) r.v[h][e] = t.v[e];
+                r.v[h][V] = p[V];
+            } else {             // the row's end
+#pragma unroll
+                for (int e = 0; e <= V; ++e) r.v[h][e] = p[min(e, cx - i0)];
+            }
+        }
+        return r;
+    }
+    __device__ __forceinline__ void bnd(int i, int j, int k, T u, T& Au, T& idg_) const {
         T s = T(0);
         int cnt = 0;
         for (int dk = -1; dk <= 0; ++dk)
@@ -141,14 +176,23 @@ struct OpVar {
                 }
         T dg = T(2) * (ax + ay + az) * (s / T(cnt));
         Au = dg * u;
-        idg = jac ? T(1) / dg : T(1);
+        idg_ = jac ? T(1) / dg : T(1);
     }
-    __device__ __forceinline__ void interior(int i, int j, int k, T uc, T w, T e, T s, T n,
-                                             T dn, T up, T& Au, T& idg) const {
-        const T c000 = cell(i - 1, j - 1, k - 1), c100 = cell(i, j - 1, k - 1);
-        const T c010 = cell(i - 1, j, k - 1), c110 = cell(i, j, k - 1);
-        const T c001 = cell(i - 1, j - 1, k), c101 = cell(i, j - 1, k);
-        const T c011 = cell(i - 1, j, k), c111 = cell(i, j, k);
+    // a boundary point of an interior row and plane (i = 0 or mx - 1): its
+    // four cells, column e of the layers below and above
+    template <int V>
+    __device__ __forceinline__ void bndx(int e, const Cells<V>& lo, const Cells<V>& hi, T u, T& Au, T& idg_) const {
+        const T s = lo.v[0][e] + lo.v[1][e] + hi.v[0][e] + hi.v[1][e];
+        const T dg = T(2) * (ax + ay + az) * (s / T(4));
+        Au = dg * u;
+        idg_ = jac ? T(1) / dg : T(1);
+    }
+    // an interior point, e-th of the V whose layers below and above are given
+    template <int V>
+    __device__ __forceinline__ void interiorc(int e, const Cells<V>& lo, const Cells<V>& hi, T uc, T w, T ea, T s, T n,
+                                              T dn, T up, T& Au, T& idg_) const {
+        const T c000 = lo.v[0][e], c100 = lo.v[0][e + 1], c010 = lo.v[1][e], c110 = lo.v[1][e + 1];
+        const T c001 = hi.v[0][e], c101 = hi.v[0][e + 1], c011 = hi.v[1][e], c111 = hi.v[1][e + 1];
         const T q = T(0.25);
         const T kw = q * (c000 + c010 + c001 + c011) * ax;
         const T ke = q * (c100 + c110 + c101 + c111) * ax;
@@ -157,8 +201,12 @@ struct OpVar {
         const T kd = q * (c000 + c100 + c010 + c110) * az;
         const T ku = q * (c001 + c101 + c011 + c111) * az;
         const T dg = kw + ke + ks + kn + kd + ku;
-        Au = dg * uc - kw * w - ke * e - ks * s - kn * n - kd * dn - ku * up;
-        idg = jac ? T(1) / dg : T(1);
+        Au = dg * uc - kw * w - ke * ea - ks * s - kn * n - kd * dn - ku * up;
+        idg_ = jac ? T(1) / dg : T(1);
+    }
+    __device__ __forceinline__ void interior(int i, int j, int k, T uc, T w, T e, T s, T n, T dn, T up, T& Au,
+                                             T& idg_) const {
+        interiorc<1>(0, cells<1>(i, j, k - 1), cells<1>(i, j, k), uc, w, e, s, n, dn, up, Au, idg_);
     }
 };
 
@@ -195,6 +243,25 @@ struct SrcZero {                      // u = 0 (first smoothing step from a zero
         TV<T, V> r;
 #pragma unroll
         for (int e = 0; e < V; ++e) r.v[e] = T(0);
+        return r;
+    }
+    __device__ __forceinline__ void put(long, T) const {}
+    template <int V>
+    __device__ __forceinline__ void putv(long, const TV<T, V>&) const {}
+};
+
+template <typename T>
+struct SrcMul {                       // u = s (d b): a Jacobi step from a zero guess
+    const T* __restrict__ b;
+    const T* __restrict__ d;
+    T s;
+    __device__ __forceinline__ T load(long q) const { return s * (d[q] * b[q]); }
+    template <int V>
+    __device__ __forceinline__ TV<T, V> loadv(long q) const {
+        TV<T, V> r = ldv<T, V>(b + q);
+        const TV<T, V> dd = ldv<T, V>(d + q);
+#pragma unroll
+        for (int e = 0; e < V; ++e) r.v[e] = s * (dd.v[e] * r.v[e]);
         return r;
     }
     __device__ __forceinline__ void put(long, T) const {}
@@ -398,6 +465,18 @@ typedef FoldListT<float> FoldList;
 // marching pass load them ahead: pre / pre1 load them at q (V points or
 // one), pointvp / pointp consume them.  Those arrays must not be written by
 // the pass's source.
+
+template <typename T>
+struct OutRecipDiag {                 // the Jacobi factor of every row
+    T* __restrict__ id;
+    static constexpr int NDOT = 0, NPRE = 0;
+    __device__ __forceinline__ void point(long q, T, T, T idg, double&, double&) const { id[q] = idg; }
+    template <int V>
+    __device__ __forceinline__ void pointv(long q, const TV<T, V>&, const TV<T, V>&, const TV<T, V>& idg, double&,
+                                           double&) const {
+        stv<T, V>(id + q, idg);
+    }
+};
 
 template <typename T>
 struct OutApplyDot {                  // w = A u ; acc0 += u.w
@@ -836,6 +915,13 @@ __device__ __forceinline__ void stencil_vec(int bx, int by, int bz, int mx, int 
     // rows j-1, j+1 of plane m are read by interior rows of interior planes
     auto snok = [&](int m) -> bool { return PSN && act && !jb && m > 0 && m < M - 1; };
     const int mlast = min(m1, M - 1);  // last plane whose centre row is read
+    // the cell layers below and above plane m (OpVar, 3D)
+    typename Op::template Cells<V> cl{}, ch{};
+    auto CL = [&](int p, typename Op::template Cells<V>& c) {
+        if constexpr (Op::CELLS)
+            if (act && !jb && p >= 0 && p < M - 1) c = op.template cells<V>(i0, j, p);
+    };
+    CL(m0 - 1, ch);
     long q = base + (long)m0 * sm + i0;
     TV<T, V> ud = zv;
     TV<T, V> sc = zv, nc = zv;
@@ -853,6 +939,10 @@ __device__ __forceinline__ void stencil_vec(int bx, int by, int bz, int mx, int 
     for (int m = m0; m < m1; ++m, q += sm) {
         if (act && m + PD <= mlast)
             LR(q + PD * sm, m + PD < m1, ru[PD - 1], rx[PD - 1], ro[PD - 1], rox[PD - 1]);
+        if constexpr (Op::CELLS) {
+            cl = ch;
+            CL(m, ch);
+        }
         TV<T, V> sn = zv, nn = zv;
         if (m + 1 < m1 && snok(m + 1)) {
             if (ms) sn = LV(q + sm - sy);
@@ -904,12 +994,17 @@ __device__ __forceinline__ void stencil_vec(int bx, int by, int bz, int mx, int 
                     const int i = i0 + e;
                     if (e < ne) {
                         if (i == mx - 1) {
-                            op.bnd(i, jj, kk, uc.v[e], Au.v[e], idg.v[e]);
+                            if constexpr (Op::CELLS) op.template bndx<V>(e, cl, ch, uc.v[e], Au.v[e], idg.v[e]);
+                            else op.bnd(i, jj, kk, uc.v[e], Au.v[e], idg.v[e]);
                         } else {
                             const T w = e == 0 ? (i - 1 > 0 ? wv : z0) : uc.v[e > 0 ? e - 1 : 0];
                             const T east = i + 1 < mx - 1 ? (e == V - 1 ? ev : uc.v[e < V - 1 ? e + 1 : 0]) : z0;
-                            op.interior(i, jj, kk, uc.v[e], w, east, sv.v[e], nv.v[e], dn.v[e], up.v[e], Au.v[e],
-                                        idg.v[e]);
+                            if constexpr (Op::CELLS)
+                                op.template interiorc<V>(e, cl, ch, uc.v[e], w, east, sv.v[e], nv.v[e], dn.v[e],
+                                                         up.v[e], Au.v[e], idg.v[e]);
+                            else
+                                op.interior(i, jj, kk, uc.v[e], w, east, sv.v[e], nv.v[e], dn.v[e], up.v[e], Au.v[e],
+                                            idg.v[e]);
                         }
                     }
                 }
@@ -926,7 +1021,12 @@ __device__ __forceinline__ void stencil_vec(int bx, int by, int bz, int mx, int 
                 const T u0 = PEX ? cx : src.load(q - 1);
                 T A0, i00;
                 src.put(q - 1, u0);
-                op.bnd(0, jj, kk, u0, A0, i00);
+                if constexpr (Op::CELLS) {
+                    if (jb || m == 0 || m == M - 1) op.bnd(0, jj, kk, u0, A0, i00);
+                    else op.template bndx<V>(0, cl, ch, u0, A0, i00);
+                } else {
+                    op.bnd(0, jj, kk, u0, A0, i00);
+                }
                 if constexpr (NP > 0) out.pointp(q - 1, u0, A0, i00, cox, a0, a1);
                 else out.point(q - 1, u0, A0, i00, a0, a1);
             }
@@ -989,7 +1089,7 @@ __device__ __forceinline__ void stencil_body(int bx, int by, int bz, int mx, int
 }
 
 template <typename T, int DIM, class Op, class Src, class Out>
-__global__ void __launch_bounds__(NT)
+__global__ void __launch_bounds__(NT, Op::CELLS ? 4 : 1)   // (4 waves a SIMD: see OpVar::cells)
 k_stencil(int mx, int my, int mz, int kch, Op op, Src src, Out out, double* __restrict__ part) {
     double a0 = 0.0, a1 = 0.0;
     const Tile tl = xcd_tile();
@@ -1863,31 +1963,50 @@ __device__ __forceinline__ void prolong_smooth_3d(int bx, int by, int bz, int mx
         if (!odd) return a;
         return mix3(a, fin1(r.v1, r.x1));
     };
+    // base values on the own row: the lane's pair and the edge lane's extra
+    // value; ZG with a variable operator scales the base by its reciprocal
+    // diagonal (d, dx)
+    constexpr bool DG = ZG && Op::CELLS;
     struct BP {
         T2<T> p;
         T x;
+        T2<T> d;
+        T dx;
     };
-    // base values on the own row: the lane's pair and the edge lane's extra value
+    const BP bp00{zero2, z0, zero2, z0};
     auto bload = [&](long qq) -> BP {
-        BP r{zero2, z0};
+        BP r = bp00;
         if (la) {
             r.p = ld2(xb + qq);
             if (lane == 0) r.x = xb[qq - 1];
             else if (lane == TX - 1 && i1 + 1 < mx) r.x = xb[qq + 2];
+            if constexpr (DG) {
+                r.d = ld2(op.idg + qq);
+                if (lane == 0) r.dx = op.idg[qq - 1];
+                else if (lane == TX - 1 && i1 + 1 < mx) r.dx = op.idg[qq + 2];
+            }
         }
         return r;
     };
-    auto tpb = [&](const T3<T>& P, const T2<T>& bb) -> T2<T> {
-        const T b0 = ZG ? c * bb.a : bb.a, b1 = ZG ? c * bb.b : bb.b;
+    auto sc1 = [&](T v, T d) -> T { return DG ? c * (d * v) : (ZG ? c * v : v); };
+    auto tpb = [&](const T3<T>& P, const BP& bb) -> T2<T> {
+        const T b0 = sc1(bb.p.a, bb.d.a), b1 = sc1(bb.p.b, bb.d.b);
         return T2<T>{b0 + h * (P.w + P.v), b1 + P.v};
     };
-    auto scb = [&](T v) -> T { return ZG ? c * v : v; };
+    auto scb = [&](const BP& bb) -> T { return sc1(bb.x, bb.dx); };
+    // the cell layers below and above plane k (OpVar)
+    typename Op::template Cells<2> cl{}, ch{};
+    auto CL = [&](int p, typename Op::template Cells<2>& cc) {
+        if constexpr (Op::CELLS)
+            if (la && !halo && j > 0 && j < my - 1 && p >= 0 && p < mz - 1) cc = op.template cells<2>(i0, j, p);
+    };
+    CL(k0 - 1, ch);
     int Ka = k0 >> 1;
     long q = (long)k0 * sz + (long)(rowok ? j : 0) * sy + i0;
     T3<T> Ya = zero3, Yb = zero3, Pc = zero3;
     CR cn = cr0;
     T2<T> tc = zero2, td = zero2;
-    BP bp0{zero2, z0}, bp1{zero2, z0};
+    BP bp0 = bp00, bp1 = bp00;
     if (rowok) {
         Ya = cfin(craw(Ka));
         if (Ka + 1 < mzc) Yb = cfin(craw(Ka + 1));
@@ -1895,19 +2014,23 @@ __device__ __forceinline__ void prolong_smooth_3d(int bx, int by, int bz, int mx
         Pc = (k0 & 1) ? mix3(Ya, Yb) : Ya;
         bp0 = bload(q);
         if (k0 + 1 < mz) bp1 = bload(q + sz);
-        tc = tpb(Pc, bp0.p);
+        tc = tpb(Pc, bp0);
         if (!halo && k0 > 0) {
             const T3<T> Pd = (k0 & 1) ? Ya : mix3(cfin(craw(Ka - 1)), Ya);
             const BP bd = bload(q - sz);
-            td = tpb(Pd, bd.p);
+            td = tpb(Pd, bd);
         }
     }
     const bool jb = (j == 0) || (j == my - 1);
     for (int k = k0; k < k1; ++k, q += sz) {
         T3<T> Pu = zero3;
         T2<T> tu = zero2;
-        BP bp2{zero2, z0};
+        BP bp2 = bp00;
         if (rowok) {
+            if constexpr (Op::CELLS) {
+                cl = ch;
+                CL(k, ch);
+            }
             if (k + 2 < mz) bp2 = bload(q + 2 * sz);
             if ((k >> 1) != Ka) {
                 Ka = k >> 1;
@@ -1917,7 +2040,7 @@ __device__ __forceinline__ void prolong_smooth_3d(int bx, int by, int bz, int mx
             }
             if (k + 1 < mz) {
                 Pu = (k & 1) ? Yb : mix3(Ya, Yb);
-                tu = tpb(Pu, bp1.p);
+                tu = tpb(Pu, bp1);
             }
             if (act) tbuf[k & 1][w][lane] = tc;
         }
@@ -1932,17 +2055,27 @@ __device__ __forceinline__ void prolong_smooth_3d(int bx, int by, int bz, int mx
             const T2<T> ts = (need_sn && j - 1 > 0) ? tbuf[k & 1][w - 1][lane] : zero2;
             const T2<T> tn = (need_sn && j + 1 < my - 1) ? tbuf[k & 1][w + 1][lane] : zero2;
             const T2<T> tdd = (k - 1 > 0) ? td : zero2, tuu = (k + 1 < mz - 1) ? tu : zero2;
-            if (lane == 0 && i0 - 1 > 0) wv = scb(bp0.x) + Pc.w;
-            if (lane == TX - 1 && i1 + 1 < mx - 1) ev = scb(bp0.x) + h * (Pc.v + Pc.e);
+            if (lane == 0 && i0 - 1 > 0) wv = scb(bp0) + Pc.w;
+            if (lane == TX - 1 && i1 + 1 < mx - 1) ev = scb(bp0) + h * (Pc.v + Pc.e);
             T Aa, Ab, ia, ib;
             if (jb || k == 0 || k == mz - 1) {
                 op.bnd(i0, j, k, tc.a, Aa, ia);
                 op.bnd(i1, j, k, tc.b, Ab, ib);
             } else {
-                op.interior(i0, j, k, tc.a, i0 - 1 > 0 ? wv : z0, i1 < mx - 1 ? tc.b : z0, ts.a, tn.a, tdd.a, tuu.a,
-                            Aa, ia);
-                if (i1 == mx - 1) op.bnd(i1, j, k, tc.b, Ab, ib);
-                else op.interior(i1, j, k, tc.b, tc.a, i1 + 1 < mx - 1 ? ev : z0, ts.b, tn.b, tdd.b, tuu.b, Ab, ib);
+                const T w0 = i0 - 1 > 0 ? wv : z0, e0 = i1 < mx - 1 ? tc.b : z0, e1 = i1 + 1 < mx - 1 ? ev : z0;
+                if constexpr (Op::CELLS) {
+                    op.template interiorc<2>(0, cl, ch, tc.a, w0, e0, ts.a, tn.a, tdd.a, tuu.a, Aa, ia);
+                    if (i1 == mx - 1) op.template bndx<2>(1, cl, ch, tc.b, Ab, ib);
+                    else op.template interiorc<2>(1, cl, ch, tc.b, tc.a, e1, ts.b, tn.b, tdd.b, tuu.b, Ab, ib);
+                } else {
+                    op.interior(i0, j, k, tc.a, w0, e0, ts.a, tn.a, tdd.a, tuu.a, Aa, ia);
+                    if (i1 == mx - 1) op.bnd(i1, j, k, tc.b, Ab, ib);
+                    else op.interior(i1, j, k, tc.b, tc.a, e1, ts.b, tn.b, tdd.b, tuu.b, Ab, ib);
+                }
+            }
+            if constexpr (DG) {
+                ia = bp0.d.a;
+                ib = bp0.d.b;
             }
             const TV<T, 2> uu{{tc.a, tc.b}}, AA{{Aa, Ab}}, II{{ia, ib}};
             // with ZG the base is the output's b, its one per-point array
@@ -1954,8 +2087,13 @@ __device__ __forceinline__ void prolong_smooth_3d(int bx, int by, int bz, int mx
                 out.template pointv<2>(q, uu, AA, II, a0, a1);
             }
             if (I == 1) {      // fine 0: a boundary point
-                const T t0 = scb(bp0.x) + Pc.w;
-                op.bnd(0, j, k, t0, Aa, ia);
+                const T t0 = scb(bp0) + Pc.w;
+                if constexpr (Op::CELLS) {
+                    if (jb || k == 0 || k == mz - 1) op.bnd(0, j, k, t0, Aa, ia);
+                    else op.template bndx<2>(0, cl, ch, t0, Aa, ia);
+                } else {
+                    op.bnd(0, j, k, t0, Aa, ia);
+                }
                 if constexpr (ZG) out.pointp(q - 1, t0, Aa, ia, &bp0.x, a0, a1);
                 else out.point(q - 1, t0, Aa, ia, a0, a1);
             }

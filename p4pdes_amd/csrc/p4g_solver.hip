@@ -496,6 +496,7 @@ struct Engine {
     struct Dev {
         T *x = nullptr, *b = nullptr, *r = nullptr, *t[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
         T* kc = nullptr;
+        T* idg = nullptr;   // variable coefficients, V(1,1): the reciprocal diagonal
     };
     std::vector<Dev> dv;
     double* Ainv = nullptr;   // dense inverse of the coarsest operator
@@ -582,6 +583,17 @@ struct Engine {
                 P4G_TRY(alloc(&d.kc, ncell));
                 std::vector<T> tmp(L.kcell.begin(), L.kcell.end());
                 HIP_TRY(hipMemcpy(d.kc, tmp.data(), ncell * sizeof(T), hipMemcpyHostToDevice));
+                // a cycle's zero-guess step is then formed where it is read
+                // (mcycle): 257^3, the step's own pass 148 and the residual's
+                // 187 us before, one pass of 286 us now
+                if (pctype == PCT_MG && l > 0 && nu == 1 && L.dim == 3) {
+                    P4G_TRY(alloc(&d.idg, L.n));
+                    OpVar<T> o = opv(l, jacobi != 0);
+                    k_stencil<T, 3, OpVar<T>, SrcZero<T>, OutRecipDiag<T>>
+                        <<<stencil_grid<T>(3, L.mx, L.my, L.mz), stencil_block(3), 0, cx->stream>>>(
+                            L.mx, L.my, L.mz, kchf(3, L.my, L.mz), o, SrcZero<T>{}, OutRecipDiag<T>{d.idg}, cx->part);
+                    LAUNCH_CHECK();
+                }
             }
         }
         P4G_TRY(alloc(&r, F.n));
@@ -628,6 +640,7 @@ struct Engine {
         OpVar<T> o;
         o.kc = dv[l].kc; o.cx = L.cx; o.cy = L.cy; o.cz = L.cz;
         o.ax = T(L.ax); o.ay = T(L.ay); o.az = T(L.az); o.jac = jac ? 1 : 0;
+        o.idg = dv[l].idg;
         return o;
     }
 
@@ -1173,8 +1186,8 @@ struct Engine {
     // under it, or -1: vertex-nested constant-coefficient levels, V-cycles, up
     // to kTailSteps smoothing steps, a direct coarse solve of few points, and
     // three vectors a level within one compute unit's LDS.  Measured per
-    // cycle: 65^2 and below 69 us in 16 launches against 17 us in one; 17^3
-    // and below 45 us in 10 against 18 us.
+    // cycle: 65^2 and below 69 us in 16 launches against 22 us in one; 17^3
+    // and below 45 us in 10 against 24 us.
     int tail_level() const {
         if (!tail_mode || sor || vi || vidiag || mf_op || cycles != 1 || coarse_its > 0 || nu > kTailSteps) return -1;
         if (pctype != PCT_MG || nlev < 3 || !fuse_post || n0 > kTailCoarse) return -1;
@@ -1285,6 +1298,9 @@ struct Engine {
                 P4G_TRY(stencil(l, SrcArr<T>{b}, OR{T(s * idg), OutResid<T, 0>{b, d.r}}, P4G_K_RESID_ZG, 2, nullptr,
                                 jac));
             }
+        } else if (xzero && nu == 1 && d.idg && fuse_post) {   // variable diagonal: u = s D^-1 b formed on the fly
+            zgf = true;
+            P4G_TRY(stencil(l, SrcMul<T>{b, d.idg, T(s)}, OutResid<T, 0>{b, d.r}, P4G_K_RESID_ZG, 3, nullptr, jac));
         } else {
             xpre = d.t[3] ? d.t[3] : d.t[0];
             if (xpre == x && !xzero) return set_error(PETSC_ERR_LIB, "internal buffer aliasing");
@@ -1305,8 +1321,9 @@ struct Engine {
         const T* pre = zgf ? b : xpre;
         if (L.dim >= 2 && fuse_post && nu == 1 && !L.gal && !sor) {
             // the post-smoothing step reads the prolonged iterate on the fly
-            if (dots) P4G_TRY(post_first<true>(l, zgf, pre, T(s * idg), c.x, b, x, T(s), nb));
-            else P4G_TRY(post_first<false>(l, zgf, pre, T(s * idg), c.x, b, x, T(s), nb));
+            const T cz = T(L.var ? s : s * idg);   // (a variable diagonal comes from d.idg)
+            if (dots) P4G_TRY(post_first<true>(l, zgf, pre, cz, c.x, b, x, T(s), nb));
+            else P4G_TRY(post_first<false>(l, zgf, pre, cz, c.x, b, x, T(s), nb));
             return 0;
         }
         if (post2_fusable(L) && !zgf) {
