@@ -135,12 +135,14 @@ static void sor_pipe_run(const LevelInfo& L, SorPipe* P, const double* r, double
     }
     const Sor2Args A{L.mx, L.my, P->Tp, P->ns, L.d, L.db, L.sx, L.sy, P->pk, P->inv, r, P->S, z, P->yh, c};
     if (P->kind == SOR_9PT) {
-        k_sor2<true, false><<<P->ns * kXcds, 64, 0, st>>>(A);
-        k_sor2<true, true><<<P->ns * kXcds, 64, 0, st>>>(A);
+        typedef Sor2<true> G;
+        k_sor2<true, false><<<G::blocks(P->ns), G::NT, G::LDS, st>>>(A);
+        k_sor2<true, true><<<G::blocks(P->ns), G::NT, G::LDS, st>>>(A);
     } else {
-        const int nb = (2 * (L.mx + L.my) + 255) / 256;      // boundary rows, four points a lane
-        k_sor2<false, false><<<P->ns * kXcds + nb, 64, 0, st>>>(A);
-        k_sor2<false, true><<<P->ns * kXcds, 64, 0, st>>>(A);
+        typedef Sor2<false> G;
+        const int nb = (2 * (L.mx + L.my) + 4 * G::NT - 1) / (4 * G::NT);      // boundary rows, four points a lane
+        k_sor2<false, false><<<G::blocks(P->ns) + nb, G::NT, G::LDS, st>>>(A);
+        k_sor2<false, true><<<G::blocks(P->ns), G::NT, G::LDS, st>>>(A);
     }
 }
 
@@ -2709,9 +2711,17 @@ static void sor_splits(p4g_solver_s* s) {
 
 // the working arrays of level l's pipelined SOR sweeps (1D levels, and grids
 // without interior points, have none)
+template <bool NINE>
+static int sor2_lds() {
+    HIP_TRY(hipFuncSetAttribute((const void*)&k_sor2<NINE, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)Sor2<NINE>::LDS));
+    HIP_TRY(hipFuncSetAttribute((const void*)&k_sor2<NINE, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)Sor2<NINE>::LDS));
+    return 0;
+}
 static int sor_pipe_alloc(p4g_solver_s* s, int l, SorKind kind) {
     LevelInfo& L = s->lv[l];
-    if (L.dim < 2 || L.var || L.mx >= 1 << 20) return 0;      // (a strip's rows are addressed in 32 bits)
+    if (L.dim < 2 || L.var || L.mx > (1 << 20) - 256) return 0;      // (a strip is addressed in 32 bits)
     const bool nine = kind == SOR_9PT;
     if (!nine && (L.mx < 3 || L.my < 3 || (L.dim == 3 && L.mz < 3))) return 0;
     SorPipe& P = s->ms_pipes[l];
@@ -2726,6 +2736,7 @@ static int sor_pipe_alloc(p4g_solver_s* s, int l, SorKind kind) {
         ny = (size_t)P.ns * P.ng * (L.mx - 2) * Sor7::K * 2;
         nz = (size_t)P.ns * P.ng * (P.Tp + Sor7::K - 1) * 128;
     } else {
+        P4G_TRY(nine ? sor2_lds<true>() : sor2_lds<false>());
         P.Tp = nine ? Sor2<true>::steps(L.mx) : Sor2<false>::steps(L.mx);
         P.ns = nine ? Sor2<true>::strips(L.my) : Sor2<false>::strips(L.my);
         nS = (size_t)P.ns * (P.Tp / 2) * 64;

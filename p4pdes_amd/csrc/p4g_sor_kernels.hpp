@@ -17,8 +17,8 @@
 //    for bit.
 //  * S is stored by step (all 64 lanes of a step side by side), and the
 //    backward sweep visits the steps in reverse, so its accesses are full
-//    lines with addresses known at compile time; operands are loaded
-//    kSorAhead batches of steps early.
+//    lines with addresses known at compile time; operands are loaded batches
+//    of steps early.
 //  * A strip (plane group) hands its last row (plane) to the next one
 //    through global memory as pairs of 8-byte words, each half of the value
 //    with the sweep's 32-bit tag: a word is either the awaited one or not,
@@ -107,7 +107,7 @@ __device__ __forceinline__ unsigned sor_tag(const SorCtl& c, bool backward) {
 // one more failed poll: true when the waiting has to end
 __device__ __forceinline__ bool sor_give_up(const SorCtl& c, long& spins) {
     if (++spins > c.spin_limit) {
-        if (threadIdx.x == 0) atomicExch(c.ctl, 1u);
+        if ((threadIdx.x & 63) == 0) atomicExch(c.ctl, 1u);
         return true;
     }
     __builtin_amdgcn_s_sleep(1);
@@ -126,26 +126,55 @@ __device__ __forceinline__ bool sor_give_up(const SorCtl& c, long& spins) {
 // t - 1 - 2 r - sh (9-point) of its row in sweep order; tf = t forward and
 // Tp - 1 - t backward indexes S and the packed coefficients, and sh makes
 // the two agree.
+//
+// A strip is one workgroup on a compute unit of its own, and its waves have
+// one task each, so that the chain's wave (a lone wave issues an instruction
+// in four cycles, and a step's chain is 14 ns) does nothing but the steps:
+//   wave 0  the chain: operands from LDS, results to LDS, S to memory;
+//   wave 1  the previous strip's row: polls 64 columns at once;
+//   wave 2  the strip's own last row to the next strip;
+//   wave 3 (and 4)  step-ordered operands, NR batches ahead;
+//   the last wave  rows read along x and turned into steps (forward, b), or
+//           steps turned into rows and written (backward, x).
+// They meet in LDS words that count batches: a batch of SB steps is computed
+// when every word exceeds its index.  Measured, forward + backward: 1025^2
+// 5-point 336 -> 189 us, 513^2 9-point 342 -> 221 us against one wave a strip
+// that did all of it (a step 37-47 -> 25 ns in 5-point, 75 -> 55 in 9-point,
+// which moves 3 KB a step through one compute unit).  What is left: about
+// 2.7 us from strip to strip (0.3 to be seen and sent, 0.6 through L2, a
+// batch at either end) and 3 us to start.
 constexpr int kXcds = 8;
 
 template <bool NINE>
 struct Sor2 {
     static constexpr int SB = NINE ? 8 : 16;          // steps per batch
-    static constexpr int AH = 2;                      // batches of steps whose operands are in flight
-    static constexpr int YD = 2;                      // batches whose neighbour-row words are in flight
     static constexpr int P0 = NINE ? 127 : 63;        // steps from a column at lane 0 to lane 63
     static constexpr int PAD = 192;                   // slots before column 0
-    // slots of a strip's handed-over row: every batch's, in range or not
+    static constexpr int ND = NINE ? 2 : 1;           // operand waves
+    static constexpr int NT = 64 * (4 + ND);
+    static constexpr int NR = NINE ? 5 : 8, NO = 4;   // batches of operands and of results in LDS
+    static constexpr int VS = 1024 + (NINE ? 128 : 64);         // bytes of a pair of steps (turned without bank conflicts)
+    static constexpr int AB = NINE ? SB * 2048 : 0;             // a batch's couplings,
+    static constexpr int IB = NINE ? SB / 2 * 1024 : 0;         //   reciprocal diagonals
+    static constexpr int OB = SB / 2 * VS;                      //   and values (or results)
+    static constexpr int OPB = AB + IB + OB;
+    static constexpr int YN = 256;                              // neighbour-row steps in LDS
+    static constexpr int LO = NR * OPB, LY = LO + NO * OB, LW = LY + YN * 8, LD = LW + 64;
+    static constexpr size_t LDS = LD + 256;
+    // slots of a strip's handed-over row: every window's, in range or not
     __host__ __device__ static long slots(int Tp) { return Tp + PAD + 64; }
-    // steps of a strip, padded to whole rounds of the operand ring
+    // steps of a strip, padded to whole batches and tiles of k_sor9_pack
     __host__ __device__ static int steps(int mx) {
         const int need = NINE ? mx + 128 : mx - 2 + 63;
-        static_assert(32 % (SB * AH) == 0 && AH % YD == 0, "whole rounds of the operand rings, whole tiles of k_sor9_pack");
         return (need + 31) / 32 * 32;
     }
     __host__ __device__ static int cols(int mx) { return NINE ? mx : mx - 2; }
     __host__ __device__ static int rows(int my) { return NINE ? my : my - 2; }
     __host__ __device__ static int strips(int my) { return (rows(my) + 63) / 64; }
+    // strip o's block: runs of 32 strips on one XCD, whose L2 hands rows over
+    // soonest (264-271 ns one way against 330-494), in dispatch order
+    __host__ __device__ static int block_of(int o) { return o * kXcds + (o >> 5) % kXcds; }
+    __host__ __device__ static int blocks(int ns) { return block_of(ns - 1) + 1; }
 };
 
 struct Sor2Args {
@@ -160,17 +189,26 @@ struct Sor2Args {
     SorCtl c;
 };
 
+typedef volatile __attribute__((address_space(3))) int* lds_words;
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+
 template <bool NINE, bool BWD>
-__global__ void __launch_bounds__(64) k_sor2(Sor2Args A) {
+__global__ void __launch_bounds__(Sor2<NINE>::NT) k_sor2(Sor2Args A) {
     typedef Sor2<NINE> G;
-    constexpr int SB = G::SB, AH = G::AH, YD = G::YD;
-    const int r = threadIdx.x, mx = A.mx, my = A.my, ns = A.ns;
-    if ((int)blockIdx.x < ns * kXcds && blockIdx.x % kXcds) return;      // every strip on one XCD
-    const int o = (int)blockIdx.x < ns * kXcds ? blockIdx.x / kXcds : blockIdx.x - ns * (kXcds - 1);
-    if (!NINE && !BWD && o >= ns) {          // the boundary rows
+    constexpr int SB = G::SB, H = SB / 2, R = 64 / SB, lag = NINE ? 2 : 1;
+    constexpr int kNever = 0x7fffffff;
+    extern __shared__ __attribute__((aligned(16))) char sor_lds[];
+    // the chain is the fourth wave: the one that shares its SIMD with no other
+    // (waves go to the four SIMDs in turn; as the first of five the 5-point
+    // chain took 31 ns a step, alone 24)
+    const int r = threadIdx.x & 63, place = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave = place == 3 ? 0 : (place == 0 ? 3 : place);
+    const int mx = A.mx, my = A.my, ns = A.ns;
+    const int o = (int)blockIdx.x >> 3;
+    if (!NINE && !BWD && (int)blockIdx.x >= G::blocks(ns)) {          // the boundary rows
         const double idb = 1.0 / A.db;
-        const int per = 2 * mx + 2 * (my - 2);
-        for (int p = (o - ns) * 64 + r; p < per; p += (gridDim.x - ns * kXcds) * 64) {
+        const int per = 2 * mx + 2 * (my - 2), b0 = G::blocks(ns);
+        for (int p = ((int)blockIdx.x - b0) * G::NT + threadIdx.x; p < per; p += (gridDim.x - b0) * G::NT) {
             long q;
             if (p < mx) q = p;
             else if (p < 2 * mx) q = (long)(my - 1) * mx + (p - mx);
@@ -179,195 +217,358 @@ __global__ void __launch_bounds__(64) k_sor2(Sor2Args A) {
         }
         return;
     }
-    const int Tp = A.Tp, ncol = G::cols(mx), nrow = G::rows(my);
-    const int s = BWD ? ns - 1 - o : o, rho = BWD ? 63 - r : r;
-    const int row = 64 * s + rho;
-    const bool rl = row < nrow;
+    if (o >= ns || (int)blockIdx.x != G::block_of(o)) return;
+    const int Tp = A.Tp, NB = Tp / SB, ncol = G::cols(mx), nrow = G::rows(my);
+    const int s = BWD ? ns - 1 - o : o;
     const int sh = BWD ? (NINE ? Tp - 2 - (mx + 126) : Tp - (ncol + 63)) : 0;
-    const int off = sh + (NINE ? 1 + 2 * r : r);                 // c = t - off
-    // b and x: the rows of the strip, relative to the first.  Off the strip a
-    // load gives zero and a store is dropped, so no address is clamped; what
-    // a lane reads past its row's ends is masked by `live`.
+    // b and x: the rows of the strip, relative to the first; off the strip a
+    // load gives zero and a store is dropped
     const long strip0 = ((long)64 * s + (NINE ? 0 : 1)) * mx;
     const unsigned nrows = min(64, nrow - 64 * s);
     const __amdgpu_buffer_rsrc_t br = buffer_of((BWD ? (const double*)A.x : A.b) + strip0, nrows * mx * 8u);
-    const unsigned rowq = (unsigned)rho * mx + (NINE ? 0 : 1);
-    const unsigned vb = BWD ? (rowq + ncol - SB + off) * 8u : (rowq - off) * 8u;   // at t0: - or + 8 t0
     const __amdgpu_buffer_rsrc_t Sr = buffer_of(A.S + (long)s * (Tp / 2) * 64, Tp * 512u);
-    const __amdgpu_buffer_rsrc_t Ir = buffer_of(NINE ? A.inv + (long)s * (Tp / 2) * 64 : A.S, Tp * 512u);
-    const __amdgpu_buffer_rsrc_t Kr = buffer_of(NINE ? A.pk + (long)s * Tp * 256 : A.S, Tp * 4096u);
-    const unsigned v16 = rho * 16u, vk = v16 + (BWD ? 2048u : 0u);
-    const double invd = NINE ? 0.0 : 1.0 / A.d;
-    // handed-over rows, by slot (the column in sweep order); lanes past the
-    // batch repeat its slots, so that nothing has to be masked inside
-    char* const yout = (char*)(A.yh + ((long)o * G::slots(Tp) + G::PAD - G::P0 - sh) * 2);
-    const char* const yin = (const char*)(A.yh + ((long)(o > 0 ? o - 1 : 0) * G::slots(Tp) + G::PAD - sh) * 2);
-    const int l = r & (SB - 1);
-    const unsigned l16 = l * 16u;
+    const unsigned v16 = (BWD ? 63 - r : r) * 16u;
     const unsigned tag = sor_tag(A.c, BWD), want = tag + A.c.extra;
     bool dead = __builtin_amdgcn_readfirstlane((int)sor_dead(A.c)) != 0;
-    const bool full = 64 * s + 64 <= nrow;
-    __shared__ double ybuf[64];             // the neighbour row of the next batch's steps (0..SB - 1)
-    __shared__ double obuf[2][SB][64];      // the batch's results and those of the batch before
-
-    struct Ops {
-        double v[SB];                       // b (forward) or S (backward)
-        T2<double> a[NINE ? 2 * SB : 1];    // the earlier (later) four couplings
-        double inv[NINE ? SB : 1];
-    } ops[AH];
-    Tagged yw[YD];                          // lane e < SB: the neighbour row at step e of the next batches
-
-    auto yload = [&](int t0, Tagged& w) {
-        const char* const p = yin + (long)t0 * 16;
-        w.lo = ld_word((const u64*)(p + l16));
-        w.hi = ld_word((const u64*)(p + l16 + 8));
-    };
-    // every path issues the same loads, so that the compiler can count them
-    auto load = [&](int t0, Ops& P) {
-        unsigned vo = vb + t0 * 8u;
-        asm volatile("" : "+v"(vo));        // one address per batch, the steps by immediate offsets
-        // two addresses where a pair of steps may straddle the strip's bytes
-        // (one access of both would then be out of range as a whole)
-        unsigned vo1 = vo;
-        if (NINE) asm volatile("" : "+v"(vo1));
-#pragma unroll
-        for (int e = 0; e < SB; e += 2) {
-            const int m = BWD ? (Tp - 2 - (t0 + e)) >> 1 : (t0 + e) >> 1;    // pair of steps
-            if (BWD) {
-                const T2<double> v = buffer_ld2(Sr, v16, m * 1024u);
-                P.v[e] = v.b;
-                P.v[e + 1] = v.a;
-            } else {
-                P.v[e] = buffer_ld(br, vo + e * 8u);
-                P.v[e + 1] = buffer_ld(br, vo1 + e * 8u + 8u);
+    // the words: batches ready of each operand wave (the next of its own), of
+    // the values and of the neighbour row, and the first batch without room
+    // for its results
+    enum { W_OP = 0, W_VAL = G::ND, W_Y, W_OUT, W_X };
+    lds_words const words = (lds_words)(sor_lds + G::LW);
+    lds_words const done = (lds_words)(sor_lds + G::LD);     // [lane]: batches computed
+    if (threadIdx.x < 8) {
+        int w = kNever;
+        if ((int)threadIdx.x < G::ND) w = NINE || BWD ? (int)threadIdx.x : kNever;
+        else if (threadIdx.x == W_VAL) w = BWD ? kNever : 0;
+        else if (threadIdx.x == W_Y) w = 0;
+        else if (threadIdx.x == W_OUT) w = o + 1 < ns ? G::NO : kNever;
+        else if (threadIdx.x == W_X) w = BWD ? G::NO : kNever;
+        words[threadIdx.x] = w;
+    }
+    if (threadIdx.x < 64) done[threadIdx.x] = 0;
+    __syncthreads();
+    // waits inside the workgroup end with it: of the waves only wave 1 waits
+    // for another workgroup, and that is bounded (so are these)
+    auto inner_wait = [&](auto ready) __attribute__((always_inline)) {
+        long spins = 0;
+        while (!dead && !ready()) {
+            if (++spins > (1L << 24)) {
+                if (r == 0) atomicExch(A.c.ctl, 1u);
+                dead = true;
+                __builtin_amdgcn_s_waitcnt(0);      // so that the other path's waits stay as they are
             }
-            if (NINE) {
-                const T2<double> i2 = buffer_ld2(Ir, v16, m * 1024u);
-                P.inv[e] = BWD ? i2.b : i2.a;
-                P.inv[e + 1] = BWD ? i2.a : i2.b;
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const unsigned tf = BWD ? Tp - 1 - (t0 + e + h) : t0 + e + h;
-                    P.a[2 * (e + h)] = buffer_ld2(Kr, vk, tf * 4096u);
-                    P.a[2 * (e + h) + 1] = buffer_ld2(Kr, vk + 1024u, tf * 4096u);
-                }
-            }
+            if (wave) __builtin_amdgcn_s_sleep(1);
         }
-    };
-    double h1 = 0.0, u1 = 0.0, u2 = 0.0;    // own last result; the neighbour row's last two
-    double y[SB], keep = 0.0;
-    // steps E .. E + SB / 2 - 1 of a batch; edge: some lane is off the grid
-    auto half = [&](int t0, const Ops& P, bool edge, int E) {
-        unsigned vo = vb - t0 * 8u;
-        asm volatile("" : "+v"(vo));
-#pragma unroll
-        for (int e = E; e < E + SB / 2; ++e) {
-            const int c = t0 + e - off;
-            const bool live = !edge || (rl && (unsigned)c < (unsigned)ncol);
-            const double u3 = u2;
-            u2 = u1;
-            u1 = wave_shr1(h1, y[e]);
-            double sum = live || NINE ? P.v[e] : 0.0, res;
-            if (!NINE) {
-                if (!BWD) {
-                    sum += A.sy * u1;
-                    sum += A.sx * h1;
-                } else {
-                    sum += A.sx * h1;
-                    sum += A.sy * u1;
-                }
-                res = sum * invd;
-            } else {             // off the grid every coefficient is zero, and so is the result
-                const T2<double> p0 = P.a[2 * e], p1 = P.a[2 * e + 1];
-                if (!BWD) {      // (j-1, i-1), (j-1, i), (j-1, i+1), (j, i-1)
-                    sum -= p0.a * u3;
-                    sum -= p0.b * u2;
-                    sum -= p1.a * u1;
-                    sum -= p1.b * h1;
-                } else {         // (j, i+1), (j+1, i-1), (j+1, i), (j+1, i+1)
-                    sum -= p0.a * h1;
-                    sum -= p0.b * u1;
-                    sum -= p1.a * u2;
-                    sum -= p1.b * u3;
-                }
-                res = sum * P.inv[e];
-            }
-            if (!BWD) {
-                if (e & 1) buffer_st2(Sr, v16, (t0 + e - 1) * 512u, keep, sum);
-                else keep = sum;
-            } else {
-                buffer_st(br, (live ? vo : 0x80000000u) + (SB - 1 - e) * 8u, res);
-            }
-            h1 = res;
-            obuf[(t0 / SB) & 1][e][r] = res;
-        }
-    };
-    // the neighbour row of the batch at t0, loaded in yw[q], into LDS
-    auto ywait = [&](int t0, int q, bool edge) __attribute__((always_inline)) {
-        if (o == 0) return;
-        const int slot = t0 + l - sh;
-        const bool need = !edge || (slot >= 0 && slot < ncol);
-        if (__builtin_expect(!__all(!need || yw[q].is(want)), 0)) {
-            long spins = 0;
-            while (!dead && !__all(!need || yw[q].is(want))) {
-                dead = sor_give_up(A.c, spins);
-                yload(t0, yw[q]);
-            }
-            // the words of the batches after were loaded too early as well
-#pragma unroll
-            for (int h = 1; h < YD; ++h) yload(t0 + h * SB, yw[(q + h) % YD]);
-            __builtin_amdgcn_s_waitcnt(0);   // so that the other path's waits stay as they are
-        }
-        ybuf[r] = need ? yw[q].value() : 0.0;
         wave_lds_order();
     };
-    // the last lane's results of the batch at t0, at the slots their columns give
-    auto publish = [&](int t0, double v, bool edge) __attribute__((always_inline)) {
-        const int slot = t0 + l - G::P0 - sh;
-        char* const p = yout + (long)t0 * 16;
-        if (!edge || (slot >= 0 && slot < ncol)) st_tagged((u64*)(p + l16), (u64*)(p + l16 + 8), v, tag);
-    };
-    ybuf[r] = 0.0;
-    wave_lds_order();
+
+    if (wave == 0) {                        // ------------------------------- the chain
+        __builtin_amdgcn_s_setprio(3);
+        const double invd = NINE ? 0.0 : 1.0 / A.d;
+        struct Ops {
+            f64x2 v[H / 2], y[H / 2];       // b (forward) or S (backward), the neighbour row
+            f64x2 a[NINE ? 2 * H : 1];      // the earlier (later) four couplings
+            f64x2 inv[NINE ? H / 2 : 1];
+        } P0, P1;
+        const char* const mine = sor_lds + r * 16;
+        auto read = [&](int slot, int k, int part, Ops& P) __attribute__((always_inline)) {
+            const char* const p = mine + slot * G::OPB;
+            const f64x2* const yp = (const f64x2*)(sor_lds + G::LY) + ((k * SB + part * H) & (G::YN - 1)) / 2;
 #pragma unroll
-    for (int h = 0; h < YD; ++h) yload(h * SB, yw[h]);
-    ywait(0, 0, true);
+            for (int e = 0; e < H / 2; ++e) {
+                const int f = part * (H / 2) + e;
+                P.y[e] = yp[e];
+                P.v[e] = *(const f64x2*)(p + G::AB + G::IB + f * G::VS);
+                if (NINE) {
+                    P.inv[e] = *(const f64x2*)(p + G::AB + f * 1024);
 #pragma unroll
-    for (int e = 0; e < SB; ++e) y[e] = ybuf[e];
-    wave_lds_order();
-    yload(YD * SB, yw[0]);
+                    for (int h = 0; h < 4; ++h) P.a[4 * e + h] = *(const f64x2*)(p + f * 4096 + h * 1024);
+                }
+            }
+        };
+        double h1 = 0.0, u1 = 0.0, u2 = 0.0;    // own last result; the neighbour row's last two
+        auto steps = [&](int k, int oslot, int part, const Ops& P) __attribute__((always_inline)) {
+            char* const op = sor_lds + G::LO + oslot * G::OB + r * 16;
+            f64x2 keep, kres;
 #pragma unroll
-    for (int q = 0; q < AH; ++q) load(q * SB, ops[q]);
-    // a round of the operand ring; off the grid or not is settled per round,
-    // because a taken branch costs a lone wave as much as a step
-    auto round = [&](int t0, bool edge) __attribute__((always_inline)) {
-#pragma unroll
-        for (int q = 0; q < AH; ++q) {
-            const int t = t0 + q * SB;
-            // the words awaited below and the results published below were
-            // asked for half a batch before
-            const double v = obuf[((t / SB) & 1) ^ 1][l][63];
-            half(t, ops[q], edge, 0);
-            publish(t - SB, v, edge);
-            ywait(t + SB, (q + 1) % YD, edge);
-            double yn[SB];
-#pragma unroll
-            for (int e = 0; e < SB; ++e) yn[e] = ybuf[e];
-            half(t, ops[q], edge, SB / 2);
+            for (int e = 0; e < H; ++e) {
+                // backward, a pair's later step is stored first
+                const int g = BWD ? (e ^ 1) : e;
+                const double u3 = u2;
+                u2 = u1;
+                u1 = wave_shr1(h1, P.y[e / 2][e & 1]);
+                double sum = P.v[e / 2][(BWD ? g : e) & 1], res;
+                if (!NINE) {
+                    if (!BWD) {
+                        sum += A.sy * u1;
+                        sum += A.sx * h1;
+                    } else {
+                        sum += A.sx * h1;
+                        sum += A.sy * u1;
+                    }
+                    res = sum * invd;
+                } else {             // off the grid every coefficient is zero, and so is the result
+                    const f64x2 p0 = P.a[2 * e], p1 = P.a[2 * e + 1];
+                    if (!BWD) {      // (j-1, i-1), (j-1, i), (j-1, i+1), (j, i-1)
+                        sum -= p0[0] * u3;
+                        sum -= p0[1] * u2;
+                        sum -= p1[0] * u1;
+                        sum -= p1[1] * h1;
+                    } else {         // (j, i+1), (j+1, i-1), (j+1, i), (j+1, i+1)
+                        sum -= p0[0] * h1;
+                        sum -= p0[1] * u1;
+                        sum -= p1[0] * u2;
+                        sum -= p1[1] * u3;
+                    }
+                    res = sum * P.inv[e / 2][g & 1];
+                }
+                keep[e & 1] = sum;
+                kres[e & 1] = res;
+                h1 = res;
+                if (e & 1) {
+                    if (!BWD) buffer_st2(Sr, v16 + (e / 2) * 1024u, (k * SB + part * H) * 512u, keep[0], keep[1]);
+                    *(f64x2*)(op + (part * H + e) / 2 * G::VS) = kres;
+                }
+            }
+        };
+        lds_words const my_word = words + (r & 7);
+        inner_wait([&] { return __all(*my_word > 0); });
+        read(0, 0, 0, P0);
+        int slot = 0;
+        for (int k = 0; k < NB; ++k) {
+            const int w = *my_word;
             wave_lds_order();
+            read(slot, k, 1, P1);
+            steps(k, k & (G::NO - 1), 0, P0);
+            slot = slot + 1 == G::NR ? 0 : slot + 1;
+            if (__all(w > k + 1)) {
+                read(slot, k + 1, 0, P0);
+                steps(k, k & (G::NO - 1), 1, P1);
+                wave_lds_order();
+                done[r] = k + 1;
+            } else {                 // what there is goes on to the next strip first
+                steps(k, k & (G::NO - 1), 1, P1);
+                wave_lds_order();
+                done[r] = k + 1;
+                inner_wait([&] { return __all(*my_word > k + 1); });
+                read(slot, k + 1, 0, P0);
+            }
+        }
+        return;
+    }
+    if (wave == 1) {                        // ------------------------------- the neighbour row
+        double* const yl = (double*)(sor_lds + G::LY);
+        if (o == 0) {
+            for (int q = r; q < G::YN; q += 64) yl[q] = 0.0;
+        } else {
+            const char* const yin = (const char*)(A.yh + ((long)(o - 1) * G::slots(Tp) + G::PAD - sh + r) * 2);
+            long spins = 0;
+            for (int t = 0; t < Tp;) {
+                inner_wait([&] { return __builtin_amdgcn_readfirstlane(done[0]) * SB + G::YN >= t + 64; });
+                if (dead) break;
+                const int slot = t + r - sh;
+                const bool need = slot >= 0 && slot < ncol;
+                const char* const p = yin + (long)t * 16;
+                Tagged w;
+                w.lo = ld_word((const u64*)p);
+                w.hi = ld_word((const u64*)(p + 8));
+                const unsigned long long bad = __ballot(need && !w.is(want));
+                const int n = bad ? (int)__builtin_ctzll(bad) / SB * SB : 64;
+                if (n > 0) {
+                    if (r < n) yl[(t + r) & (G::YN - 1)] = need ? w.value() : 0.0;
+                    t += n;
+                    wave_lds_order();
+                    words[W_Y] = t / SB;
+                    spins = 0;
+                } else if (sor_give_up(A.c, spins)) {
+                    break;
+                }
+            }
+        }
+        wave_lds_order();
+        words[W_Y] = kNever;
+        return;
+    }
+
+    // tasks of the waves 2.., in batches: a lane of those that turn rows into
+    // steps (or back) has step te of a batch and rows r0, r0 + R, ..
+    const int te = r & (SB - 1), r0 = r / SB;
+    const int c0 = te - sh - (NINE ? 1 : 0) - lag * r0;          // its column at batch 0, row r0
+    const int rho0 = BWD ? 63 - r0 : r0, x0 = NINE ? 0 : 1;
+    const unsigned va = (unsigned)(rho0 * mx + x0 + (BWD ? ncol - 1 - c0 : c0)) * 8u;
+    const int dva = (BWD ? -1 : 1) * R * (mx - lag) * 8;         // from row to row
+    // batches t of the whole strip's rows and no column off the grid
+    const bool full = nrows == 64;
+    auto inside = [&](int t) { return full && t >= sh + G::P0 && t + SB - sh <= ncol; };
+    const unsigned turned = (te >> 1) * G::VS + r0 * 16u + (te & 1) * 8u;
+    // b by rows into steps; GD batches of loads in flight, in whole rounds (a
+    // batch past the last one reads nothing and is not computed), so that the
+    // compiler can count them
+    constexpr int GD = 4;
+    auto turn = [&](int word) __attribute__((always_inline)) {
+        double g[GD][SB];
+        auto ask = [&](int k, double (&v)[SB]) __attribute__((always_inline)) {
 #pragma unroll
-            for (int e = 0; e < SB; ++e) y[e] = yn[e];
-            yload(t + (YD + 1) * SB, yw[(q + 1) % YD]);
-            load(min(t + SB * AH, Tp - SB), ops[q]);
+            for (int q = 0; q < SB; ++q) {
+                const bool live = (unsigned)(k * SB + c0 - q * R * lag) < (unsigned)ncol;
+                v[q] = buffer_ld(br, live ? va + k * SB * 8u + q * dva : 0x80000000u);
+            }
+        };
+#pragma unroll
+        for (int h = 0; h < GD; ++h) {
+            ask(h, g[h]);
+            __builtin_amdgcn_sched_barrier(0);      // in this order, as the loop does
+        }
+        for (int k = 0; k < NB; k += GD) {
+#pragma unroll
+            for (int h = 0; h < GD; ++h) {
+                inner_wait([&] { return __builtin_amdgcn_readfirstlane(done[0]) + G::NR > k + h; });
+                char* const p = sor_lds + (k + h) % G::NR * G::OPB + G::AB + G::IB + turned;
+#pragma unroll
+                for (int q = 0; q < SB; ++q) *(double*)(p + q * R * 16) = g[h][q];
+                wave_lds_order();
+                words[word] = k + h + 1;
+                ask(k + h + GD, g[h]);
+            }
+        }
+        words[word] = kNever;
+    };
+    // batches of results as the chain leaves them in LDS
+    auto results = [&](int word, auto take) __attribute__((always_inline)) {
+        for (int k = 0; k < NB; ++k) {
+            inner_wait([&] { return __builtin_amdgcn_readfirstlane(done[0]) > k; });
+            take(sor_lds + G::LO + (k & (G::NO - 1)) * G::OB, k * SB);
+            wave_lds_order();
+            words[word] = k + 1 + G::NO;
         }
     };
-    round(0, true);      // apart from the loop, whose waits it would shorten (fewer accesses precede it)
-    for (int t0 = SB * AH; t0 < Tp; t0 += SB * AH) {
-        if (!full || t0 < 63 * (NINE ? 2 : 1) + sh + 1 || t0 + SB * AH + SB - sh > ncol) round(t0, true);
-        else round(t0, false);
+    if (wave == 2) {                        // ------------------------------- the last row, to the next strip
+        char* const yout = (char*)(A.yh + ((long)o * G::slots(Tp) + G::PAD - G::P0 - sh + te) * 2);
+        if (o + 1 < ns) {
+            results(W_OUT, [&](const char* ob, int t) __attribute__((always_inline)) {
+                const int slot = t + te - G::P0 - sh;
+                const double v = *(const double*)(ob + (te >> 1) * G::VS + 63 * 16 + (te & 1) * 8);
+                char* const p = yout + (long)t * 16;
+                if (r < SB && slot >= 0 && slot < ncol) st_tagged((u64*)p, (u64*)(p + 8), v, tag);
+            });
+        }
+        return;
     }
-    publish(Tp - SB, obuf[((Tp / SB) & 1) ^ 1][l][63], true);
-    if (BWD && o == ns - 1 && r == 0) A.c.ctl[1] += 1;
+    if (wave == 3 + G::ND) {                // ------------------------------- rows
+        if (!BWD) {
+            turn(W_VAL);
+        } else {
+            results(W_X, [&](const char* ob, int t) __attribute__((always_inline)) {
+                double xv[SB];
+#pragma unroll
+                for (int q = 0; q < SB; ++q) xv[q] = *(const double*)(ob + turned + q * R * 16);
+                if (inside(t)) {
+#pragma unroll
+                    for (int q = 0; q < SB; ++q) buffer_st(br, va - t * 8u + q * dva, xv[q]);
+                } else {
+#pragma unroll
+                    for (int q = 0; q < SB; ++q) {
+                        const int c = t + c0 - q * R * lag;
+                        const bool live = (unsigned)c < (unsigned)ncol && (unsigned)(rho0 - q * R) < nrows;
+                        buffer_st(br, live ? va - t * 8u + q * dva : 0x80000000u, xv[q]);
+                    }
+                }
+            });
+            if (o == ns - 1 && r == 0) A.c.ctl[1] += 1;
+        }
+        return;
+    }
+    if constexpr (!NINE) {                  // ------------------------------- 5-point sums
+        if (BWD) {                          // S; off the grid it is left as the forward sweep's chain ran on
+            f64x2 g[GD][H];
+            const bool rl = 64 * s + 63 - r < nrow;
+            auto ask = [&](int k, f64x2 (&v)[H]) __attribute__((always_inline)) {
+#pragma unroll
+                for (int e = 0; e < H; ++e) {
+                    const T2<double> t = buffer_ld2(Sr, v16, (unsigned)((Tp - 2 - (k * SB + 2 * e)) >> 1) * 1024u);
+                    v[e] = f64x2{t.a, t.b};
+                }
+            };
+#pragma unroll
+            for (int h = 0; h < GD; ++h) {
+                ask(min(h, NB - 1), g[h]);
+                __builtin_amdgcn_sched_barrier(0);      // in this order, as the loop does
+            }
+            for (int k = 0; k < NB; k += GD) {
+#pragma unroll
+                for (int h = 0; h < GD; ++h) {
+                    inner_wait([&] { return __builtin_amdgcn_readfirstlane(done[0]) + G::NR > k + h; });
+                    char* const p = sor_lds + (k + h) % G::NR * G::OPB + r * 16;
+                    const int c = (k + h) * SB - sh - r;
+                    if (!inside((k + h) * SB)) {
+#pragma unroll
+                        for (int e = 0; e < H; ++e) {     // (a pair's later step comes first)
+                            if (!rl || (unsigned)(c + 2 * e) >= (unsigned)ncol) g[h][e][1] = 0.0;
+                            if (!rl || (unsigned)(c + 2 * e + 1) >= (unsigned)ncol) g[h][e][0] = 0.0;
+                        }
+                    }
+#pragma unroll
+                    for (int e = 0; e < H; ++e) *(f64x2*)(p + e * G::VS) = g[h][e];
+                    wave_lds_order();
+                    words[W_OP] = k + h + 1;
+                    ask(min(k + h + GD, NB - 1), g[h]);
+                }
+            }
+            words[W_OP] = kNever;
+        }
+    } else {                                // ------------------------------- 9-point operands
+        const int i = wave - 3;
+        const __amdgpu_buffer_rsrc_t Ir = buffer_of(A.inv + (long)s * (Tp / 2) * 64, Tp * 512u);
+        const __amdgpu_buffer_rsrc_t Kr = buffer_of(A.pk + (long)s * Tp * 256, Tp * 4096u);
+        const unsigned vk = v16 + (BWD ? 2048u : 0u);
+        constexpr int NL = 2 * SB + H * (BWD ? 2 : 1), GW = 2;   // loads of a batch, batches in flight
+        f64x2 g[GW][NL];
+        auto ld = [&](__amdgpu_buffer_rsrc_t b, unsigned vo, unsigned so) __attribute__((always_inline)) {
+            const T2<double> t = buffer_ld2(b, vo, so);
+            return f64x2{t.a, t.b};
+        };
+        auto ask = [&](int k, f64x2 (&v)[NL]) __attribute__((always_inline)) {
+            const int t = min(k, NB - 1) * SB;
+#pragma unroll
+            for (int e = 0; e < H; ++e) {
+                const int m = BWD ? (Tp - 2 - (t + 2 * e)) >> 1 : (t + 2 * e) >> 1;    // pair of steps
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const unsigned tf = BWD ? Tp - 1 - (t + 2 * e + h) : t + 2 * e + h;
+                    v[2 * (2 * e + h)] = ld(Kr, vk, tf * 4096u);
+                    v[2 * (2 * e + h) + 1] = ld(Kr, vk + 1024u, tf * 4096u);
+                }
+                v[2 * SB + e] = ld(Ir, v16, m * 1024u);
+                if (BWD) v[2 * SB + H + e] = ld(Sr, v16, m * 1024u);
+            }
+        };
+#pragma unroll
+        for (int h = 0; h < GW; ++h) {
+            ask(i + h * G::ND, g[h]);
+            __builtin_amdgcn_sched_barrier(0);      // in this order, as the loop does
+        }
+        int sl = i;
+        for (int k = i; k < NB; k += GW * G::ND) {
+#pragma unroll
+            for (int h = 0; h < GW; ++h) {
+                const int kk = k + h * G::ND;
+                inner_wait([&] { return __builtin_amdgcn_readfirstlane(done[0]) + G::NR > kk; });
+                char* const p = sor_lds + sl * G::OPB + r * 16;
+                sl = sl + G::ND >= G::NR ? sl + G::ND - G::NR : sl + G::ND;
+#pragma unroll
+                for (int e = 0; e < 2 * SB; ++e) *(f64x2*)(p + e * 1024) = g[h][e];
+#pragma unroll
+                for (int e = 0; e < H; ++e) {
+                    *(f64x2*)(p + G::AB + e * 1024) = g[h][2 * SB + e];
+                    if (BWD) *(f64x2*)(p + G::AB + G::IB + e * G::VS) = g[h][2 * SB + H + e];
+                }
+                wave_lds_order();
+                words[W_OP + i] = kk + G::ND;
+                ask(kk + GW * G::ND, g[h]);
+            }
+        }
+        words[W_OP + i] = kNever;
+    }
 }
 
 // the packed operator of a 9-point level: pk[(s Tp + tf) 4 + p][rho] the
