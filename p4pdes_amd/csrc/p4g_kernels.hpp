@@ -2992,155 +2992,261 @@ k_band_fill(int mx, int my, int n, int bw, const double* __restrict__ g, int uni
     }
 }
 
-// Band LU without pivoting, in place, by one workgroup (bw < 64).  Bound by
-// its n dependent steps, so the window of a step (rows and columns k ..
-// k + bw, at most 64 x 64) stays in registers, four entries a thread, at
-// places that its indices modulo bw + 1 give: a step publishes row and column
-// k through LDS, everyone updates, and row and column k + bw + 1 take the
-// free places.  The entering rows and columns are read kLuChunk steps ahead.
-// One barrier per step; 1089 points with bw 34: 0.26 ms, where the host took
-// 1.5 ms and two copies.  info: the first row whose pivot is zero (spd: not
-// positive), + 1, or 0.
-constexpr int kLuChunk = 8;
-__global__ void __launch_bounds__(1024)
-k_band_lu(int n, int bw, double* __restrict__ B, int spd, int* __restrict__ info) {
-    const int w = 2 * bw + 1, W = bw + 1, tid = threadIdx.x;
-    const int a = tid >> 4, b0 = tid & 15;               // place (a, b0 + 16 m)
-    __shared__ double row[2][64], col[2][64];
-    __shared__ double in[2][kLuChunk][128];              // entering row (0..63) and column (64..127), by place
-    double v[4];
-    auto entry = [&](int i, int j) {
-        return i < n && j < n && i - j <= bw && j - i <= bw ? B[(long)i * w + (j - i + bw)] : 0.0;
+// The dense inverse of a band operator (bw < 64) by blocks of nb >= bw rows,
+// between which it is block tridiagonal:
+//   D_0 = A_00,  G_I = D_I^-1,  D_I+1 = A_I+1,I+1 - A_I+1,I G_I A_I,I+1
+//   P_I = G_I Y_I,  Y_I+1 = E_I+1 - A_I+1,I P_I            (forward)
+//   X_I = P_I - G_I A_I,I+1 X_I+1                          (backward)
+// without pivoting (the pivots are a band LU's).  A row couples to a few
+// places only (BandOff), so the products with A's blocks are short sums and
+// G_I is all that is kept.  Bound by the chain of n pivots in k_blk_factor and
+// of 2 n / nb block products in k_blk_inverse.
+struct BandOff {
+    int n;
+    int d[13];                                           // distances of the later neighbours
+};
+constexpr int kBlkMax = 63;
+inline int blk_rows(int n, int bw) { return std::max(bw, std::min(n, 16)); }       // (short blocks cost more barriers)
+inline long blk_words(int n, int bw) {
+    const long nb = blk_rows(n, bw);
+    return (n + nb - 1) / nb * nb * nb;
+}
+
+// G_I of every block, by one workgroup: Gauss-Jordan in registers (a thread
+// has column j = lane of the rows wave + 4 m), a barrier a pivot, the next
+// block's coefficients on their way meanwhile; nb <= 4 MR rows.  1089 points with bw 34:
+// 0.68 ms where a band LU with a 64 x 64 window took 1.05 ms.  info: the first row
+// whose pivot is zero (spd: not positive), + 1, or 0.
+template <int MR>
+__global__ void __launch_bounds__(256)
+k_blk_factor(int n, int bw, int nb, BandOff of, const double* __restrict__ B, int spd, double* __restrict__ G,
+             int* __restrict__ info) {
+    const int w = 2 * bw + 1, tid = threadIdx.x, j = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nblk = (n + nb - 1) / nb, ncf = nb * of.n;
+    __shared__ double gs[kBlkMax][64], row[2][64];       // G, then A_I+1,I G; the pivot row
+    __shared__ double cl[kBlkMax * 13], cu[kBlkMax * 13];        // couplings of rows I+1 to I, I to I+1
+    auto entry = [&](int q, int p) {
+        if (q >= n || p >= n) return q == p ? 1.0 : 0.0;
+        return q - p <= bw && p - q <= bw ? B[(long)q * w + (p - q + bw)] : 0.0;
     };
+    double a[MR], d[MR], pl[4], pu[4];
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-        const int b = b0 + 16 * m;
-        v[m] = a < W && b < W ? entry(a, b) : 0.0;
-    }
-    // what enters after step k: row and column e = k + W; place p holds the
-    // column (row) in k + 1 .. k + W congruent to p
-    const int ls = tid >> 7, lp = tid & 127, lq = lp & 63;
-    auto enter = [&](int k) {
-        if (lq >= W) return 0.0;
-        const int e = k + W, base = k + 1, other = base + (lq - base % W + W) % W;
-        return lp < 64 ? entry(e, other) : entry(other, e);
-    };
-    in[0][ls][lp] = enter(ls);
+    for (int m = 0; m < MR; ++m) a[m] = wv + 4 * m < nb && j < nb ? entry(wv + 4 * m, j) : 0.0;
     int bad = 0;
-    __syncthreads();
-    int kw = 0;
-    for (int k0 = 0; k0 < n; k0 += kLuChunk) {
-        const int buf = (k0 / kLuChunk) & 1;
-        const double next = enter(k0 + kLuChunk + ls);
+    for (int I = 0, base = 0; I < nblk; ++I, base += nb) {
+        const bool more = I + 1 < nblk;
+#pragma unroll
+        for (int m = 0; m < MR; ++m) {
+            const int i = wv + 4 * m;
+            d[m] = more && i < nb && j < nb ? entry(base + nb + i, base + nb + j) : 0.0;
+        }
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+            const int t = tid + 256 * h, i = t / of.n, dd = t < ncf ? of.d[t % of.n] : 0;
+            const int ql = base + nb + i, qu = base + i;
+            pl[h] = more && t < ncf && ql < n ? B[(long)ql * w + (bw - dd)] : 0.0;
+            pu[h] = more && t < ncf && qu + dd < n ? B[(long)qu * w + (bw + dd)] : 0.0;
+        }
+#pragma unroll
+        for (int km = 0; km < MR; ++km) {
+            if (4 * km < nb) {
 #pragma unroll 1
-        for (int s = 0; s < kLuChunk && k0 + s < n; ++s) {
-            const int k = k0 + s, par = k & 1;
-            if (a == kw) {
+                for (int kt = 0; kt < 4; ++kt) {
+                    const int k = 4 * km + kt;
+                    if (k >= nb) break;
+                    if (wv == kt) row[k & 1][j] = a[km];
+                    __syncthreads();
+                    const double piv = row[k & 1][k], rk0 = row[k & 1][j], pi = 1.0 / piv;
+                    if (!bad && (spd ? !(piv > 0.0) : piv == 0.0)) bad = base + k + 1;
+                    const double rk = j == k ? pi : rk0 * pi;
 #pragma unroll
-                for (int m = 0; m < 4; ++m) row[par][b0 + 16 * m] = v[m];
-            }
-#pragma unroll
-            for (int m = 0; m < 4; ++m)
-                if (b0 + 16 * m == kw) col[par][a] = v[m];
-            if (s == kLuChunk - 1) in[buf ^ 1][ls][lp] = next;
-            __syncthreads();
-            const double piv = row[par][kw];
-            if (!bad && (spd ? !(piv > 0.0) : piv == 0.0)) bad = k + 1;
-            const double l = col[par][a] / piv;
-            const int i = k + (a - kw + W) % W;          // the row at place a
-#pragma unroll
-            for (int m = 0; m < 4; ++m) {
-                const int b = b0 + 16 * m, j = k + (b - kw + W) % W;
-                if (a >= W || b >= W) continue;
-                if (a == kw || b == kw) {                // final: U's row and L's column
-                    if (i < n && j < n) B[(long)i * w + (j - i + bw)] = b == kw && a != kw ? l : v[m];
-                    v[m] = a == kw ? in[buf][s][b] : in[buf][s][64 + a];
-                } else {
-                    v[m] -= l * row[par][b];
+                    for (int m = 0; m < MR; ++m) {
+                        const long long b = __double_as_longlong(a[m]);
+                        const int flo = __builtin_amdgcn_readlane((int)b, k);
+                        const int fhi = __builtin_amdgcn_readlane((int)(b >> 32), k);
+                        const double f = __longlong_as_double(((long long)fhi << 32) | (unsigned)flo);
+                        a[m] = (j == k ? 0.0 : a[m]) - f * rk;
+                    }
+                    if (wv == kt) a[km] = rk;
                 }
             }
-            kw = kw + 1 == W ? 0 : kw + 1;
+        }
+#pragma unroll
+        for (int m = 0; m < MR; ++m) {
+            const int i = wv + 4 * m;
+            if (i < nb && j < nb) {
+                G[((long)I * nb + i) * nb + j] = a[m];
+                gs[i][j] = a[m];
+            }
+        }
+#pragma unroll
+        for (int h = 0; h < 4; ++h)
+            if (tid + 256 * h < ncf) {
+                cl[tid + 256 * h] = pl[h];
+                cu[tid + 256 * h] = pu[h];
+            }
+        __syncthreads();
+        if (!more) break;
+#pragma unroll
+        for (int m = 0; m < MR; ++m) {                   // A_I+1,I G
+            const int i = wv + 4 * m;
+            double t = 0.0;
+            if (i < nb)
+                for (int q = 0; q < of.n; ++q) {
+                    const int k = nb + i - of.d[q];
+                    if (k < nb) t += cl[i * of.n + q] * gs[k][j];
+                }
+            a[m] = t;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < MR; ++m)
+            if (wv + 4 * m < nb) gs[wv + 4 * m][j] = a[m];
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < MR; ++m) {                   // D_I+1
+            const int i = wv + 4 * m;
+            double t = d[m];
+            if (i < nb && j < nb)
+                for (int q = 0; q < of.n; ++q) {
+                    const int k = nb + j - of.d[q];
+                    if (k < nb) t -= gs[i][k] * cu[k * of.n + q];
+                }
+            a[m] = t;
         }
         __syncthreads();
     }
     if (tid == 0) *info = bad;
 }
 
-// The dense inverse of a band LU factor (bw < 64): a wave takes 16 columns of
-// the identity through both substitutions, four lanes a column, each a
-// quarter of a row's sum; the last rows of the solution stay in LDS and the
-// factor's rows come through LDS a chunk ahead.  Bound by the 2 n dependent
-// rows: 1089 points with bw 34 took 9.1 ms with a thread per column and its
-// column read back from memory.
-constexpr int kInvRows = 8;
-__global__ void __launch_bounds__(64)
-k_band_inverse(int n, int bw, const double* __restrict__ B, double* __restrict__ Ainv) {
-    const int w = 2 * bw + 1, r = threadIdx.x, c = r >> 2, p = r & 3;
-    const int c0 = blockIdx.x * 16, cc = c0 + c;
-    __shared__ double win[128][16];                      // the last solution rows, by row modulo 128
-    __shared__ double Bs[2][kInvRows][136];              // factor rows, four zeros on either side
-    constexpr int PF = kInvRows * 136 / 64;
-    double pf[PF];
-    // forward rows r0 .. r0 + 7, or backward rows r0 .. r0 - 7
-    auto fetch = [&](int r0, int dir) {
+// The inverse's columns c0 .. c0 + 15 through both substitutions, a workgroup
+// each: thread (row i = tid / 16 + 16 m, column tid % 16), blocks in LDS, the
+// next one's on their way.  1089 points with bw 34: 0.24 ms where one wave
+// took 16 columns row by row in 1.88 ms.
+__global__ void __launch_bounds__(256)
+k_blk_inverse(int n, int bw, int nb, BandOff of, const double* __restrict__ B, const double* __restrict__ G,
+              double* __restrict__ Ainv) {
+    const int w = 2 * bw + 1, tid = threadIdx.x, c = tid & 15, r0 = tid >> 4;
+    const int nblk = (n + nb - 1) / nb, c0 = blockIdx.x * 16, cc = c0 + c, I0 = c0 / nb;
+    const int nn = nb * nb, ncf = nb * of.n;
+    __shared__ double gs[kBlkMax * kBlkMax], ys[kBlkMax][16], ps[kBlkMax][16], cf[kBlkMax * 13];
+    double pg[16], pc[4];
+    // block I's G and its rows' couplings to block I - dir
+    auto fetch = [&](int I, int dir) {
+        if (I < 0 || I >= nblk) return;
 #pragma unroll
-        for (int e = 0; e < PF; ++e) {
-            const int t = e * 64 + r, i = r0 + dir * (t / 136), x = t % 136 - 4;
-            pf[e] = i >= 0 && i < n && x >= 0 && x < w ? B[(long)i * w + x] : 0.0;
+        for (int h = 0; h < 16; ++h) {
+            const int t = tid + 256 * h;
+            pg[h] = t < nn ? G[(long)I * nn + t] : 0.0;
+        }
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+            const int t = tid + 256 * h, q = I * nb + t / of.n, dd = t < ncf ? of.d[t % of.n] : 0;
+            const bool ok = t < ncf && q < n && (dir > 0 ? q >= dd : q + dd < n);
+            pc[h] = ok ? B[(long)q * w + (bw - dir * dd)] : 0.0;
         }
     };
-    auto stage = [&](int buf) {
+    auto stage = [&]() {
 #pragma unroll
-        for (int e = 0; e < PF; ++e) {
-            const int t = e * 64 + r;
-            Bs[buf][t / 136][t % 136] = pf[e];
-        }
-        wave_lds_order();
+        for (int h = 0; h < 16; ++h)
+            if (tid + 256 * h < nn) gs[tid + 256 * h] = pg[h];
+#pragma unroll
+        for (int h = 0; h < 4; ++h)
+            if (tid + 256 * h < ncf) cf[tid + 256 * h] = pc[h];
     };
-    auto quad = [&](double s) {                          // the sum over the column's four lanes
-        s += __shfl_xor(s, 1, 4);
-        return s + __shfl_xor(s, 2, 4);
-    };
-    const int terms = (bw + 3) / 4;
-    for (int dir = 1; dir >= -1; dir -= 2) {
-        const int first = dir > 0 ? c0 : n - 1, count = dir > 0 ? n - c0 : n;
-        for (int e = r; e < 128 * 16; e += 64) win[e >> 4][e & 15] = 0.0;
-        fetch(first, dir);
-        stage(0);
-        double z = dir < 0 && first >= c0 && cc < n ? Ainv[(long)first * n + cc] : 0.0;
-        for (int h = 0; h < count; h += kInvRows) {
-            const int buf = (h / kInvRows) & 1;
-            fetch(first + dir * (h + kInvRows), dir);
-            for (int s = 0; s < kInvRows && h + s < count; ++s) {
-                const int i = first + dir * (h + s);
-                const double* const br = Bs[buf][s] + 4 + bw;
-                double s0 = 0.0, s1 = 0.0;
-                int m = 0;
-                for (; m + 1 < terms; m += 2) {
-                    const int t0 = dir * (p + 1 + 4 * m), t1 = dir * (p + 5 + 4 * m);
-                    s0 += br[-t0] * win[(i - t0) & 127][c];
-                    s1 += br[-t1] * win[(i - t1) & 127][c];
-                }
-                if (m < terms) {
-                    const int t0 = dir * (p + 1 + 4 * m);
-                    s0 += br[-t0] * win[(i - t0) & 127][c];
-                }
-                const double base = dir > 0 ? (i == cc ? 1.0 : 0.0) : z;
-                if (dir < 0) {                           // the row after: asked for a row ahead
-                    const int in = i - 1;
-                    z = in >= c0 && cc < n ? Ainv[(long)in * n + cc] : 0.0;
-                }
-                double v = base - quad(s0 + s1);
-                if (dir < 0) v /= br[0];
-                if (p == 0) {
-                    win[i & 127][c] = v;
-                    if (cc < n) Ainv[(long)i * n + cc] = v;
-                }
-                wave_lds_order();
+    auto product = [&](double (&v)[4]) {                 // G ys
+        v[0] = v[1] = v[2] = v[3] = 0.0;
+        const double* g[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) g[m] = gs + min(r0 + 16 * m, nb - 1) * nb;
+        if (nb <= 16) {
+#pragma unroll 8
+            for (int k = 0; k < nb; ++k) v[0] += g[0][k] * ys[k][c];
+        } else if (nb <= 48) {
+#pragma unroll 8
+            for (int k = 0; k < nb; ++k) {
+                const double y = ys[k][c];
+#pragma unroll
+                for (int m = 0; m < 3; ++m) v[m] += g[m][k] * y;
             }
-            stage(buf ^ 1);
+        } else {
+#pragma unroll 8
+            for (int k = 0; k < nb; ++k) {
+                const double y = ys[k][c];
+#pragma unroll
+                for (int m = 0; m < 4; ++m) v[m] += g[m][k] * y;
+            }
         }
-        __syncthreads();                                 // the forward solution, read back by the column's lanes
+    };
+    double v[4];
+    fetch(I0, 1);
+    for (int I = I0; I < nblk; ++I) {
+        const int base = I * nb;
+        stage();
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {                    // Y = E - A_I,I-1 P
+            const int i = r0 + 16 * m;
+            if (i < nb) {
+                double t = base + i == cc ? 1.0 : 0.0;
+                if (I > I0)
+#pragma unroll 4
+                    for (int q = 0; q < of.n; ++q) {
+                        const int k = nb + i - of.d[q];
+                        if (k < nb) t -= cf[i * of.n + q] * ps[k][c];
+                    }
+                ys[i][c] = t;
+            }
+        }
+        __syncthreads();
+        fetch(I + 1, 1);
+        product(v);
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            const int i = r0 + 16 * m;
+            if (i < nb) {
+                ps[i][c] = v[m];
+                if (base + i < n && cc < n) Ainv[(long)(base + i) * n + cc] = v[m];
+            }
+        }
+        __syncthreads();
+    }
+    fetch(nblk - 2, -1);
+    for (int I = nblk - 2; I >= 0; --I) {
+        const int base = I * nb;
+        stage();
+        double p[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            const int i = r0 + 16 * m;
+            p[m] = I >= I0 && i < nb && cc < n ? Ainv[(long)(base + i) * n + cc] : 0.0;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {                    // A_I,I+1 X_I+1
+            const int i = r0 + 16 * m;
+            if (i < nb) {
+                double t = 0.0;
+                for (int q = 0; q < of.n; ++q) {
+                    const int k = i + of.d[q] - nb;
+                    if (k >= 0) t += cf[i * of.n + q] * ps[k][c];
+                }
+                ys[i][c] = t;
+            }
+        }
+        __syncthreads();
+        fetch(I - 1, -1);
+        product(v);
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            const int i = r0 + 16 * m;
+            if (i < nb) {
+                ps[i][c] = p[m] - v[m];
+                if (cc < n) Ainv[(long)(base + i) * n + cc] = p[m] - v[m];
+            }
+        }
+        __syncthreads();
     }
 }
 

@@ -2053,7 +2053,7 @@ struct p4g_solver_s {
     double* ms_buf = nullptr;             // its vectors
     double* ms_ilu9 = nullptr;            // its box-pattern ILU(0) factor (-pc_type ilu)
     std::vector<SorPipe> ms_pipes;        // its levels' pipelined SOR flags (-mg_levels_pc_type sor)
-    double* ms_band = nullptr;            // the coarse band LU factor, uploaded for the inverse
+    double* ms_band = nullptr;            // the coarse operator in band form, its blocks' inverses
     long ms_band_cap = 0;
     std::vector<double> ms_fhist;         // |F| per Newton iterate
     std::vector<int> ms_kits, ms_kreason, ms_sym;   // per Newton step

@@ -101,7 +101,8 @@ static int coarse_factor_band(p4g_solver_s* s, const LevelInfo& L, const double*
         P4G_TRY(coarse_factor(L, g27, Ainv));
         return e.set_coarse_inverse(Ainv);
     }
-    const size_t cap = (size_t)n * w + 1;               // and the pivot word
+    // the band, the pivot word and the blocks' inverses
+    const size_t cap = (size_t)n * w + 1 + (bw < 64 ? blk_words(n, bw) : 0);
     if (!s->ms_band || s->ms_band_cap < (long)cap) {
         P4G_TRY(dalloc(s, (void**)&s->ms_band, cap * sizeof(double)));
         s->ms_band_cap = (long)cap;
@@ -111,8 +112,19 @@ static int coarse_factor_band(p4g_solver_s* s, const LevelInfo& L, const double*
     LAUNCH_CHECK();
     int bad = 0;
     if (bw < 64) {
-        k_band_lu<<<1, 1024, 0, st>>>(n, bw, s->ms_band, spd ? 1 : 0, info);
-        k_band_inverse<<<(n + 15) / 16, 64, 0, st>>>(n, bw, s->ms_band, e.Ainv);
+        BandOff of{0, {}};
+        for (int c = 14; c < 27; ++c) {                  // the later neighbours' distances, each once
+            const int d = ((c / 9 - 1) * my + (c / 3 % 3 - 1)) * mx + c % 3 - 1;
+            const bool there = (L.dim == 3 || c / 9 == 1) && (L.dim >= 2 || c / 3 % 3 == 1) && d >= 1 && d <= bw && d < n;
+            if (there && std::find(of.d, of.d + of.n, d) == of.d + of.n) of.d[of.n++] = d;
+        }
+        if (!of.n) of.d[of.n++] = 1;                     // (a single point)
+        double* const G = s->ms_band + (size_t)n * w + 1;
+        const int nb = blk_rows(n, bw);
+        if (nb <= 16) k_blk_factor<4><<<1, 256, 0, st>>>(n, bw, nb, of, s->ms_band, spd ? 1 : 0, G, info);
+        else if (nb <= 36) k_blk_factor<9><<<1, 256, 0, st>>>(n, bw, nb, of, s->ms_band, spd ? 1 : 0, G, info);
+        else k_blk_factor<16><<<1, 256, 0, st>>>(n, bw, nb, of, s->ms_band, spd ? 1 : 0, G, info);
+        k_blk_inverse<<<(n + 15) / 16, 256, 0, st>>>(n, bw, nb, of, s->ms_band, G, e.Ainv);
         LAUNCH_CHECK();
         HIP_TRY(hipMemcpyAsync(&bad, info, sizeof(int), hipMemcpyDeviceToHost, st));
         HIP_TRY(hipStreamSynchronize(st));
