@@ -310,7 +310,7 @@ int p4g_vi_get_history(p4g_Solver s, double *fnorm, int *ksp_its, int *ksp_reaso
  * Jacobian by colored finite differences (PETSc's "wp" step), the solver's
  * KSP (GMRES unless -ksp_type cg; -ksp_gmres_restart) with PC ILU(0)
  * (default), mg (each coarser level: the finite-difference Jacobian at the
- * injected iterate; coarse band LU) or none, the bt (alpha 1e-4) or basic
+ * injected iterate; coarse direct solve) or none, the bt (alpha 1e-4) or basic
  * line search, SNESConvergedDefault.  -snes_mf_operator: the Krylov
  * operator is MatMFFD at the iterate ("wp" step h = 1.49e-8 sqrt(1 + |x|) /
  * |a|), the grid's Jacobian callback (minimal.c registers the Poisson

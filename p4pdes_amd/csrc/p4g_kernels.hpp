@@ -3250,8 +3250,9 @@ k_blk_inverse(int n, int bw, int nb, BandOff of, const double* __restrict__ B, c
     }
 }
 
-// The same for wider bands: thread c solves L U z = e_c and writes column c of
-// the row-major inverse, which is also its workspace (coalesced across c).
+// The inverse from a band LU, for bands of 64 and more: thread c solves
+// L U z = e_c and writes column c of the row-major inverse, which is also its
+// workspace (coalesced across c).
 __global__ void __launch_bounds__(256)
 k_band_inverse_wide(int n, int bw, const double* __restrict__ B, double* __restrict__ Ainv) {
     const int c = blockIdx.x * 256 + threadIdx.x;

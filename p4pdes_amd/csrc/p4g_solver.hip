@@ -129,8 +129,8 @@ static void sor_pipe_run(const LevelInfo& L, SorPipe* P, const double* r, double
     if (P->kind == SOR_7PT) {
         k_sor7_pack<<<dim3(P->Tp / 64, P->ns * P->ng), 256, 0, st>>>(L.mx, L.my, L.mz, P->Tp, P->ns, r, P->S);
         const Sor7Args A{L.mx, L.my, L.mz, P->Tp, P->ns, P->ng, L.d, L.sx, L.sy, L.sz, P->S, P->yh, P->zh, c};
-        k_sor7<false><<<P->ns * P->ng, 64, 0, st>>>(A);
-        k_sor7<true><<<P->ns * P->ng, 64, 0, st>>>(A);
+        k_sor7<false><<<Sor7::blocks(P->ns * P->ng), 64, 0, st>>>(A);
+        k_sor7<true><<<Sor7::blocks(P->ns * P->ng), 64, 0, st>>>(A);
         return;
     }
     const Sor2Args A{L.mx, L.my, P->Tp, P->ns, L.d, L.db, L.sx, L.sy, P->pk, P->inv, r, P->S, z, P->yh, c};

@@ -622,7 +622,12 @@ k_sor9_pack(int mx, int my, int Tp, const double* __restrict__ g, T2<double>* __
 // kk, so plane kk - 1's value at that point is the lane's result of the step
 // before, and the planes of a step are independent chains that hide each
 // other's latency.  The wave's last plane goes to the next plane group by
-// step, tagged; its last row to the next strip as in 2D.
+// step, tagged; its last row to the next strip as in 2D.  Bound by the
+// hand-over from group to group (257^3: 63 of them at 4.7 us each, in a sweep
+// of 393 us; a step is 0.22 us), so the words are asked for half a batch
+// before they are needed: four batches ahead, they were asked for too early
+// and a group settled four batches behind the one before (553 us a sweep).
+// Batches of 2 steps: 415 us.
 constexpr int kSor7Planes = 4;
 
 struct Sor7 {
@@ -633,6 +638,12 @@ struct Sor7 {
         return (need + 63) / 64 * 64;
     }
     __host__ __device__ static int strips(int my) { return (my - 2 + 63) / 64; }
+    // workgroup o's block, in dispatch order: an eighth of the workgroups, but
+    // no fewer than 32, on one XCD
+    __host__ __device__ static int block_of(int o, int nwg) {
+        return o * kXcds + o / (nwg > 32 * kXcds ? (nwg + kXcds - 1) / kXcds : 32);
+    }
+    __host__ __device__ static int blocks(int nwg) { return block_of(nwg - 1, nwg) + 1; }
     __host__ __device__ static int groups(int mz) { return (mz - 2 + K - 1) / K; }
 };
 
@@ -648,7 +659,8 @@ struct Sor7Args {
 template <bool BWD>
 __global__ void __launch_bounds__(64) k_sor7(Sor7Args A) {
     constexpr int K = Sor7::K, SB = Sor7::SB, D = Sor7::D;
-    const int r = threadIdx.x, o = blockIdx.x, ns = A.ns, ng = A.ng;
+    const int r = threadIdx.x, o = blockIdx.x >> 3, ns = A.ns, ng = A.ng;
+    if ((int)blockIdx.x != Sor7::block_of(o, ns * ng)) return;
     const int os = o % ns, og = o / ns;
     const int s = BWD ? ns - 1 - os : os, g = BWD ? ng - 1 - og : og, rho = BWD ? 63 - r : r;
     const int Tp = A.Tp, ncol = A.mx - 2;
@@ -674,18 +686,18 @@ __global__ void __launch_bounds__(64) k_sor7(Sor7Args A) {
     __shared__ double obuf[SB * K][64];    // the batch's results
     const int ye = r / K, yk = r % K;      // lane r < SB * K carries step ye, plane yk
 
-    struct Ops {
-        T2<double> v[SB][K / 2];
+    T2<double> ops[D][SB][K / 2];
+    struct Words {               // loaded half a batch ahead: any earlier, and they are not there yet
         Tagged z[SB];            // the previous group's last plane at the lane's column
         Tagged y;                // lane r < SB * K: the previous strip's last row, of the batch after
-    } ops[D];
+    } zw[2];
 
-    auto yload = [&](int t0, Ops& P) {
+    auto yload = [&](int t0, Words& P) {
         const int c = min(max(t0 + min(ye, SB - 1) - yk - sh, 0), ncol - 1);
         P.y.lo = ld_word(yin + 2 * (c * K + yk));
         P.y.hi = ld_word(yin + 2 * (c * K + yk) + 1);
     };
-    auto zload = [&](int t0, Ops& P) {
+    auto zload = [&](int t0, Words& P) {
 #pragma unroll
         for (int e = 0; e < SB; ++e) {
             const char* const p = zin + (long)(t0 + e) * 1024;
@@ -694,21 +706,19 @@ __global__ void __launch_bounds__(64) k_sor7(Sor7Args A) {
         }
     };
     // every path issues the same loads, so that the compiler can count them
-    auto load = [&](int t0, Ops& P) {
-        yload(t0 + SB, P);
-        zload(t0, P);
+    auto load = [&](int t0, T2<double> (&P)[SB][K / 2]) {
 #pragma unroll
         for (int e = 0; e < SB; ++e) {
             const unsigned tf = BWD ? Tp - 1 - (t0 + e) : t0 + e;
 #pragma unroll
-            for (int p = 0; p < K / 2; ++p) P.v[e][p] = buffer_ld2(Sr, v16, (tf * (K / 2) + p) * 1024u);
+            for (int p = 0; p < K / 2; ++p) P[e][p] = buffer_ld2(Sr, v16, (tf * (K / 2) + p) * 1024u);
         }
     };
     auto yneed = [&](int t0) {
         const int c = t0 + ye - yk - sh;
         return hy && r < SB * K && c >= 0 && c < ncol;
     };
-    auto zready = [&](int t0, const Ops& P) {
+    auto zready = [&](int t0, const Words& P) {
         bool ok = true;
 #pragma unroll
         for (int e = 0; e < SB; ++e) {
@@ -720,14 +730,14 @@ __global__ void __launch_bounds__(64) k_sor7(Sor7Args A) {
     double xs[K];
 #pragma unroll
     for (int kk = 0; kk < K; ++kk) xs[kk] = 0.0;
-    // the steps of a batch; edge: some point is off the grid
-    auto steps = [&](int t0, const Ops& P, bool edge) {
+    // half the steps of a batch; edge: some point is off the grid
+    auto steps = [&](int t0, const T2<double> (&P)[SB][K / 2], const Words& W, bool edge, int E) __attribute__((always_inline)) {
         const double* const yb = ybuf[(t0 / SB) & 1];
 #pragma unroll
-        for (int e = 0; e < SB; ++e) {
+        for (int e = E; e < E + SB / 2; ++e) {
             const int t = t0 + e, c0 = t - off;
             const unsigned tf = BWD ? Tp - 1 - t : t;
-            const double z0 = hz && (!edge || (rl && (unsigned)c0 < (unsigned)ncol)) ? P.z[e].value() : 0.0;
+            const double z0 = hz && (!edge || (rl && (unsigned)c0 < (unsigned)ncol)) ? W.z[e].value() : 0.0;
             double keep[K];
 #pragma unroll
             for (int kk = K - 1; kk >= 0; --kk) {      // plane kk - 1 still holds the step before
@@ -735,7 +745,7 @@ __global__ void __launch_bounds__(64) k_sor7(Sor7Args A) {
                 const double nb = wave_shr1(xs[kk], yb[e * K + kk]);
                 const double below = kk ? xs[kk > 0 ? kk - 1 : 0] : z0;
                 const double own = xs[kk];
-                double sum = (kf & 1) ? P.v[e][kf / 2].b : P.v[e][kf / 2].a;
+                double sum = (kf & 1) ? P[e][kf / 2].b : P[e][kf / 2].a;
                 if (!BWD) {
                     sum += A.sz * below;
                     sum += A.sy * nb;
@@ -761,7 +771,7 @@ __global__ void __launch_bounds__(64) k_sor7(Sor7Args A) {
         }
     };
     // waits for the words of batch t0's planes and of the next batch's rows
-    auto wait = [&](int t0, Ops& P, int q) {
+    auto wait = [&](int t0, Words& P) __attribute__((always_inline)) {
         const bool need = yneed(t0 + SB);
         if (!dead && !((!hz || zready(t0, P)) && (!hy || __all(!need || P.y.is(want))))) {
             long spins = 0;
@@ -770,19 +780,13 @@ __global__ void __launch_bounds__(64) k_sor7(Sor7Args A) {
                 zload(t0, P);
                 yload(t0 + SB, P);
             } while (!dead && !((!hz || zready(t0, P)) && (!hy || __all(!need || P.y.is(want)))));
-            // the words of the batches after were loaded too early as well
-#pragma unroll
-            for (int h = 1; h < D; ++h) {
-                zload(min(t0 + h * SB, Tp - SB), ops[(q + h) % D]);
-                yload(t0 + h * SB + SB, ops[(q + h) % D]);
-            }
             __builtin_amdgcn_s_waitcnt(0);   // so that the other path's waits stay as they are
         }
         if (r < SB * K) ybuf[((t0 / SB) & 1) ^ 1][r] = need ? P.y.value() : 0.0;
         wave_lds_order();
     };
     {   // the first batch's rows
-        Ops first;
+        Words first;
         yload(0, first);
         const bool need = yneed(0);
         long spins = 0;
@@ -794,14 +798,22 @@ __global__ void __launch_bounds__(64) k_sor7(Sor7Args A) {
         __builtin_amdgcn_s_waitcnt(0);
     }
 #pragma unroll
-    for (int q = 0; q < D; ++q) load(q * SB, ops[q]);
-    for (int t0 = 0; t0 < Tp; t0 += SB * D) {
+    for (int q = 0; q < D; ++q) {
+        load(q * SB, ops[q]);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    zload(0, zw[0]);
+    yload(SB, zw[0]);
+    auto round = [&](int t0, bool edge) __attribute__((always_inline)) {
 #pragma unroll
         for (int q = 0; q < D; ++q) {
             const int t = t0 + q * SB;
-            wait(t, ops[q], q);
-            if (full && t - sh >= 63 + K - 1 && t + SB - sh <= ncol) steps(t, ops[q], false);
-            else steps(t, ops[q], true);
+            wait(t, zw[q & 1]);
+            steps(t, ops[q], zw[q & 1], edge, 0);
+            const int tn = min(t + SB, Tp - SB);
+            zload(tn, zw[(q & 1) ^ 1]);
+            yload(tn + SB, zw[(q & 1) ^ 1]);
+            steps(t, ops[q], zw[q & 1], edge, SB / 2);
             wave_lds_order();
             if (os < ns - 1) {             // the last lane's results, at their columns
                 const int c = t + ye - 63 - yk - sh;
@@ -812,7 +824,14 @@ __global__ void __launch_bounds__(64) k_sor7(Sor7Args A) {
             wave_lds_order();
             load(min(t + SB * D, Tp - SB), ops[q]);
         }
-    }
+    };
+    // three loops, because a ring that two paths of one loop load ends in
+    // moves between registers
+    int t0 = 0;
+    const int lo = full ? sh + 63 + K - 1 : Tp, hi = ncol + sh - SB * D;
+    for (; t0 < min(lo, Tp); t0 += SB * D) round(t0, true);
+    for (; t0 <= hi; t0 += SB * D) round(t0, false);
+    for (; t0 < Tp; t0 += SB * D) round(t0, true);
     if (BWD && o == ns * ng - 1 && r == 0) A.c.ctl[1] += 1;
 }
 
