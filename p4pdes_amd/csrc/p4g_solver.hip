@@ -133,17 +133,22 @@ static void sor_pipe_run(const LevelInfo& L, SorPipe* P, const double* r, double
         k_sor7<true><<<Sor7::blocks(P->ns * P->ng), 64, 0, st>>>(A);
         return;
     }
-    const Sor2Args A{L.mx, L.my, P->Tp, P->ns, L.d, L.db, L.sx, L.sy, P->pk, P->inv, r, P->S, z, P->yh, c};
-    if (P->kind == SOR_9PT) {
-        typedef Sor2<true> G;
-        k_sor2<true, false><<<G::blocks(P->ns), G::NT, G::LDS, st>>>(A);
-        k_sor2<true, true><<<G::blocks(P->ns), G::NT, G::LDS, st>>>(A);
-    } else {
-        typedef Sor2<false> G;
-        const int nb = (2 * (L.mx + L.my) + 4 * G::NT - 1) / (4 * G::NT);      // boundary rows, four points a lane
-        k_sor2<false, false><<<G::blocks(P->ns) + nb, G::NT, G::LDS, st>>>(A);
-        k_sor2<false, true><<<G::blocks(P->ns), G::NT, G::LDS, st>>>(A);
-    }
+    Sor2Args A{L.mx, L.my, P->Tp, P->ns, 0, L.d, L.db, L.sx, L.sy, P->pk, P->inv, r, P->S, z, P->yh, c};
+    for (int bwd = 0; bwd < 2; ++bwd)
+        for (A.o0 = 0; A.o0 < P->ns; A.o0 += Sor2<false>::NSTRIP) {
+            const int nl = std::min<int>(P->ns - A.o0, Sor2<false>::NSTRIP);
+            if (P->kind == SOR_9PT) {
+                typedef Sor2<true> G;
+                if (bwd) k_sor2<true, true><<<G::blocks(nl), G::NT, G::LDS, st>>>(A);
+                else k_sor2<true, false><<<G::blocks(nl), G::NT, G::LDS, st>>>(A);
+            } else {
+                typedef Sor2<false> G;
+                // the boundary rows, four points a lane
+                const int nb = A.o0 ? 0 : (2 * (L.mx + L.my) + 4 * G::NT - 1) / (4 * G::NT);
+                if (bwd) k_sor2<false, true><<<G::blocks(nl), G::NT, G::LDS, st>>>(A);
+                else k_sor2<false, false><<<G::blocks(nl) + nb, G::NT, G::LDS, st>>>(A);
+            }
+        }
 }
 
 // y = a p + c q + e SSOR(r) from the sweep's order (3D)

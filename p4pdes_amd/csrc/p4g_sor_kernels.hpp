@@ -172,13 +172,17 @@ struct Sor2 {
     __host__ __device__ static int rows(int my) { return NINE ? my : my - 2; }
     __host__ __device__ static int strips(int my) { return (rows(my) + 63) / 64; }
     // strip o's block: runs of 32 strips on one XCD, whose L2 hands rows over
-    // soonest (264-271 ns one way against 330-494), in dispatch order
-    __host__ __device__ static int block_of(int o) { return o * kXcds + (o >> 5) % kXcds; }
+    // soonest (264-271 ns one way against 330-494), in dispatch order.  A
+    // launch takes 256 strips at most, a compute unit each, so that an XCD's
+    // strips wait for lower ones on it or on a lower XCD only, also where
+    // several sweeps share the GPU.
+    static constexpr int NSTRIP = 32 * kXcds;
+    __host__ __device__ static int block_of(int o) { return o * kXcds + (o >> 5); }
     __host__ __device__ static int blocks(int ns) { return block_of(ns - 1) + 1; }
 };
 
 struct Sor2Args {
-    int mx, my, Tp, ns;
+    int mx, my, Tp, ns, o0;          // strips, and the launch's first (in sweep order)
     double d, db, sx, sy;            // 5-point
     const T2<double>* pk;            // 9-point: per step 4 x 64 coefficient pairs (k_sor9_pack)
     const T2<double>* inv;           // 9-point: reciprocal diagonals, two steps per pair
@@ -204,10 +208,10 @@ __global__ void __launch_bounds__(Sor2<NINE>::NT) k_sor2(Sor2Args A) {
     const int r = threadIdx.x & 63, place = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wave = place == 3 ? 0 : (place == 0 ? 3 : place);
     const int mx = A.mx, my = A.my, ns = A.ns;
-    const int o = (int)blockIdx.x >> 3;
-    if (!NINE && !BWD && (int)blockIdx.x >= G::blocks(ns)) {          // the boundary rows
+    const int nl = min(ns - A.o0, (int)G::NSTRIP), ol = (int)blockIdx.x >> 3, o = A.o0 + ol;
+    if (!NINE && !BWD && (int)blockIdx.x >= G::blocks(nl)) {          // the boundary rows
         const double idb = 1.0 / A.db;
-        const int per = 2 * mx + 2 * (my - 2), b0 = G::blocks(ns);
+        const int per = 2 * mx + 2 * (my - 2), b0 = G::blocks(nl);
         for (int p = ((int)blockIdx.x - b0) * G::NT + threadIdx.x; p < per; p += (gridDim.x - b0) * G::NT) {
             long q;
             if (p < mx) q = p;
@@ -217,7 +221,7 @@ __global__ void __launch_bounds__(Sor2<NINE>::NT) k_sor2(Sor2Args A) {
         }
         return;
     }
-    if (o >= ns || (int)blockIdx.x != G::block_of(o)) return;
+    if (ol >= nl || (int)blockIdx.x != G::block_of(ol)) return;
     const int Tp = A.Tp, NB = Tp / SB, ncol = G::cols(mx), nrow = G::rows(my);
     const int s = BWD ? ns - 1 - o : o;
     const int sh = BWD ? (NINE ? Tp - 2 - (mx + 126) : Tp - (ncol + 63)) : 0;

@@ -2,7 +2,8 @@
 (k_sor_plane): every point is updated from the same values in the same order,
 so one preconditioner application agrees bit for bit.  One-level grids take
 any size (the smoother is the preconditioner): the edges of a strip's 64 rows,
-of the batches of steps and of the plane groups, 35 strips (on two XCDs), single
+of the batches of steps and of the plane groups, 35 strips (on two XCDs), 258
+(two launches), single
 interior points, and boxes longer in each direction."""
 import numpy as np
 import pytest
@@ -11,7 +12,7 @@ from p4pdes_amd import capi
 
 pytestmark = pytest.mark.gpu
 
-GRIDS_2D = [(19, 2200), (3, 3), (4, 3), (3, 70), (35, 5), (66, 66), (67, 65), (34, 131), (130, 67), (260, 130), (97, 200)]
+GRIDS_2D = [(19, 2200), (5, 16500), (3, 3), (4, 3), (3, 70), (35, 5), (66, 66), (67, 65), (34, 131), (130, 67), (260, 130), (97, 200)]
 GRIDS_3D = [(3, 3, 3), (4, 5, 6), (66, 5, 3), (5, 66, 7), (6, 67, 8), (7, 4, 70), (33, 34, 35), (67, 130, 9), (65, 65, 65)]
 
 
