@@ -139,8 +139,8 @@ struct OpVar {
     // read its eight cells one by one.  What bounds these passes is registers:
     // loading a layer a plane ahead took 141-145 and left one block of eight
     // waves a compute unit (257^3: the CG operator pass 305 us against 254
-    // with single cells); without, and held to 128 (4 waves a SIMD, a few
-    // spills), it is 243, and the post-smoothing pass 353 against 386.
+    // with single cells); without, and held to 128 (4 waves a SIMD, at most
+    // five spills), it is 243, and the post-smoothing pass 353 against 386.
     template <int V>
     struct Cells {
         T v[2][V + 1];
@@ -206,7 +206,9 @@ struct OpVar {
     }
     __device__ __forceinline__ void interior(int i, int j, int k, T uc, T w, T e, T s, T n, T dn, T up, T& Au,
                                              T& idg_) const {
-        interiorc<1>(0, cells<1>(i, j, k - 1), cells<1>(i, j, k), uc, w, e, s, n, dn, up, Au, idg_);
+        const Cells<1> lo{{{cell(i - 1, j - 1, k - 1), cell(i, j - 1, k - 1)}, {cell(i - 1, j, k - 1), cell(i, j, k - 1)}}};
+        const Cells<1> hi{{{cell(i - 1, j - 1, k), cell(i, j - 1, k)}, {cell(i - 1, j, k), cell(i, j, k)}}};
+        interiorc<1>(0, lo, hi, uc, w, e, s, n, dn, up, Au, idg_);
     }
 };
 
@@ -814,6 +816,19 @@ __device__ __forceinline__ Tile xcd_tile() {
 
 // ------------------------------------------------------------- stencil
 
+// The passes over cell coefficients that march whole cell layers
+// (OpVar::cells); the others read a point's eight cells one by one.  In FP64
+// an output that loads arrays ahead leaves no registers for the layers: held
+// to 128 such a pass spilled 7-39 of them (257^3, layers against single
+// cells: Chebyshev step 225 / 195 us, with a second array and dots 445 / 273,
+// residual 191 / 183, residual of the zero-guess step 288 / 245).  Without
+// such an array, and in FP32, the layers are faster (CG operator pass 242 /
+// 254 us; FP32 V(2,2) solve 7.1 / 8.3 ms).
+template <typename T, class Op, class Out>
+constexpr bool cells_marched() {
+    return Op::CELLS && (sizeof(T) == 4 || Out::NPRE == 0);
+}
+
 // Marching stencil pass over a 2D or 3D grid: for every vertex, u from Src,
 // A u and the Jacobi factor from Op, result written by Out.  A lane owns V
 // consecutive x points i0 .. i0+V-1, i0 = 1 + V (64 bx + lane), moved with
@@ -839,6 +854,7 @@ __device__ __forceinline__ void stencil_vec(int bx, int by, int bz, int mx, int 
     static_assert(PD >= 1 && PD <= 4, "prefetch distance");
     constexpr bool PSN = (PF & 1) != 0 && DIM == 3, PEX = (PF & 2) != 0;
     constexpr int NP = Out::NPRE, NPA = NP > 0 ? NP : 1;
+    constexpr bool MC = cells_marched<T, Op, Out>();
     const int lane = threadIdx.x;
     const int i0 = 1 + V * (bx * TX + lane);
     const T z0 = T(0);
@@ -918,7 +934,7 @@ __device__ __forceinline__ void stencil_vec(int bx, int by, int bz, int mx, int 
     // the cell layers below and above plane m (OpVar, 3D)
     typename Op::template Cells<V> cl{}, ch{};
     auto CL = [&](int p, typename Op::template Cells<V>& c) {
-        if constexpr (Op::CELLS)
+        if constexpr (MC)
             if (act && !jb && p >= 0 && p < M - 1) c = op.template cells<V>(i0, j, p);
     };
     CL(m0 - 1, ch);
@@ -939,7 +955,7 @@ __device__ __forceinline__ void stencil_vec(int bx, int by, int bz, int mx, int 
     for (int m = m0; m < m1; ++m, q += sm) {
         if (act && m + PD <= mlast)
             LR(q + PD * sm, m + PD < m1, ru[PD - 1], rx[PD - 1], ro[PD - 1], rox[PD - 1]);
-        if constexpr (Op::CELLS) {
+        if constexpr (MC) {
             cl = ch;
             CL(m, ch);
         }
@@ -994,12 +1010,12 @@ __device__ __forceinline__ void stencil_vec(int bx, int by, int bz, int mx, int 
                     const int i = i0 + e;
                     if (e < ne) {
                         if (i == mx - 1) {
-                            if constexpr (Op::CELLS) op.template bndx<V>(e, cl, ch, uc.v[e], Au.v[e], idg.v[e]);
+                            if constexpr (MC) op.template bndx<V>(e, cl, ch, uc.v[e], Au.v[e], idg.v[e]);
                             else op.bnd(i, jj, kk, uc.v[e], Au.v[e], idg.v[e]);
                         } else {
                             const T w = e == 0 ? (i - 1 > 0 ? wv : z0) : uc.v[e > 0 ? e - 1 : 0];
                             const T east = i + 1 < mx - 1 ? (e == V - 1 ? ev : uc.v[e < V - 1 ? e + 1 : 0]) : z0;
-                            if constexpr (Op::CELLS)
+                            if constexpr (MC)
                                 op.template interiorc<V>(e, cl, ch, uc.v[e], w, east, sv.v[e], nv.v[e], dn.v[e],
                                                          up.v[e], Au.v[e], idg.v[e]);
                             else
@@ -1021,7 +1037,7 @@ __device__ __forceinline__ void stencil_vec(int bx, int by, int bz, int mx, int 
                 const T u0 = PEX ? cx : src.load(q - 1);
                 T A0, i00;
                 src.put(q - 1, u0);
-                if constexpr (Op::CELLS) {
+                if constexpr (MC) {
                     if (jb || m == 0 || m == M - 1) op.bnd(0, jj, kk, u0, A0, i00);
                     else op.template bndx<V>(0, cl, ch, u0, A0, i00);
                 } else {
@@ -1089,7 +1105,7 @@ __device__ __forceinline__ void stencil_body(int bx, int by, int bz, int mx, int
 }
 
 template <typename T, int DIM, class Op, class Src, class Out>
-__global__ void __launch_bounds__(NT, Op::CELLS ? 4 : 1)   // (4 waves a SIMD: see OpVar::cells)
+__global__ void __launch_bounds__(NT, (cells_marched<T, Op, Out>() ? 4 : 1))   // (4 waves a SIMD: see OpVar::cells)
 k_stencil(int mx, int my, int mz, int kch, Op op, Src src, Out out, double* __restrict__ part) {
     double a0 = 0.0, a1 = 0.0;
     const Tile tl = xcd_tile();

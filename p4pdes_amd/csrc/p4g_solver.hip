@@ -592,7 +592,7 @@ struct Engine {
                 HIP_TRY(hipMemcpy(d.kc, tmp.data(), ncell * sizeof(T), hipMemcpyHostToDevice));
                 // a cycle's zero-guess step is then formed where it is read
                 // (mcycle): 257^3, the step's own pass 148 and the residual's
-                // 187 us before, one pass of 286 us now
+                // 187 us before, one pass of 245 us now
                 if (pctype == PCT_MG && l > 0 && nu == 1 && L.dim == 3) {
                     P4G_TRY(alloc(&d.idg, L.n));
                     OpVar<T> o = opv(l, jacobi != 0);
