@@ -201,7 +201,7 @@ static const double* solver_ainv(p4g_solver_s* s) {
 static GridRef gref_stencil(const LevelInfo& L, long start, int V) {
     const dim3 g = stencil_grid_v(L.dim, L.mx, L.my, L.mz, V);
     GridRef r;
-    r.mx = L.mx; r.my = L.my; r.mz = L.mz; r.kch = kchf(L.dim, L.my, L.mz);
+    r.mx = L.mx; r.my = L.my; r.mz = L.mz; r.kch = kchf(L.dim, L.mx, L.my, L.mz);
     r.gx = g.x; r.gy = g.y; r.gz = g.z; r.start = start;
     return r;
 }
@@ -210,14 +210,14 @@ static GridRef gref_stencil(const LevelInfo& L, long start, int V) {
 static GridRef gref_fused(const LevelInfo& L, long start) {
     const dim3 g = fused_grid(L.dim, L.mx, L.my, L.mz);
     GridRef r;
-    r.mx = L.mx; r.my = L.my; r.mz = L.mz; r.kch = kch_fused(L.dim, L.my, L.mz);
+    r.mx = L.mx; r.my = L.my; r.mz = L.mz; r.kch = kch_fused(L.dim, L.mx, L.my, L.mz);
     r.gx = g.x; r.gy = g.y; r.gz = g.z; r.start = start;
     return r;
 }
 
 // restriction launch over the coarse grid L (lanes over its columns 1..mx-1)
 static GridRef gref_restrict(const LevelInfo& L, long start) {
-    const int kch = kch_restrict(L.dim, L.my, L.mz);
+    const int kch = kch_restrict(L.dim, L.mz);
     const dim3 g = transfer_grid(L.dim, L.mx, L.my, L.mz, kch);
     GridRef r;
     r.mx = L.mx; r.my = L.my; r.mz = L.mz; r.kch = kch;

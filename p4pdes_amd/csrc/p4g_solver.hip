@@ -59,14 +59,18 @@ enum { PCT_MG = 0, PCT_JACOBI, PCT_NONE, PCT_ILU, PCT_ASM };
 enum { SM_CHEB = 0, SM_RICH };
 enum { NT_PRECOND = 0, NT_UNPRECOND, NT_NATURAL };
 
-// marching chunk: one plane (row in 2D) per thread on small grids
-// (latency-bound, want parallelism), longer chunks on large ones (fewer halo
-// re-reads).  A 2D row is one wave per 128 points, so a 2D grid fills the
-// chip's 1024 SIMDs from about 400^2 on and takes the short chunks to 800^2
-// (129^2: direction pass 8.2 us with four rows a thread, prolongation and
-// smoothing 15.1 us with eight).
-static inline int kchf(int dim, int my, int mz) {
-    if (dim == 2) return my >= 1600 ? 8 : (my >= 800 ? 4 : (my >= 400 ? 2 : 1));
+// marching chunk, planes (rows in 2D) per thread: one on small grids
+// (latency-bound, want parallelism), longer ones on large grids (fewer halo
+// re-reads).  In 2D a row is a wave for 128 points, so one row a thread fills
+// the chip's 1024 SIMDs from about 128 000 points on, and the re-read rows come
+// from the caches until the grid has outgrown them: two rows beyond 4.5
+// million points (solves with one / two / four rows a thread: 2049^2 1.51 /
+// 1.57 / 1.77 ms, 16385x129 1.20 / 1.27 / 1.41, 129x16385 1.29 / 1.31 / 1.63;
+// 6145x769 with one / two 1.64 / 1.58, 4097^2 4.42 / 4.20 / 4.41, 131073x257
+// 8.54 / 8.19 / 8.25, 257x65537 4.56 / 4.44 / 4.88; eight rows are slower than
+// four in all of them).
+static inline int kchf(int dim, int mx, int my, int mz) {
+    if (dim == 2) return (long)mx * my > 4500000 ? 2 : 1;
     const int slow = dim == 3 ? mz : 1;
     return slow >= 400 ? 8 : (slow >= 100 ? 4 : 1);
 }
@@ -384,16 +388,16 @@ static dim3 stencil_grid_k(int dim, int mx, int my, int mz, int V, int kch) {
     return dim3(gx, ((my + kch - 1) / kch + TY - 1) / TY, 1);
 }
 static dim3 stencil_grid_v(int dim, int mx, int my, int mz, int V) {
-    return stencil_grid_k(dim, mx, my, mz, V, kchf(dim, my, mz));
+    return stencil_grid_k(dim, mx, my, mz, V, kchf(dim, mx, my, mz));
 }
 // marching chunk of the fused prolongation + smoothing kernel: its per-chunk
 // set-up (coarse planes, the first iterates, the halo rows) is longer, so
 // chunks are longer than those of the stencil passes (3D, 6-row blocks:
 // 257^3 120 us at 16 planes, 134 us at 8; 513^3 855 us at 16, 939 us at 8)
-static inline int kch_fused(int dim, int my, int mz) {
-    if (dim == 2) return 2 * kchf(dim, my, mz);
+static inline int kch_fused(int dim, int mx, int my, int mz) {
+    if (dim == 2) return 2 * kchf(dim, mx, my, mz);
     const int slow = dim == 3 ? mz : 1;
-    return slow >= 200 ? 16 : std::min(16, 2 * kchf(dim, my, mz));
+    return slow >= 200 ? 16 : std::min(16, 2 * kchf(dim, mx, my, mz));
 }
 template <typename T>
 static dim3 stencil_grid(int dim, int mx, int my, int mz) { return stencil_grid_v(dim, mx, my, mz, VecOf<T>::V); }
@@ -401,7 +405,7 @@ static dim3 stencil_grid(int dim, int mx, int my, int mz) { return stencil_grid_
 static dim3 pair_grid(int dim, int mx, int my, int mz) { return stencil_grid_v(dim, mx, my, mz, 2); }
 // the fused prolongation + smoothing kernel (two points per lane)
 static dim3 fused_grid(int dim, int mx, int my, int mz) {
-    const int kch = kch_fused(dim, my, mz);
+    const int kch = kch_fused(dim, mx, my, mz);
     if (dim == 3) return dim3((mx - 1 + 2 * TX - 1) / (2 * TX), (my + TYF - 1) / TYF, (mz + kch - 1) / kch);
     return stencil_grid_k(dim, mx, my, mz, 2, kch);
 }
@@ -424,10 +428,11 @@ static dim3 transfer_grid(int dim, int mxc, int my, int mz, int kch) {
     return dim3(gx, 1, 1);
 }
 // marching chunk of the restriction, in coarse planes (rows in 2D) of the
-// coarse grid (my, mz): each is two fine planes read (fine 257^3: 45 us at
-// 1-2, 48 us at 4; fine 513^3: 293 us at 4, 303 us at 2 or 8)
-static inline int kch_restrict(int dim, int my, int mz) {
-    if (dim == 2) return my >= 800 ? 4 : (my >= 400 ? 2 : 1);
+// coarse grid: each is two fine planes read (fine 257^3: 45 us at 1-2, 48 us
+// at 4; fine 513^3: 293 us at 4, 303 us at 2 or 8).  In 2D one row a thread at
+// every size (2049^2 solve 1.67 ms, with two 1.70 and with four 1.77;
+// 131073x257 8.56, 8.61 and 8.63).
+static inline int kch_restrict(int dim, int mz) {
     const int slow = dim == 3 ? mz : 1;
     return slow >= 200 ? 4 : (slow >= 100 ? 2 : 1);
 }
@@ -598,7 +603,7 @@ struct Engine {
                     OpVar<T> o = opv(l, jacobi != 0);
                     k_stencil<T, 3, OpVar<T>, SrcZero<T>, OutRecipDiag<T>>
                         <<<stencil_grid<T>(3, L.mx, L.my, L.mz), stencil_block(3), 0, cx->stream>>>(
-                            L.mx, L.my, L.mz, kchf(3, L.my, L.mz), o, SrcZero<T>{}, OutRecipDiag<T>{d.idg}, cx->part);
+                            L.mx, L.my, L.mz, kchf(3, L.mx, L.my, L.mz), o, SrcZero<T>{}, OutRecipDiag<T>{d.idg}, cx->part);
                     LAUNCH_CHECK();
                 }
             }
@@ -714,7 +719,7 @@ struct Engine {
             if (L.dim != 3) return set_error(PETSC_ERR_SUP, "variable coefficient needs 3D");
             OpVar<T> o = opv(l, jac);
             return cx->launch(cls, fine, bytes, [&] {
-                k_stencil<T, 3, OpVar<T>, Src, Out><<<g, b, 0, s>>>(L.mx, L.my, L.mz, kchf(L.dim, L.my, L.mz), o, src, out,
+                k_stencil<T, 3, OpVar<T>, Src, Out><<<g, b, 0, s>>>(L.mx, L.my, L.mz, kchf(L.dim, L.mx, L.my, L.mz), o, src, out,
                                                                  part);
             });
         }
@@ -723,19 +728,19 @@ struct Engine {
             if (lds_level(L)) {   // the same grid and block as k_stencil (TYD = TY)
                 return cx->launch(cls, fine, bytes, [&] {
                     k_stencil_lds<T, OpConst<T>, Src, Out, TY, 1><<<g, b, 0, s>>>(
-                        L.mx, L.my, L.mz, kchf(L.dim, L.my, L.mz), o, src, out, part);
+                        L.mx, L.my, L.mz, kchf(L.dim, L.mx, L.my, L.mz), o, src, out, part);
                 });
             }
         }
         return cx->launch(cls, fine, bytes, [&] {
             if (L.dim == 3)
-                k_stencil<T, 3, OpConst<T>, Src, Out><<<g, b, 0, s>>>(L.mx, L.my, L.mz, kchf(L.dim, L.my, L.mz), o, src,
+                k_stencil<T, 3, OpConst<T>, Src, Out><<<g, b, 0, s>>>(L.mx, L.my, L.mz, kchf(L.dim, L.mx, L.my, L.mz), o, src,
                                                                    out, part);
             else if (L.dim == 2)
-                k_stencil<T, 2, OpConst<T>, Src, Out><<<g, b, 0, s>>>(L.mx, L.my, L.mz, kchf(L.dim, L.my, L.mz), o, src,
+                k_stencil<T, 2, OpConst<T>, Src, Out><<<g, b, 0, s>>>(L.mx, L.my, L.mz, kchf(L.dim, L.mx, L.my, L.mz), o, src,
                                                                    out, part);
             else
-                k_stencil<T, 1, OpConst<T>, Src, Out><<<g, b, 0, s>>>(L.mx, L.my, L.mz, kchf(L.dim, L.my, L.mz), o, src,
+                k_stencil<T, 1, OpConst<T>, Src, Out><<<g, b, 0, s>>>(L.mx, L.my, L.mz, kchf(L.dim, L.mx, L.my, L.mz), o, src,
                                                                    out, part);
         });
     }
@@ -755,7 +760,7 @@ struct Engine {
         const LevelInfo& F = (*lv)[l];
         const LevelInfo& C = (*lv)[l - 1];
         const int tyc = rr_rows == 4 ? 4 : 8;
-        const int kch = rr_planes > 0 ? rr_planes : kch_restrict(C.dim, C.my, C.mz);
+        const int kch = rr_planes > 0 ? rr_planes : kch_restrict(C.dim, C.mz);
         constexpr int V = VecOf<T>::V;   // fine points per lane (16-byte accesses)
         if ((F.mx - 1) % (V * TX) != 0) return set_error(PETSC_ERR_LIB, "internal: residual + restriction tile width");
         const dim3 g((F.mx - 1) / (V * TX), (C.my + tyc - 1) / tyc, (C.mz + kch - 1) / kch), b(TX, tyc);
@@ -774,7 +779,7 @@ struct Engine {
     int restrict_(int l, const T* rf, T* bc) {   // level l -> l-1
         const LevelInfo& F = (*lv)[l];
         const LevelInfo& C = (*lv)[l - 1];
-        const int kch = kch_restrict(C.dim, C.my, C.mz);
+        const int kch = kch_restrict(C.dim, C.mz);
         const dim3 g = transfer_grid(C.dim, C.mx, C.my, C.mz, kch), b = stencil_block(C.dim);
         hipStream_t s = cx->stream;
         return cx->launch(P4G_K_RESTRICT, l == nlev - 1, double(F.n + C.n) * sizeof(T), [&] {
@@ -799,7 +804,7 @@ struct Engine {
             return set_error(PETSC_ERR_LIB, "internal: partial-sum buffer too small");
         hipStream_t s = cx->stream;
         const double bytes = passes * L.n * sizeof(T) + C.n * sizeof(T);
-        const int kch = kch_fused(L.dim, L.my, L.mz);
+        const int kch = kch_fused(L.dim, L.mx, L.my, L.mz);
         if (L.var) {
             if (L.dim != 3) return set_error(PETSC_ERR_SUP, "variable coefficient needs 3D");
             OpVar<T> o = opv(l, jac);
@@ -857,18 +862,18 @@ struct Engine {
     int prolong_q1(int l, bool zg, const T* base, T c, const T* xc, T* out) {
         const LevelInfo& F = (*lv)[l];
         const LevelInfo& C = (*lv)[l - 1];
-        const dim3 g = transfer_grid(F.dim, C.mx, F.my, F.mz, kchf(F.dim, F.my, F.mz)), b = stencil_block(F.dim);
+        const dim3 g = transfer_grid(F.dim, C.mx, F.my, F.mz, kchf(F.dim, F.mx, F.my, F.mz)), b = stencil_block(F.dim);
         hipStream_t s = cx->stream;
         return cx->launch(P4G_K_PROLONG, l == nlev - 1, double(2 * F.n + C.n) * sizeof(T), [&] {
             if (F.dim == 3) {
-                if (zg) k_prolong<T, 3, true><<<g, b, 0, s>>>(F.mx, F.my, F.mz, C.mx, C.my, kchf(F.dim, F.my, F.mz), base, c, xc, out);
-                else k_prolong<T, 3, false><<<g, b, 0, s>>>(F.mx, F.my, F.mz, C.mx, C.my, kchf(F.dim, F.my, F.mz), base, c, xc, out);
+                if (zg) k_prolong<T, 3, true><<<g, b, 0, s>>>(F.mx, F.my, F.mz, C.mx, C.my, kchf(F.dim, F.mx, F.my, F.mz), base, c, xc, out);
+                else k_prolong<T, 3, false><<<g, b, 0, s>>>(F.mx, F.my, F.mz, C.mx, C.my, kchf(F.dim, F.mx, F.my, F.mz), base, c, xc, out);
             } else if (F.dim == 2) {
-                if (zg) k_prolong<T, 2, true><<<g, b, 0, s>>>(F.mx, F.my, F.mz, C.mx, C.my, kchf(F.dim, F.my, F.mz), base, c, xc, out);
-                else k_prolong<T, 2, false><<<g, b, 0, s>>>(F.mx, F.my, F.mz, C.mx, C.my, kchf(F.dim, F.my, F.mz), base, c, xc, out);
+                if (zg) k_prolong<T, 2, true><<<g, b, 0, s>>>(F.mx, F.my, F.mz, C.mx, C.my, kchf(F.dim, F.mx, F.my, F.mz), base, c, xc, out);
+                else k_prolong<T, 2, false><<<g, b, 0, s>>>(F.mx, F.my, F.mz, C.mx, C.my, kchf(F.dim, F.mx, F.my, F.mz), base, c, xc, out);
             } else {
-                if (zg) k_prolong<T, 1, true><<<g, b, 0, s>>>(F.mx, F.my, F.mz, C.mx, C.my, kchf(F.dim, F.my, F.mz), base, c, xc, out);
-                else k_prolong<T, 1, false><<<g, b, 0, s>>>(F.mx, F.my, F.mz, C.mx, C.my, kchf(F.dim, F.my, F.mz), base, c, xc, out);
+                if (zg) k_prolong<T, 1, true><<<g, b, 0, s>>>(F.mx, F.my, F.mz, C.mx, C.my, kchf(F.dim, F.mx, F.my, F.mz), base, c, xc, out);
+                else k_prolong<T, 1, false><<<g, b, 0, s>>>(F.mx, F.my, F.mz, C.mx, C.my, kchf(F.dim, F.mx, F.my, F.mz), base, c, xc, out);
             }
         });
     }
@@ -2310,7 +2315,7 @@ static int estimate_level(p4g_solver_s* s, int l) {
         ov.ax = L.ax; ov.ay = L.ay; ov.az = L.az; ov.jac = jac ? 1 : 0;
         P4G_TRY(get(&idv));
         k_stencil<double, 3, OpVar<double>, SrcZero<double>, OutIdiag>
-            <<<g, bk, 0, st>>>(L.mx, L.my, L.mz, kchf(L.dim, L.my, L.mz), ov, SrcZero<double>{}, OutIdiag{idv}, s->cx.part);
+            <<<g, bk, 0, st>>>(L.mx, L.my, L.mz, kchf(L.dim, L.mx, L.my, L.mz), ov, SrcZero<double>{}, OutIdiag{idv}, s->cx.part);
         LAUNCH_CHECK();
     }
     const double idc = jac ? 1.0 / L.d : 1.0;
@@ -2358,16 +2363,16 @@ static int estimate_level(p4g_solver_s* s, int l) {
                 og, SrcDir<double>{z, pold, pnew, S + S_BCOEF}, OutApplyDot<double>{w}, s->cx.part);
         else if (L.var)
             k_stencil<double, 3, OpVar<double>, SrcDir<double>, OutApplyDot<double>><<<g, bk, 0, st>>>(
-                L.mx, L.my, L.mz, kchf(L.dim, L.my, L.mz), ov, SrcDir<double>{z, pold, pnew, S + S_BCOEF}, OutApplyDot<double>{w}, s->cx.part);
+                L.mx, L.my, L.mz, kchf(L.dim, L.mx, L.my, L.mz), ov, SrcDir<double>{z, pold, pnew, S + S_BCOEF}, OutApplyDot<double>{w}, s->cx.part);
         else if (L.dim == 3)
             k_stencil<double, 3, OpConst<double>, SrcDir<double>, OutApplyDot<double>><<<g, bk, 0, st>>>(
-                L.mx, L.my, L.mz, kchf(L.dim, L.my, L.mz), oc, SrcDir<double>{z, pold, pnew, S + S_BCOEF}, OutApplyDot<double>{w}, s->cx.part);
+                L.mx, L.my, L.mz, kchf(L.dim, L.mx, L.my, L.mz), oc, SrcDir<double>{z, pold, pnew, S + S_BCOEF}, OutApplyDot<double>{w}, s->cx.part);
         else if (L.dim == 2)
             k_stencil<double, 2, OpConst<double>, SrcDir<double>, OutApplyDot<double>><<<g, bk, 0, st>>>(
-                L.mx, L.my, L.mz, kchf(L.dim, L.my, L.mz), oc, SrcDir<double>{z, pold, pnew, S + S_BCOEF}, OutApplyDot<double>{w}, s->cx.part);
+                L.mx, L.my, L.mz, kchf(L.dim, L.mx, L.my, L.mz), oc, SrcDir<double>{z, pold, pnew, S + S_BCOEF}, OutApplyDot<double>{w}, s->cx.part);
         else
             k_stencil<double, 1, OpConst<double>, SrcDir<double>, OutApplyDot<double>><<<g, bk, 0, st>>>(
-                L.mx, L.my, L.mz, kchf(L.dim, L.my, L.mz), oc, SrcDir<double>{z, pold, pnew, S + S_BCOEF}, OutApplyDot<double>{w}, s->cx.part);
+                L.mx, L.my, L.mz, kchf(L.dim, L.mx, L.my, L.mz), oc, SrcDir<double>{z, pold, pnew, S + S_BCOEF}, OutApplyDot<double>{w}, s->cx.part);
         LAUNCH_CHECK();
         std::swap(pold, pnew);
         k_finalize<<<1, FT, 0, st>>>(nbs, s->cx.part, S, FIN_RAW, 0);
@@ -2896,7 +2901,7 @@ static int fine64(p4g_solver_s* s, Src src, Out out, int cls, double bytes, long
         ov.kc = s->kc64; ov.cx = F.cx; ov.cy = F.cy; ov.cz = F.cz;
         ov.ax = F.ax; ov.ay = F.ay; ov.az = F.az; ov.jac = 0;
         return s->cx.launch(cls, true, bytes, [&] {
-            k_stencil<double, 3, OpVar<double>, Src, Out><<<g, bk, 0, st>>>(F.mx, F.my, F.mz, kchf(F.dim, F.my, F.mz), ov, src, out, part);
+            k_stencil<double, 3, OpVar<double>, Src, Out><<<g, bk, 0, st>>>(F.mx, F.my, F.mz, kchf(F.dim, F.mx, F.my, F.mz), ov, src, out, part);
         });
     }
     OpConst<double> oc;
@@ -2907,16 +2912,16 @@ static int fine64(p4g_solver_s* s, Src src, Out out, int cls, double bytes, long
         if (F.dim == 3 && !F.gal && s->lds != 0 && (F.mx - 1) % W == 0 && (s->lds == 1 || F.mz >= 400))
             return s->cx.launch(cls, true, bytes, [&] {
                 k_stencil_lds<double, OpConst<double>, Src, Out, TY, 1><<<g, bk, 0, st>>>(
-                    F.mx, F.my, F.mz, kchf(F.dim, F.my, F.mz), oc, src, out, part);
+                    F.mx, F.my, F.mz, kchf(F.dim, F.mx, F.my, F.mz), oc, src, out, part);
             });
     }
     return s->cx.launch(cls, true, bytes, [&] {
         if (F.dim == 3)
-            k_stencil<double, 3, OpConst<double>, Src, Out><<<g, bk, 0, st>>>(F.mx, F.my, F.mz, kchf(F.dim, F.my, F.mz), oc, src, out, part);
+            k_stencil<double, 3, OpConst<double>, Src, Out><<<g, bk, 0, st>>>(F.mx, F.my, F.mz, kchf(F.dim, F.mx, F.my, F.mz), oc, src, out, part);
         else if (F.dim == 2)
-            k_stencil<double, 2, OpConst<double>, Src, Out><<<g, bk, 0, st>>>(F.mx, F.my, F.mz, kchf(F.dim, F.my, F.mz), oc, src, out, part);
+            k_stencil<double, 2, OpConst<double>, Src, Out><<<g, bk, 0, st>>>(F.mx, F.my, F.mz, kchf(F.dim, F.mx, F.my, F.mz), oc, src, out, part);
         else
-            k_stencil<double, 1, OpConst<double>, Src, Out><<<g, bk, 0, st>>>(F.mx, F.my, F.mz, kchf(F.dim, F.my, F.mz), oc, src, out, part);
+            k_stencil<double, 1, OpConst<double>, Src, Out><<<g, bk, 0, st>>>(F.mx, F.my, F.mz, kchf(F.dim, F.mx, F.my, F.mz), oc, src, out, part);
     });
 }
 
