@@ -284,7 +284,7 @@ static int ms_solve(p4g_solver_s* s, double q, const double* gb, double* x, p4g_
             s->e64->g27[l] = s->g27[l];
         }
         if (s->sor && s->pctype == PCT_MG) {   // pipelined strip sweeps on every level
-            s->ms_pipes.resize(s->nlev);
+            P4G_TRY(sor_pipes_create(s));
             for (int l = l0; l <= L; ++l) P4G_TRY(sor_pipe_alloc(s, l, SOR_9PT));
         }
         if (s->pctype == PCT_ILU) {
@@ -357,7 +357,6 @@ static int ms_solve(p4g_solver_s* s, double q, const double* gb, double* x, p4g_
     out.fnorm0 = fnorm;
     s->ms_fhist.push_back(fnorm);
     P4G_TRY(monitor(0, fnorm));
-    P4G_TRY(sor_pipes_reset(s));
     int reason = vi_converged(s, 0, 0.0, 0.0, fnorm, ttol, rnorm0);
     int i = 0, iter = 0;
     // the engine's finest operator is the matrix-free product while this
@@ -371,6 +370,7 @@ static int ms_solve(p4g_solver_s* s, double q, const double* gb, double* x, p4g_
         s->e64->mf_op = [s, &R](const double* a, double* y) { return ms_mffd(s, R, R.mfw, a, y); };
     }
     for (; !reason && i < s->snes_maxit; ++i) {
+        P4G_TRY(sor_pipes_begin(s));
         P4G_TRY(ms_operator(s, R, fd));
         if (symcheck) {
             int sym = 0;

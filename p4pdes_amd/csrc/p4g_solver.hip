@@ -2052,7 +2052,7 @@ struct p4g_solver_s {
     size_t asm_cap_idx = 0, asm_cap_inv = 0, asm_cap_row = 0;
     bool tail = true;                 // -p4g_tail 1|0: the coarse end of a V-cycle in one launch
     int post_fuse = -1;               // -p4g_post_fuse auto|1|0: prolongation + first of several post steps
-    bool sor_test_stall = false;      // -p4g_sor_test_stall: every pipelined-SOR wait gives up at once
+    int sor_test_stall = 0;           // -p4g_sor_test_stall 1|once: pipelined-SOR waits give up at once, in the first call only
     bool sor_pipeline = true;         // -p4g_sor_pipeline 1|0: 3D SOR by pipelined strips (else hyperplanes)
     // reduced-space VI Newton (p4g_vi_solve): SNES options and state
     double snes_rtol = 1e-8, snes_atol = 1e-50, snes_stol = 1e-8, snes_divtol = 1e4;
@@ -2062,7 +2062,10 @@ struct p4g_solver_s {
     bool ms_mode = false;                 // set up for p4g_ms_solve
     double* ms_buf = nullptr;             // its vectors
     double* ms_ilu9 = nullptr;            // its box-pattern ILU(0) factor (-pc_type ilu)
-    std::vector<SorPipe> ms_pipes;        // its levels' pipelined SOR flags (-mg_levels_pc_type sor)
+    std::vector<SorPipe> ms_pipes;        // the levels' pipelined SOR sweeps (-mg_levels_pc_type sor)
+    unsigned* sor_ctl = nullptr;          //   their control words (SorPipe::ctl), two a level
+    unsigned* sor_hctl = nullptr;         //   the words as read back (pinned)
+    bool sor_open = false;                //   sweeps have run since the words were last read and found good
     double* ms_band = nullptr;            // the coarse operator in band form, its blocks' inverses
     long ms_band_cap = 0;
     std::vector<double> ms_fhist;         // |F| per Newton iterate
@@ -2098,6 +2101,7 @@ struct p4g_solver_s {
         if (cx.part_rr) hipFree(cx.part_rr);
         if (cx.S) hipFree(cx.S);
         if (cx.hS) hipHostFree(cx.hS);
+        if (sor_hctl) hipHostFree(sor_hctl);
         if (cx.stream) hipStreamDestroy(cx.stream);
     }
 };
@@ -2483,7 +2487,7 @@ static int configure(p4g_solver_s* s) {
             o.geti("mg_levels_pc_sor_lits", 1) != 1)
             return set_error(PETSC_ERR_SUP, "the device SOR smoother has omega 1 and one sweep");
         s->sor_blocks = o.geti("p4g_sor_blocks", 1);
-        s->sor_test_stall = o.getb("p4g_sor_test_stall", false);
+        s->sor_test_stall = o.gets("p4g_sor_test_stall", "") == "once" ? 2 : (o.getb("p4g_sor_test_stall", false) ? 1 : 0);
         s->sor_pipeline = o.getb("p4g_sor_pipeline", true);
         if (s->sor_blocks < 1 || s->sor_blocks > 16)
             return set_error(PETSC_ERR_ARG_OUTOFRANGE, "-p4g_sor_blocks must be in 1..16");
@@ -2729,6 +2733,48 @@ static int sor2_lds() {
                                 (int)Sor2<NINE>::LDS));
     return 0;
 }
+// the pipelined sweeps' records, one a level, and their control words
+static int sor_pipes_create(p4g_solver_s* s) {
+    s->ms_pipes.assign(s->nlev, SorPipe());
+    const size_t bytes = 2 * s->nlev * sizeof(unsigned);
+    P4G_TRY(dalloc(s, (void**)&s->sor_ctl, bytes));
+    HIP_TRY(hipMemset(s->sor_ctl, 0, bytes));
+    if (!s->sor_hctl) HIP_TRY(hipHostMalloc((void**)&s->sor_hctl, bytes, hipHostMallocDefault));
+    s->sor_open = false;
+    return 0;
+}
+// Every call that runs sweeps is bracketed by these two.  A sweep whose wait
+// gives up sets its level's stall word and the rest of the call runs without
+// waiting, so its results are worthless: sor_pipes_check reports it (it reads
+// the words back, all levels in one copy).  After a call that did not get
+// there, or found a stall, sor_pipes_begin clears the stall words and advances
+// the tags, past any that such a call may have left in the handed-over words.
+static int sor_pipes_begin(p4g_solver_s* s) {
+    if (!s->sor_ctl) return 0;
+    const bool stall = s->sor_test_stall != 0;
+    if (s->sor_test_stall == 2) s->sor_test_stall = 0;
+    for (SorPipe& P : s->ms_pipes) {
+        P.spin_limit = stall ? 64 : (1L << 24);
+        P.extra = stall ? 1u << 21 : 0;
+    }
+    if (s->sor_open) {
+        k_sor_reset<<<1, 64, 0, s->cx.stream>>>(s->nlev, s->sor_ctl);
+        LAUNCH_CHECK();
+    }
+    s->sor_open = true;
+    return 0;
+}
+static int sor_pipes_check(p4g_solver_s* s, const char* who) {
+    if (!s->sor_ctl) return 0;
+    HIP_TRY(hipMemcpyAsync(s->sor_hctl, s->sor_ctl, 2 * s->nlev * sizeof(unsigned), hipMemcpyDeviceToHost,
+                           s->cx.stream));
+    HIP_TRY(hipStreamSynchronize(s->cx.stream));
+    for (int l = 0; l < s->nlev; ++l)
+        if (s->sor_hctl[2 * l]) return set_error(PETSC_ERR_LIB, "%s: a pipelined SOR sweep stalled", who);
+    s->sor_open = false;
+    return 0;
+}
+
 static int sor_pipe_alloc(p4g_solver_s* s, int l, SorKind kind) {
     LevelInfo& L = s->lv[l];
     if (L.dim < 2 || L.var || L.mx > (1 << 20) - 256) return 0;      // (a strip is addressed in 32 bits)
@@ -2760,7 +2806,7 @@ static int sor_pipe_alloc(p4g_solver_s* s, int l, SorKind kind) {
     P4G_TRY(zeroed((void**)&P.S, nS * sizeof(T2<double>)));
     P4G_TRY(zeroed((void**)&P.yh, ny * sizeof(u64)));
     if (nz) P4G_TRY(zeroed((void**)&P.zh, nz * sizeof(u64)));
-    P4G_TRY(zeroed((void**)&P.ctl, 2 * sizeof(unsigned)));
+    P.ctl = s->sor_ctl + 2 * l;
     if (nine) {
         P4G_TRY(dalloc(s, (void**)&P.pk, (size_t)P.ns * P.Tp * 256 * sizeof(T2<double>)));
         P4G_TRY(dalloc(s, (void**)&P.inv, nS * sizeof(T2<double>)));
@@ -2775,7 +2821,7 @@ int solver_setup(p4g_solver_s* s) {
     P4G_TRY(build_levels(s));
     sor_splits(s);
     if (s->pctype == PCT_MG && s->sor && !s->lilu && s->sor_pipeline && !s->vi_mode && !s->ms_mode) {
-        s->ms_pipes.resize(s->nlev);   // pipelined SOR sweeps on the smoothing levels
+        P4G_TRY(sor_pipes_create(s));   // pipelined SOR sweeps on the smoothing levels
         for (int l = s->nlev > 1 ? 1 : 0; l < s->nlev; ++l)
             if (s->lv[l].sor_nblk <= 1 && !(s->galerkin && l < s->nlev - 1))
                 P4G_TRY(sor_pipe_alloc(s, l, s->lv[l].dim == 3 ? SOR_7PT : SOR_5PT));
@@ -2824,8 +2870,11 @@ int solver_setup(p4g_solver_s* s) {
             s->n0 = 1;
             s->Ainv.assign(1, 0.0);
         }
-        if (s->smoother == SM_CHEB)
+        if (s->smoother == SM_CHEB) {
+            P4G_TRY(sor_pipes_begin(s));
             for (int l = s->nlev > 1 ? 1 : 0; l < s->nlev; ++l) P4G_TRY(estimate_level(s, l));
+            P4G_TRY(sor_pipes_check(s, "PCSetUp"));
+        }
     }
     auto cfg = [&](auto& e) {
         e->pctype = s->pctype; e->cycles = s->cycles; e->smoother = s->smoother; e->nu = s->nu;
@@ -3245,12 +3294,9 @@ static int ksp_views(p4g_solver_s* s, const double* b, double* x) {
     return 0;
 }
 
-static int sor_pipes_reset(p4g_solver_s* s);
-static int sor_pipes_check(p4g_solver_s* s, const char* who);
-
 int ksp_solve_device(p4g_solver_s* s, const double* b, double* x) {
     P4G_TRY(solver_setup(s));
-    P4G_TRY(sor_pipes_reset(s));
+    P4G_TRY(sor_pipes_begin(s));
     hipStream_t st = s->cx.stream;
     hipEvent_t e0, e1;
     HIP_TRY(hipEventCreate(&e0));
@@ -3511,6 +3557,7 @@ int p4g_pc_apply_device(p4g_Solver s, const double* d_r, double* d_z) {
     clear_error();
     if (!s || !d_r || !d_z) return set_error(PETSC_ERR_ARG_WRONG, "p4g_pc_apply_device: null argument");
     P4G_TRY(solver_setup(s));
+    P4G_TRY(sor_pipes_begin(s));
     if (s->mixed) {
         Engine<float>& e = *s->e32;
         const long n = s->lv.back().n;
@@ -3523,7 +3570,7 @@ int p4g_pc_apply_device(p4g_Solver s, const double* d_r, double* d_z) {
     }
     HIP_TRY(hipStreamSynchronize(s->cx.stream));
     s->cx.tm.collect();
-    return 0;
+    return sor_pipes_check(s, "PCApply");
 }
 
 // ---------------------------------------------- no-allocation PCApply
@@ -3586,6 +3633,7 @@ int p4g_pc_apply_device_noalloc(p4g_Solver s, const double* d_r, double* d_z) {
                          kNoAllocBytes >> 20);
     unsigned char* base = nullptr;
     P4G_TRY(noalloc_scratch(&base));
+    P4G_TRY(sor_pipes_begin(s));
     // swap the carve in, run the cycle, swap the solver's arrays back
     constexpr int kMaxWork = 8 * 32;
     double* saved[kMaxWork];
@@ -3609,6 +3657,7 @@ int p4g_pc_apply_device_noalloc(p4g_Solver s, const double* d_r, double* d_z) {
         const hipError_t h = hipStreamSynchronize(s->cx.stream);
         if (h != hipSuccess) e = set_error(PETSC_ERR_LIB, "p4g_pc_apply_device_noalloc: %s", hipGetErrorString(h));
     }
+    if (!e) e = sor_pipes_check(s, "PCApply");
     size_t q = 0;
     E.each_work([&](double*& p, long) { p = saved[q++]; });
     s->cx.part = part0;
@@ -3765,33 +3814,6 @@ const char* p4g_version(void) { return "p4g 0.1 (gfx950)"; }
 }  // extern "C"
 
 // continuous-batching server (uses the types above)
-namespace p4g {
-// The stall words of the pipelined SOR sweeps: cleared at the
-// start of a solve, read after each linear solve, where the solve has just
-// synchronized its stream, so a stall stops the solve at the Newton step it
-// happened in.
-static int sor_pipes_reset(p4g_solver_s* s) {
-    for (SorPipe& P : s->ms_pipes) {
-        if (!P.ctl) continue;
-        P.spin_limit = s->sor_test_stall ? 64 : (1L << 24);
-        P.extra = s->sor_test_stall ? 1u << 21 : 0;
-        HIP_TRY(hipMemsetAsync(P.ctl, 0, sizeof(unsigned), s->cx.stream));
-    }
-    return 0;
-}
-
-static int sor_pipes_check(p4g_solver_s* s, const char* who) {
-    for (const SorPipe& P : s->ms_pipes) {
-        if (!P.ctl) continue;
-        int e = 0;
-        HIP_TRY(hipMemcpyAsync(&e, P.ctl, sizeof(int), hipMemcpyDeviceToHost, s->cx.stream));
-        HIP_TRY(hipStreamSynchronize(s->cx.stream));
-        if (e) return set_error(PETSC_ERR_LIB, "%s: a pipelined SOR sweep stalled", who);
-    }
-    return 0;
-}
-}  // namespace p4g
-
 #include "p4g_serve_impl.hpp"
 // reduced-space VI Newton (SNESVINEWTONRSLS) over the solver's levels
 #include "p4g_vi_impl.hpp"

@@ -29,7 +29,7 @@
 // Workgroups depend on workgroups of lower index only (the dispatch order).
 // A wait longer than spin_limit polls sets ctl[0] and gives up, and a launch
 // that finds ctl[0] set waits for nothing: every kernel ends, and the host
-// checks ctl[0] after the solve.  `extra` is added to every awaited tag (0;
+// checks ctl[0] after the call (sor_pipes_check).  `extra` is added to every awaited tag (0;
 // the host's stall test awaits a tag that no workgroup writes).
 #pragma once
 
@@ -96,6 +96,16 @@ struct SorCtl {
     long spin_limit;
     unsigned extra;
 };
+
+// the levels' control words after a call that stalled or was cut short: no
+// stall, and tags that such a call has not used (a workgroup that started late
+// in a stalled backward sweep may have tagged its words for the next one)
+__global__ void k_sor_reset(int nlev, unsigned* ctl) {
+    for (int l = threadIdx.x; l < nlev; l += 64) {
+        ctl[2 * l] = 0;
+        ctl[2 * l + 1] += 1;
+    }
+}
 
 __device__ __forceinline__ bool sor_dead(const SorCtl& c) {
     return __hip_atomic_load(c.ctl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;

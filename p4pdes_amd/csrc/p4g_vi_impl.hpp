@@ -490,7 +490,7 @@ static int vi_solve(p4g_solver_s* s, const double* xl, const double* xu, double*
         // the Chebyshev bounds are re-estimated every Newton step: keep their
         // vectors (6 of the finest size) instead of allocating per level
         if (s->sor && s->pctype == PCT_MG && s->lv[L].dim == 2) {   // pipelined strip sweeps on every level
-            s->ms_pipes.resize(s->nlev);
+            P4G_TRY(sor_pipes_create(s));
             for (int l = 0; l <= L; ++l) P4G_TRY(sor_pipe_alloc(s, l, SOR_9PT));
         }
         if (s->pctype == PCT_MG && s->smoother == SM_CHEB) {
@@ -539,7 +539,6 @@ static int vi_solve(p4g_solver_s* s, const double* xl, const double* xu, double*
     std::memset(&out, 0, sizeof out);
     out.fnorm0 = fnorm;
     s->vi_fhist.push_back(fnorm);
-    P4G_TRY(sor_pipes_reset(s));
     // PCASM: the engine's preconditioner while this solve runs
     struct AsmScope {
         Engine<double>* e;
@@ -558,6 +557,7 @@ static int vi_solve(p4g_solver_s* s, const double* xl, const double* xu, double*
     int reason = vi_converged(s, 0, 0.0, 0.0, fnorm, ttol, rnorm0);
     int i = 0, iter = 0;
     for (; !reason && i < s->snes_maxit; ++i) {
+        P4G_TRY(sor_pipes_begin(s));
         const double* rhs = R.Fm;
         if (ssls) {   // the semismooth Jacobian at X; Jss Y = phi
             P4G_TRY(ssls_operator(s, R));

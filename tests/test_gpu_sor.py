@@ -5,6 +5,8 @@ any size (the smoother is the preconditioner): the edges of a strip's 64 rows,
 of the batches of steps and of the plane groups, 35 strips (on two XCDs), 258
 (two launches), single
 interior points, and boxes longer in each direction."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -60,3 +62,78 @@ def test_sor2_stall_stops_the_solve():
     assert "pipelined SOR sweep stalled" in text
     rc, text, _, _ = capi.fish_run(args)
     assert rc == 0, text
+
+
+# grids of several strips, and 3D plane groups; Richardson smoothing, so that set-up runs no sweeps
+STALLS = {"2d": ("-fsh_dim 2 -fsh_problem zero -da_grid_x 40 -da_grid_y 200", 40 * 200),
+          "3d": ("-fsh_dim 3 -fsh_problem zero -da_grid_x 6 -da_grid_y 67 -da_grid_z 18", 6 * 67 * 18)}
+RICH = " -pc_type mg -pc_mg_levels 1 -mg_levels_ksp_type richardson -mg_levels_ksp_max_it 2"
+
+
+def _call(s, entry, b):
+    """(error code, result) of one entry point on device copies of b."""
+    L = capi.lib()
+    d = [L.p4g_device_malloc(b.nbytes) for _ in range(2)]
+    try:
+        capi.check(L.p4g_memcpy_htod(d[0], b.ctypes.data, b.nbytes))
+        if entry == "ksp":
+            rep = capi.Report()
+            rc = L.p4g_ksp_solve_device(s.solver, d[0], d[1], ctypes.byref(rep))
+        else:
+            rc = getattr(L, "p4g_pc_apply_device" + entry)(s.solver, d[0], d[1])
+        x = np.empty_like(b)
+        capi.check(L.p4g_memcpy_dtoh(x.ctypes.data, d[1], b.nbytes))
+        return rc, x
+    finally:
+        for p in d:
+            L.p4g_device_free(p)
+
+
+@pytest.mark.parametrize("entry", ["", "_noalloc", "ksp"])
+@pytest.mark.parametrize("dim", sorted(STALLS))
+def test_stalled_call_is_reported_and_the_next_is_right(dim, entry):
+    # the first call's waits give up at once: it must say so, and leave nothing
+    # behind that a later call on the handle could take for its own
+    args, n = STALLS[dim]
+    b = np.random.default_rng(n).standard_normal(n)
+    print("sor stall", dim, entry, flush=True)
+    with capi.Session(args + RICH + " -p4g_sor_pipeline 0") as s:
+        capi.check(capi.lib().p4g_solver_setup(s.solver))
+        rc, ref = _call(s, entry, b)
+        assert rc == 0
+    with capi.Session(args + RICH + " -p4g_sor_test_stall once") as s:
+        capi.check(capi.lib().p4g_solver_setup(s.solver))
+        rc, _ = _call(s, entry, b)
+        assert rc == 76 and "pipelined SOR sweep stalled" in capi.last_error()
+        for _ in range(2):
+            rc, x = _call(s, entry, b)
+            assert rc == 0
+            assert np.array_equal(x, ref)
+
+
+def test_stall_during_setup_is_reported():
+    # the eigenvalue estimates run sweeps: bounds from a stalled one must not stay
+    L, vp = capi.lib(), ctypes.c_void_p
+    ctx = (ctypes.c_double * 9)(1, 1, 1, 1, 1, 1, 0, 0, 0)      # PoissonCtx: unit lengths and coefficients
+    L.p4g_da_set_jacobian_local.argtypes = [vp, vp, vp]
+
+    def bounds(extra, codes):
+        opts = ("-da_grid_x 11 -da_grid_y 101 -da_refine 1 -pc_type mg" + extra).encode()
+        da, solver, rep = vp(), vp(), capi.Report()
+        capi.check(L.p4g_da_create(2, 3, 3, 1, 1.0, 1.0, 1.0, ctypes.byref(da)))
+        try:
+            capi.check(L.p4g_da_set_from_options(da, opts))
+            capi.check(L.p4g_da_set_jacobian_local(da, ctypes.cast(capi.fishlib().Poisson2DJacobianLocal, vp),
+                                                   ctypes.cast(ctx, vp)))
+            capi.check(L.p4g_solver_create(da, opts, ctypes.byref(solver)))
+            for code in codes:
+                assert L.p4g_solver_setup(solver) == code
+                if code:
+                    assert "PCSetUp: a pipelined SOR sweep stalled" in capi.last_error()
+            capi.check(L.p4g_solver_get_report(solver, ctypes.byref(rep)))
+            return rep.emax_fine
+        finally:
+            L.p4g_solver_destroy(ctypes.byref(solver))
+            L.p4g_da_destroy(ctypes.byref(da))
+
+    assert bounds(" -p4g_sor_test_stall once", [76, 0]) == bounds(" -p4g_sor_pipeline 0", [0]) > 0
