@@ -2052,7 +2052,10 @@ struct p4g_solver_s {
     size_t asm_cap_idx = 0, asm_cap_inv = 0, asm_cap_row = 0;
     bool tail = true;                 // -p4g_tail 1|0: the coarse end of a V-cycle in one launch
     int post_fuse = -1;               // -p4g_post_fuse auto|1|0: prolongation + first of several post steps
-    int sor_test_stall = 0;           // -p4g_sor_test_stall 1|once: pipelined-SOR waits give up at once, in the first call only
+    // -p4g_sor_test_stall 1|once|n: pipelined-SOR waits cannot succeed (once: in the first call), and give up
+    // after 64 (n) polls
+    int sor_test_stall = 0;           // 0 off, 1 on, 2 once
+    long sor_test_polls = 64;
     bool sor_pipeline = true;         // -p4g_sor_pipeline 1|0: 3D SOR by pipelined strips (else hyperplanes)
     // reduced-space VI Newton (p4g_vi_solve): SNES options and state
     double snes_rtol = 1e-8, snes_atol = 1e-50, snes_stol = 1e-8, snes_divtol = 1e4;
@@ -2487,7 +2490,12 @@ static int configure(p4g_solver_s* s) {
             o.geti("mg_levels_pc_sor_lits", 1) != 1)
             return set_error(PETSC_ERR_SUP, "the device SOR smoother has omega 1 and one sweep");
         s->sor_blocks = o.geti("p4g_sor_blocks", 1);
-        s->sor_test_stall = o.gets("p4g_sor_test_stall", "") == "once" ? 2 : (o.getb("p4g_sor_test_stall", false) ? 1 : 0);
+        const std::string stall = o.gets("p4g_sor_test_stall", "0");
+        if (stall == "once") s->sor_test_stall = 2;
+        else if (std::atol(stall.c_str()) > 1) {
+            s->sor_test_stall = 1;
+            s->sor_test_polls = std::min(std::atol(stall.c_str()), 1L << 24);
+        } else s->sor_test_stall = o.getb("p4g_sor_test_stall", false) ? 1 : 0;
         s->sor_pipeline = o.getb("p4g_sor_pipeline", true);
         if (s->sor_blocks < 1 || s->sor_blocks > 16)
             return set_error(PETSC_ERR_ARG_OUTOFRANGE, "-p4g_sor_blocks must be in 1..16");
@@ -2754,7 +2762,7 @@ static int sor_pipes_begin(p4g_solver_s* s) {
     const bool stall = s->sor_test_stall != 0;
     if (s->sor_test_stall == 2) s->sor_test_stall = 0;
     for (SorPipe& P : s->ms_pipes) {
-        P.spin_limit = stall ? 64 : (1L << 24);
+        P.spin_limit = stall ? s->sor_test_polls : (1L << 24);
         P.extra = stall ? 1u << 21 : 0;
     }
     if (s->sor_open) {

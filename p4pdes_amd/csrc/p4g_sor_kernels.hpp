@@ -261,12 +261,17 @@ __global__ void __launch_bounds__(Sor2<NINE>::NT) k_sor2(Sor2Args A) {
     }
     if (threadIdx.x < 64) done[threadIdx.x] = 0;
     __syncthreads();
-    // waits inside the workgroup end with it: of the waves only wave 1 waits
-    // for another workgroup, and that is bounded (so are these)
+    // Waits inside the workgroup end with it.  Only wave 1 polls another
+    // workgroup, and its limit is the one that counts: when it gives up it
+    // releases the chain (W_Y), and the chain the rest.  These waits, the
+    // chain's for W_Y among them, have a limit only so that no mistake can
+    // make them endless: 64 polls of LDS (63 ns each) for each of wave
+    // 1's polls through L2 (0.35 us), so wave 1 always comes first.
+    const long inner_limit = (A.c.spin_limit << 6) + (1L << 16);
     auto inner_wait = [&](auto ready) __attribute__((always_inline)) {
         long spins = 0;
         while (!dead && !ready()) {
-            if (++spins > (1L << 24)) {
+            if (++spins > inner_limit) {
                 if (r == 0) atomicExch(A.c.ctl, 1u);
                 dead = true;
                 __builtin_amdgcn_s_waitcnt(0);      // so that the other path's waits stay as they are

@@ -6,6 +6,7 @@ of the batches of steps and of the plane groups, 35 strips (on two XCDs), 258
 (two launches), single
 interior points, and boxes longer in each direction."""
 import ctypes
+import time
 
 import numpy as np
 import pytest
@@ -137,3 +138,19 @@ def test_stall_during_setup_is_reported():
             L.p4g_da_destroy(ctypes.byref(da))
 
     assert bounds(" -p4g_sor_test_stall once", [76, 0]) == bounds(" -p4g_sor_pipeline 0", [0]) > 0
+
+
+@pytest.mark.parametrize("polls", [1 << 12, 1 << 22])
+def test_late_neighbour_is_awaited_to_the_limit(polls):
+    # a strip that waits for the one before it polls through L2, 0.35 us each
+    # (0.3 allowed for); the chain of steps, which waits in LDS, must not give
+    # up for it first.  1.5 s at the larger limit, a quarter of the real one
+    args, n = STALLS["2d"]
+    print("sor late neighbour", polls, flush=True)
+    with capi.Session(args + RICH + " -p4g_sor_test_stall %d" % polls) as s:
+        b = np.ones(n)
+        t = time.perf_counter()
+        rc, _ = _call(s, "", b)
+        t = time.perf_counter() - t
+    assert rc == 76 and "pipelined SOR sweep stalled" in capi.last_error()
+    assert t >= 0.3e-6 * polls
