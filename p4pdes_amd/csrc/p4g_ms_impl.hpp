@@ -283,7 +283,7 @@ static int ms_solve(p4g_solver_s* s, double q, const double* gb, double* x, p4g_
             s->lv[l].gal = true;
             s->e64->g27[l] = s->g27[l];
         }
-        if (s->sor && s->pctype == PCT_MG) {   // pipelined strip sweeps on every level
+        if (s->sor && s->sor_pipeline && s->pctype == PCT_MG) {   // pipelined sweeps on every level
             P4G_TRY(sor_pipes_create(s));
             for (int l = l0; l <= L; ++l) P4G_TRY(sor_pipe_alloc(s, l, SOR_9PT));
         }

@@ -2056,7 +2056,7 @@ struct p4g_solver_s {
     // after 64 (n) polls
     int sor_test_stall = 0;           // 0 off, 1 on, 2 once
     long sor_test_polls = 64;
-    bool sor_pipeline = true;         // -p4g_sor_pipeline 1|0: 3D SOR by pipelined strips (else hyperplanes)
+    bool sor_pipeline = true;         // -p4g_sor_pipeline 1|0: SOR by pipelined strips (else hyperplanes)
     // reduced-space VI Newton (p4g_vi_solve): SNES options and state
     double snes_rtol = 1e-8, snes_atol = 1e-50, snes_stol = 1e-8, snes_divtol = 1e4;
     int snes_maxit = 50;

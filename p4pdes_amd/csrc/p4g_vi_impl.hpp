@@ -489,7 +489,7 @@ static int vi_solve(p4g_solver_s* s, const double* xl, const double* xu, double*
         P4G_TRY(dalloc(s, (void**)&s->vi_g27, 27 * n * sizeof(double)));
         // the Chebyshev bounds are re-estimated every Newton step: keep their
         // vectors (6 of the finest size) instead of allocating per level
-        if (s->sor && s->pctype == PCT_MG && s->lv[L].dim == 2) {   // pipelined strip sweeps on every level
+        if (s->sor && s->sor_pipeline && s->pctype == PCT_MG && s->lv[L].dim == 2) {   // pipelined sweeps on every level
             P4G_TRY(sor_pipes_create(s));
             for (int l = 0; l <= L; ++l) P4G_TRY(sor_pipe_alloc(s, l, SOR_9PT));
         }

@@ -1,6 +1,7 @@
 """Pipelined SOR sweeps (k_sor2, k_sor7) against the hyperplane sweeps
 (k_sor_plane): every point is updated from the same values in the same order,
-so one preconditioner application agrees bit for bit.  One-level grids take
+so one preconditioner application agrees bit for bit, and with it a whole
+Newton solve whose levels have 9-point operators.  One-level grids take
 any size (the smoother is the preconditioner): the edges of a strip's 64 rows,
 of the batches of steps and of the plane groups, 35 strips (on two XCDs), 258
 (two launches), single
@@ -52,6 +53,41 @@ def test_sor7_matches_hyperplanes(grid):
 
 def test_sor2_multigrid_matches_hyperplanes():
     _pair("-fsh_dim 2 -fsh_problem zero -da_refine 8 -pc_type mg -pc_mg_cycle_type w", 513 * 513, 5)
+
+
+# 9-point levels: one strip and less, edges of strips and of batches of steps, 35 strips (on two XCDs), 258 (two launches)
+GRIDS_9PT = [(3, 3), (5, 4), (35, 5), (67, 65), (130, 67), (97, 200), (19, 2200), (5, 16500)]
+
+
+def _newton_pair(run, args, mg):
+    print("sor9 pair", args, mg, flush=True)
+    out = []
+    for extra in (" -p4g_sor_pipeline 0", ""):
+        rc, text, res, u = run(args + " -pc_type mg -pc_mg_levels %d" % mg + extra, want_u=True)
+        assert rc == 0, text
+        out.append((res.its, res.ksp_its_total, res.reason, res.fnorm, u))
+    assert out[0][1] > 0                   # the preconditioner was applied
+    assert np.isfinite(out[0][4]).all()
+    assert out[0][:4] == out[1][:4]
+    assert np.array_equal(out[0][4], out[1][4])
+
+
+@pytest.mark.parametrize("grid", GRIDS_9PT, ids=lambda g: "x".join(map(str, g)))
+def test_sor9_matches_hyperplanes(grid):
+    # one level (the smoother is the preconditioner): the obstacle problem's
+    # reduced operator, two Newton steps of loosely solved systems
+    _newton_pair(capi.obstacle_run, "-da_grid_x %d -da_grid_y %d -ksp_rtol 0.3 -snes_max_it 2" % grid, 1)
+
+
+@pytest.mark.parametrize("grid", [(5, 4), (35, 5), (67, 65), (66, 130)], ids=lambda g: "x".join(map(str, g)))
+def test_sor9_nonsymmetric_matches_hyperplanes(grid):
+    # the minimal surface's finite-difference Jacobian
+    _newton_pair(capi.minimal_run, "-da_grid_x %d -da_grid_y %d -snes_fd_color -ksp_rtol 0.3 -snes_max_it 2" % grid, 1)
+
+
+def test_sor9_multigrid_matches_hyperplanes():
+    _newton_pair(capi.obstacle_run, "-da_grid_x 10 -da_grid_y 12 -da_refine 4", 5)
+    _newton_pair(capi.minimal_run, "-da_grid_x 9 -da_grid_y 10 -da_refine 3 -snes_fd_color", 4)
 
 
 def test_sor2_stall_stops_the_solve():
