@@ -598,7 +598,7 @@ struct Engine {
                 // a cycle's zero-guess step is then formed where it is read
                 // (mcycle): 257^3, the step's own pass 148 and the residual's
                 // 187 us before, one pass of 245 us now
-                if (pctype == PCT_MG && l > 0 && nu == 1 && L.dim == 3) {
+                if (pctype == PCT_MG && l > 0 && nu == 1 && L.dim == 3 && !sor) {
                     P4G_TRY(alloc(&d.idg, L.n));
                     OpVar<T> o = opv(l, jacobi != 0);
                     k_stencil<T, 3, OpVar<T>, SrcZero<T>, OutRecipDiag<T>>
@@ -1002,7 +1002,9 @@ struct Engine {
                 P4G_TRY(e);
                 rr = r;
             }
-            SorPipe* const P3 = sor_pipe_of(L) && L.pipe->kind == SOR_7PT && !lilu ? L.pipe : nullptr;
+            SorPipe* P3 = nullptr;      // 3D pipelined sweeps: in FP64, like every SOR solve
+            if constexpr (std::is_same<T, double>::value)
+                if (!lilu && sor_pipe_of(L) && L.pipe->kind == SOR_7PT) P3 = L.pipe;
             if (lilu) P4G_TRY(ilu_run<T>(L, ilu_u.size() > (size_t)l ? ilu_u[l] : nullptr, rr, z, st));
             else if (!P3) P4G_TRY(sor_run<T>(L, g27.size() > (size_t)l ? g27[l] : nullptr, rr, z, st));
             T* dst = out;
@@ -1310,7 +1312,7 @@ struct Engine {
                 P4G_TRY(stencil(l, SrcArr<T>{b}, OR{T(s * idg), OutResid<T, 0>{b, d.r}}, P4G_K_RESID_ZG, 2, nullptr,
                                 jac));
             }
-        } else if (xzero && nu == 1 && d.idg && fuse_post) {   // variable diagonal: u = s D^-1 b formed on the fly
+        } else if (xzero && nu == 1 && d.idg && fuse_post && !sor) {   // variable diagonal: u = s D^-1 b formed on the fly
             zgf = true;
             P4G_TRY(stencil(l, SrcMul<T>{b, d.idg, T(s)}, OutResid<T, 0>{b, d.r}, P4G_K_RESID_ZG, 3, nullptr, jac));
         } else {
