@@ -158,7 +158,8 @@ int p4g_da_destroy(p4g_DA *da);
  *   -p4g_tail 1|0 (default 1): the coarse levels of a V-cycle (65^2 or 17^3
  *       points and below, constant coefficients, Jacobi) in one launch,
  *   -p4g_sor_pipeline 1|0 (default 1): SOR levels swept by pipelined
- *       strips, one launch per direction (else one per hyperplane).
+ *       strips, one launch per direction (else, and on levels whose sweep
+ *       arrays do not fit the device's memory, one per hyperplane).
  * Options and combinations the device path does not implement are rejected
  * with PETSC_ERR_SUP and a message naming them, never silently replaced:
  * e.g. -pc_type lu|sor, -pc_type asm outside p4g_vi_solve, -pc_mg_type

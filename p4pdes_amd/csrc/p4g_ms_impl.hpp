@@ -283,10 +283,6 @@ static int ms_solve(p4g_solver_s* s, double q, const double* gb, double* x, p4g_
             s->lv[l].gal = true;
             s->e64->g27[l] = s->g27[l];
         }
-        if (s->sor && s->sor_pipeline && s->pctype == PCT_MG) {   // pipelined sweeps on every level
-            P4G_TRY(sor_pipes_create(s));
-            for (int l = l0; l <= L; ++l) P4G_TRY(sor_pipe_alloc(s, l, SOR_9PT));
-        }
         if (s->pctype == PCT_ILU) {
             P4G_TRY(dalloc(s, (void**)&s->ms_ilu9, 9 * n * sizeof(double)));
             s->e64->ilu9 = s->ms_ilu9;
@@ -294,6 +290,11 @@ static int ms_solve(p4g_solver_s* s, double q, const double* gb, double* x, p4g_
         if (s->pctype == PCT_MG && s->smoother == SM_CHEB) {
             s->est_cap = 6 * n;
             P4G_TRY(dalloc(s, (void**)&s->est_scratch, s->est_cap * sizeof(double)));
+        }
+        if (s->sor && s->sor_pipeline && s->pctype == PCT_MG) {   // pipelined sweeps on every level
+            P4G_TRY(sor_pipes_create(s));
+            const size_t rest = (gmres ? s->gmres_restart + 1 : 0) * n * sizeof(double);   // (besides them: its basis)
+            for (int l = l0; l <= L; ++l) P4G_TRY(sor_pipe_alloc(s, l, SOR_9PT, rest));
         }
     }
     {

@@ -82,6 +82,17 @@ static double now_ms() {
     return duration<double, std::milli>(steady_clock::now().time_since_epoch()).count();
 }
 
+// Whether `bytes` fit the device's free memory beside the `rest` that a solver
+// still takes: arrays that only make a solver faster give way to those it
+// cannot do without.  free_mb >= 0: the free memory, in MB, to assume
+// (-p4g_test_free_mb).
+static bool device_room(size_t bytes, size_t rest, long free_mb) {
+    size_t avail = 0, total = 0;
+    if (free_mb >= 0) avail = (size_t)free_mb << 20;
+    else if (hipMemGetInfo(&avail, &total) != hipSuccess) return true;
+    return avail >= bytes + rest;
+}
+
 // precision-independent description of one multigrid level
 // a level's pipelined SOR sweeps (k_sor2, k_sor7): their working arrays
 enum SorKind { SOR_5PT, SOR_9PT, SOR_7PT };
@@ -484,6 +495,8 @@ struct Engine {
     // steps the prolonged iterate would have to be stored for the Chebyshev
     // recurrence, and the fused kernel then loses to the separate passes)
     bool fuse_post = true;
+    size_t room_rest = 0;      // what the solver takes after this engine's set-up
+    long room_free_mb = -1;    // device_room's free_mb
     bool tail_mode = true;     // -p4g_tail 1|0: the coarse end of a V-cycle in one launch (k_vtail)
     bool tail_ready = false;   // its dynamic LDS size set
     // CG updates fused into stencil passes: the residual update into the
@@ -508,7 +521,7 @@ struct Engine {
     struct Dev {
         T *x = nullptr, *b = nullptr, *r = nullptr, *t[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
         T* kc = nullptr;
-        T* idg = nullptr;   // variable coefficients, V(1,1): the reciprocal diagonal
+        T* idg = nullptr;   // variable coefficients, V(1,1): the reciprocal diagonal (null: no room for it)
     };
     std::vector<Dev> dv;
     double* Ainv = nullptr;   // dense inverse of the coarsest operator
@@ -595,17 +608,6 @@ struct Engine {
                 P4G_TRY(alloc(&d.kc, ncell));
                 std::vector<T> tmp(L.kcell.begin(), L.kcell.end());
                 HIP_TRY(hipMemcpy(d.kc, tmp.data(), ncell * sizeof(T), hipMemcpyHostToDevice));
-                // a cycle's zero-guess step is then formed where it is read
-                // (mcycle): 257^3, the step's own pass 148 and the residual's
-                // 187 us before, one pass of 245 us now
-                if (pctype == PCT_MG && l > 0 && nu == 1 && L.dim == 3 && !sor) {
-                    P4G_TRY(alloc(&d.idg, L.n));
-                    OpVar<T> o = opv(l, jacobi != 0);
-                    k_stencil<T, 3, OpVar<T>, SrcZero<T>, OutRecipDiag<T>>
-                        <<<stencil_grid<T>(3, L.mx, L.my, L.mz), stencil_block(3), 0, cx->stream>>>(
-                            L.mx, L.my, L.mz, kchf(3, L.mx, L.my, L.mz), o, SrcZero<T>{}, OutRecipDiag<T>{d.idg}, cx->part);
-                    LAUNCH_CHECK();
-                }
             }
         }
         P4G_TRY(alloc(&r, F.n));
@@ -626,6 +628,22 @@ struct Engine {
             HIP_TRY(hipMemcpy(Ainv, Ainv_host.data(), Ainv_host.size() * sizeof(double),
                               hipMemcpyHostToDevice));
         }
+        // variable coefficients, V(1,1): with the reciprocal diagonal kept, a
+        // cycle's zero-guess step is formed where it is read (mcycle): 257^3,
+        // the step's own pass 148 and the residual's 187 us before, one pass
+        // of 245 us now
+        if (pctype == PCT_MG && nu == 1 && !sor)
+            for (int l = 1; l < nlev; ++l) {
+                const LevelInfo& L = (*lv)[l];
+                if (!L.var || !device_room(L.n * sizeof(T), room_rest, room_free_mb)) continue;
+                P4G_TRY(alloc(&dv[l].idg, L.n));
+                OpVar<T> o = opv(l, jacobi != 0);
+                k_stencil<T, 3, OpVar<T>, SrcZero<T>, OutRecipDiag<T>>
+                    <<<stencil_grid<T>(3, L.mx, L.my, L.mz), stencil_block(3), 0, cx->stream>>>(
+                        L.mx, L.my, L.mz, kchf(3, L.mx, L.my, L.mz), o, SrcZero<T>{}, OutRecipDiag<T>{dv[l].idg},
+                        cx->part);
+                LAUNCH_CHECK();
+            }
         return 0;
     }
 
@@ -2052,6 +2070,7 @@ struct p4g_solver_s {
     long* asm_row = nullptr;          // per owned row: [inverse row offset, index offset, count, vertex]
     long asm_nrows = 0;
     size_t asm_cap_idx = 0, asm_cap_inv = 0, asm_cap_row = 0;
+    long test_free_mb = -1;           // -p4g_test_free_mb: device memory that optional arrays take as free
     bool tail = true;                 // -p4g_tail 1|0: the coarse end of a V-cycle in one launch
     int post_fuse = -1;               // -p4g_post_fuse auto|1|0: prolongation + first of several post steps
     // -p4g_sor_test_stall 1|once|n: pipelined-SOR waits cannot succeed (once: in the first call), and give up
@@ -2111,6 +2130,16 @@ struct p4g_solver_s {
     }
 };
 
+// deferred iterate updates of the FP64 CG of KSP solves (not of the Newton
+// solves of p4g_vi_solve / p4g_ms_solve); by default as many as 16 GiB of FP64
+// directions hold, at most 15; none below 3, where the folds move as much as
+// the per-iteration updates
+static inline int cg_defer(const p4g_solver_s* s, long n) {
+    if (s->vi_mode || s->ms_mode) return 0;
+    if (s->x_defer >= 0) return s->x_defer;
+    const int d = (int)std::min<long>(kFoldMax - 1, (16L << 30) / std::max(1L, n * (long)sizeof(double)));
+    return d < 3 ? 0 : d;
+}
 // deferred FP64 iterate updates of the mixed-precision PCG (-p4g_x_defer, default 6)
 static inline int mixed_defer(const p4g_solver_s* s) { return s->x_defer < 0 ? 6 : s->x_defer; }
 
@@ -2552,6 +2581,7 @@ static int configure(p4g_solver_s* s) {
         if (s->rr_planes < 0 || s->rr_planes > 64)
             return set_error(PETSC_ERR_ARG_OUTOFRANGE, "-p4g_rr_planes must be in 0..64");
         s->tail = o.getb("p4g_tail", true);
+        s->test_free_mb = o.geti("p4g_test_free_mb", -1);
         P4G_TRY(tri(o.gets("p4g_post_fuse", "auto"), "p4g_post_fuse", s->post_fuse));
         const std::string both = o.gets("p4g_fuse_cg", "auto");
         P4G_TRY(tri(both, "p4g_fuse_cg", s->fuse_r));
@@ -2745,6 +2775,7 @@ static int sor2_lds() {
 }
 // the pipelined sweeps' records, one a level, and their control words
 static int sor_pipes_create(p4g_solver_s* s) {
+    if (s->sor_ctl) return 0;      // a set-up tried again
     s->ms_pipes.assign(s->nlev, SorPipe());
     const size_t bytes = 2 * s->nlev * sizeof(unsigned);
     P4G_TRY(dalloc(s, (void**)&s->sor_ctl, bytes));
@@ -2785,12 +2816,18 @@ static int sor_pipes_check(p4g_solver_s* s, const char* who) {
     return 0;
 }
 
-static int sor_pipe_alloc(p4g_solver_s* s, int l, SorKind kind) {
+// level l's sweep arrays; none (hyperplane sweeps) where they leave less than
+// `rest` bytes of device memory
+static int sor_pipe_alloc(p4g_solver_s* s, int l, SorKind kind, size_t rest) {
     LevelInfo& L = s->lv[l];
     if (L.dim < 2 || L.var || L.mx > (1 << 20) - 256) return 0;      // (a strip is addressed in 32 bits)
     const bool nine = kind == SOR_9PT;
     if (!nine && (L.mx < 3 || L.my < 3 || (L.dim == 3 && L.mz < 3))) return 0;
     SorPipe& P = s->ms_pipes[l];
+    if (P.S) {                     // a set-up tried again
+        L.pipe = &P;
+        return 0;
+    }
     P.kind = kind;
     P.ng = 1;
     size_t nS, ny, nz = 0;
@@ -2808,19 +2845,22 @@ static int sor_pipe_alloc(p4g_solver_s* s, int l, SorKind kind) {
         nS = (size_t)P.ns * (P.Tp / 2) * 64;
         ny = (size_t)P.ns * (nine ? Sor2<true>::slots(P.Tp) : Sor2<false>::slots(P.Tp)) * 2;
     }
+    const size_t npk = nine ? (size_t)P.ns * P.Tp * 256 : 0;
+    if (!device_room((nS + npk + (nine ? nS : 0)) * sizeof(T2<double>) + (ny + nz) * sizeof(u64), rest, s->test_free_mb))
+        return 0;
     auto zeroed = [&](void** p, size_t bytes) -> int {
         P4G_TRY(dalloc(s, p, bytes));
         HIP_TRY(hipMemset(*p, 0, bytes));
         return 0;
     };
-    P4G_TRY(zeroed((void**)&P.S, nS * sizeof(T2<double>)));
-    P4G_TRY(zeroed((void**)&P.yh, ny * sizeof(u64)));
-    if (nz) P4G_TRY(zeroed((void**)&P.zh, nz * sizeof(u64)));
-    P.ctl = s->sor_ctl + 2 * l;
     if (nine) {
-        P4G_TRY(dalloc(s, (void**)&P.pk, (size_t)P.ns * P.Tp * 256 * sizeof(T2<double>)));
+        P4G_TRY(dalloc(s, (void**)&P.pk, npk * sizeof(T2<double>)));
         P4G_TRY(dalloc(s, (void**)&P.inv, nS * sizeof(T2<double>)));
     }
+    P4G_TRY(zeroed((void**)&P.yh, ny * sizeof(u64)));
+    if (nz) P4G_TRY(zeroed((void**)&P.zh, nz * sizeof(u64)));
+    P4G_TRY(zeroed((void**)&P.S, nS * sizeof(T2<double>)));
+    P.ctl = s->sor_ctl + 2 * l;
     L.pipe = &P;
     return 0;
 }
@@ -2832,9 +2872,13 @@ int solver_setup(p4g_solver_s* s) {
     sor_splits(s);
     if (s->pctype == PCT_MG && s->sor && !s->lilu && s->sor_pipeline && !s->vi_mode && !s->ms_mode) {
         P4G_TRY(sor_pipes_create(s));   // pipelined SOR sweeps on the smoothing levels
+        // what the solver takes besides, in fine vectors: the levels' 8, the
+        // Krylov solver's 7 and the caller's 2, deferred updates, GMRES's basis
+        const long n = s->lv.back().n;
+        const size_t rest = (17 + cg_defer(s, n) + (s->ksp_gmres ? s->gmres_restart + 1 : 0)) * n * sizeof(double);
         for (int l = s->nlev > 1 ? 1 : 0; l < s->nlev; ++l)
             if (s->lv[l].sor_nblk <= 1 && !(s->galerkin && l < s->nlev - 1))
-                P4G_TRY(sor_pipe_alloc(s, l, s->lv[l].dim == 3 ? SOR_7PT : SOR_5PT));
+                P4G_TRY(sor_pipe_alloc(s, l, s->lv[l].dim == 3 ? SOR_7PT : SOR_5PT, rest));
     }
     // ILU(0) pivots: the finest level for -pc_type ilu, the smoothing levels
     // for -mg_levels_pc_type ilu (computed once on the host, in the factor's
@@ -2906,6 +2950,9 @@ int solver_setup(p4g_solver_s* s) {
         e->rr_planes = s->rr_planes;
         e->post2_mode = s->post_fuse;
         e->tail_mode = s->tail;
+        // the device copies of p4g_ksp_solve's arrays; mixed: the FP64 outer vectors too; GMRES's basis
+        e->room_free_mb = s->test_free_mb;
+        e->room_rest = F.n * (s->mixed ? 40 + 4 * mixed_defer(s) : 16 + 8 * (s->ksp_gmres ? s->gmres_restart + 1 : 0));
     };
     if (F.var) {
         const size_t nc = F.kcell.size();
@@ -2930,13 +2977,7 @@ int solver_setup(p4g_solver_s* s) {
         cfg(s->e64);
         fuse_rules(s, s->e64.get(), F.n * sizeof(double));
         if (s->vi_mode) s->e64->fuse_r = s->e64->fuse_dir = false;
-        // KSP solves (not the Newton solves of p4g_vi_solve / p4g_ms_solve)
-        // (default: as many as 16 GiB of FP64 directions hold, at most 15;
-        // none below 3, where the folds move as much as the per-iteration updates)
-        const long dbytes = F.n * (long)sizeof(double);
-        int dauto = (int)std::min<long>(kFoldMax - 1, (16L << 30) / std::max(1L, dbytes));
-        if (dauto < 3) dauto = 0;
-        s->e64->x_defer = s->vi_mode || s->ms_mode ? 0 : (s->x_defer < 0 ? dauto : s->x_defer);
+        s->e64->x_defer = cg_defer(s, F.n);
         P4G_TRY(s->e64->setup(&s->cx, &s->lv, s->Ainv, s->n0));
     }
     HIP_TRY(hipStreamSynchronize(s->cx.stream));

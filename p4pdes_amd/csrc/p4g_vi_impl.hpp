@@ -489,13 +489,15 @@ static int vi_solve(p4g_solver_s* s, const double* xl, const double* xu, double*
         P4G_TRY(dalloc(s, (void**)&s->vi_g27, 27 * n * sizeof(double)));
         // the Chebyshev bounds are re-estimated every Newton step: keep their
         // vectors (6 of the finest size) instead of allocating per level
-        if (s->sor && s->sor_pipeline && s->pctype == PCT_MG && s->lv[L].dim == 2) {   // pipelined sweeps on every level
-            P4G_TRY(sor_pipes_create(s));
-            for (int l = 0; l <= L; ++l) P4G_TRY(sor_pipe_alloc(s, l, SOR_9PT));
-        }
         if (s->pctype == PCT_MG && s->smoother == SM_CHEB) {
             s->est_cap = 6 * n;
             P4G_TRY(dalloc(s, (void**)&s->est_scratch, s->est_cap * sizeof(double)));
+        }
+        if (s->sor && s->sor_pipeline && s->pctype == PCT_MG && s->lv[L].dim == 2) {   // pipelined sweeps on every level
+            P4G_TRY(sor_pipes_create(s));
+            // (besides them: the coarse operators, GMRES's basis)
+            const size_t rest = (9 + (s->ksp_gmres ? s->gmres_restart + 1 : 0)) * n * sizeof(double);
+            for (int l = 0; l <= L; ++l) P4G_TRY(sor_pipe_alloc(s, l, SOR_9PT, rest));
         }
     }
     double* b = s->vi_buf;
