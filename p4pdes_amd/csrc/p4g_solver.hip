@@ -2832,7 +2832,7 @@ static int sor_pipe_alloc(p4g_solver_s* s, int l, SorKind kind, size_t rest) {
     P.ng = 1;
     size_t nS, ny, nz = 0;
     if (kind == SOR_7PT) {
-        P.Tp = Sor7::steps(L.mx);
+        P.Tp = Sor7::steps(L.mx, L.my);
         P.ns = Sor7::strips(L.my);
         P.ng = Sor7::groups(L.mz);
         nS = (size_t)P.ns * P.ng * P.Tp * (Sor7::K / 2) * 64;

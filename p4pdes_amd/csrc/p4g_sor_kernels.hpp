@@ -651,8 +651,12 @@ constexpr int kSor7Planes = 4;
 
 struct Sor7 {
     static constexpr int K = kSor7Planes, SB = 4, D = 4;
-    __host__ __device__ static int steps(int mx) {
-        const int need = mx - 2 + 63 + K - 1;
+    // steps of a strip, in whole tiles of the pack kernels: its columns, and
+    // the lag of the last row and plane.  A single strip's last row may come
+    // before lane 63 (a 5^3 level took 128 steps for 8, now 64: an application
+    // 349 -> 242 us, 306 with the flagged strips that these sweeps replaced)
+    __host__ __device__ static int steps(int mx, int my) {
+        const int need = mx - 2 + (strips(my) > 1 ? 63 : my - 3) + K - 1;
         static_assert(64 % (SB * D) == 0, "whole tiles of the pack kernels, whole rounds of the ring");
         return (need + 63) / 64 * 64;
     }
@@ -684,7 +688,7 @@ __global__ void __launch_bounds__(64) k_sor7(Sor7Args A) {
     const int s = BWD ? ns - 1 - os : os, g = BWD ? ng - 1 - og : og, rho = BWD ? 63 - r : r;
     const int Tp = A.Tp, ncol = A.mx - 2;
     const bool rl = 64 * s + rho < A.my - 2;
-    const int sh = BWD ? Tp - (ncol + 63 + K - 1) : 0;
+    const int sh = BWD ? Tp - (ncol + 63 + K - 1) : 0;    // (below zero where a single strip's lanes start late)
     const int off = sh + r;                               // plane 0's column is t - off
     const __amdgpu_buffer_rsrc_t Sr = buffer_of(A.S + ((long)(g * ns + s) * Tp) * (K / 2) * 64, Tp * (K / 2) * 1024u);
     const unsigned v16 = rho * 16u, v8 = r * 8u;

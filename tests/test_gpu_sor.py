@@ -4,8 +4,8 @@ so one preconditioner application agrees bit for bit, and with it a whole
 Newton solve whose levels have 9-point operators.  One-level grids take
 any size (the smoother is the preconditioner): the edges of a strip's 64 rows,
 of the batches of steps and of the plane groups, 35 strips (on two XCDs), 258
-(two launches), single
-interior points, and boxes longer in each direction."""
+(two launches), single interior points, 3D strips whose steps just fill 64 or
+128 or go one past, and boxes longer in each direction."""
 import ctypes
 import time
 
@@ -17,7 +17,8 @@ from p4pdes_amd import capi
 pytestmark = pytest.mark.gpu
 
 GRIDS_2D = [(19, 2200), (5, 16500), (3, 3), (4, 3), (3, 70), (35, 5), (66, 66), (67, 65), (34, 131), (130, 67), (260, 130), (97, 200)]
-GRIDS_3D = [(3, 3, 3), (4, 5, 6), (66, 5, 3), (5, 66, 7), (6, 67, 8), (7, 4, 70), (33, 34, 35), (67, 130, 9), (65, 65, 65)]
+GRIDS_3D = [(3, 3, 3), (4, 5, 6), (66, 5, 3), (5, 66, 7), (6, 67, 8), (7, 4, 70), (33, 34, 35), (67, 130, 9), (65, 65, 65),
+            (33, 33, 9), (34, 33, 9), (3, 63, 5), (3, 64, 5), (3, 66, 5), (3, 67, 5), (98, 32, 11)]
 
 
 def _apply(args, b):
