@@ -3631,8 +3631,10 @@ int p4g_pc_apply_device(p4g_Solver s, const double* d_r, double* d_z) {
 // once per device with hipGetSymbolAddress) until the process ends; calls on
 // one GPU share it and overlapping calls race.  The cycle writes every work
 // element before it reads it, so nothing in it is cleared between calls.
-constexpr size_t kNoAllocBytes = size_t(128) << 20;
-static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
+// Block partial sums have their own room behind the vectors, so that the
+// passes' block counts do not decide which hierarchies fit.
+constexpr size_t kNoAllocBytes = size_t(128) << 20, kNoAllocParts = size_t(8) << 20;
+static __device__ __align__(256) unsigned char scratch[kNoAllocBytes + kNoAllocParts];
 constexpr int kNoAllocDevices = 64;
 static std::mutex noalloc_mu;
 static unsigned char* noalloc_ptr[kNoAllocDevices];
@@ -3675,12 +3677,13 @@ int p4g_pc_apply_device_noalloc(p4g_Solver s, const double* d_r, double* d_z) {
         return o;
     };
     E.each_work([&](double*& p, long n) { if (p) room(n); });
+    const size_t vectors = off;
     room(2 * s->cx.npart_cap);
     room(2 * s->cx.npart_cap);
-    if (off > kNoAllocBytes)
+    if (vectors > kNoAllocBytes || off - vectors > kNoAllocParts)
         return set_error(PETSC_ERR_ARG_OUTOFRANGE,
                          "p4g_pc_apply_device_noalloc: this hierarchy's cycle needs %zu bytes of work arrays, more than "
-                         "the %zu MiB scratch (FP64 V(1,1) hierarchies up to 129^3 or 2049^2 fit)", off,
+                         "the %zu MiB scratch (FP64 V(1,1) hierarchies up to 129^3 or 2049^2 fit)", vectors,
                          kNoAllocBytes >> 20);
     unsigned char* base = nullptr;
     P4G_TRY(noalloc_scratch(&base));

@@ -91,3 +91,15 @@ def test_noalloc_refuses_unset_solver_and_oversize_hierarchy():
             assert rc == 63 and "more than the 128 MiB scratch" in capi.last_error()   # PETSC_ERR_ARG_OUTOFRANGE
         finally:
             L.p4g_device_free(d)
+
+
+def test_noalloc_takes_a_hierarchy_that_just_fits():
+    # 321x6017 with SOR smoothing: its vectors fill all but 0.1 MB of the
+    # 128 MiB, and its many blocks' partial sums do not count against them
+    L = capi.lib()
+    args = "-fsh_dim 2 -fsh_problem zero -da_grid_x 6 -da_grid_y 95 -da_refine 6 -pc_type mg -mg_levels_ksp_max_it 1"
+    print("noalloc full", args, flush=True)
+    with capi.Session(args) as s:
+        capi.check(L.p4g_solver_setup(s.solver))
+        r = np.random.default_rng(7).standard_normal(s.n)
+        assert np.array_equal(_run(L.p4g_pc_apply_device_noalloc, s.solver, r), _run(L.p4g_pc_apply_device, s.solver, r))
