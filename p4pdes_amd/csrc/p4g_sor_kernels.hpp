@@ -185,7 +185,11 @@ struct Sor2 {
     // soonest (264-271 ns one way against 330-494), in dispatch order.  A
     // launch takes 256 strips at most, a compute unit each, so that an XCD's
     // strips wait for lower ones on it or on a lower XCD only, also where
-    // several sweeps share the GPU.
+    // several sweeps share the GPU.  (Sweeps of up to 32 strips of several
+    // solvers meet on XCD 0; measured, an application at 1025^2, 16 strips, with
+    // 1 / 2 / 4 / 8 solvers at once: 1.98 / 2.05 / 4.08 / 6.3 ms, and at 257^2,
+    // where eight solvers' strips together have a compute unit each, 0.74 / 0.76 /
+    // 1.49 / 2.26: the queues set this, not the compute units.)
     static constexpr int NSTRIP = 32 * kXcds;
     __host__ __device__ static int block_of(int o) { return o * kXcds + (o >> 5); }
     __host__ __device__ static int blocks(int ns) { return block_of(ns - 1) + 1; }
@@ -642,11 +646,14 @@ k_sor9_pack(int mx, int my, int Tp, const double* __restrict__ g, T2<double>* __
 // before, and the planes of a step are independent chains that hide each
 // other's latency.  The wave's last plane goes to the next plane group by
 // step, tagged; its last row to the next strip as in 2D.  Bound by the
-// hand-over from group to group (257^3: 63 of them at 4.7 us each, in a sweep
-// of 393 us; a step is 0.22 us), so the words are asked for half a batch
-// before they are needed: four batches ahead, they were asked for too early
-// and a group settled four batches behind the one before (553 us a sweep).
-// Batches of 2 steps: 415 us.
+// hand-over from group to group (257^3: 63 of them at 5-6 us each, in sweeps
+// of 467 us forward and 402 us backward; a step is 0.22 us), so the words are
+// asked for half a batch before they are needed: four batches ahead, they were
+// asked for too early and a group settled four batches behind the one before
+// (sweeps run on their own over and over: 393 us, four batches ahead 553 us,
+// batches of 2 steps 415 us).  A level holds S, padded to whole strips and
+// steps, and every group's last plane besides the solver's vectors (257^3: 1.5
+// and 0.75 vectors).
 constexpr int kSor7Planes = 4;
 
 struct Sor7 {

@@ -7,7 +7,9 @@
 // levels from 0 up to the largest whose three vectors fit the LDS of one
 // compute unit (65^2 or 17^3 points in FP64) as one workgroup: every
 // neighbour read is an LDS access and every phase ends in a workgroup barrier
-// instead of a launch.  Bound by LDS bandwidth on its top level.
+// instead of a launch.  Bound by the instructions that one workgroup issues:
+// indices, masks and addresses of every point in every phase (129^2: 23 us,
+// of which the LDS bytes would take about 3).
 // Constant-coefficient levels with a Jacobi-preconditioned Chebyshev or
 // Richardson smoother; the formulas are those of the passes it stands for
 // (OpConst, OutCheb, OutResid, the Q1 transfers).

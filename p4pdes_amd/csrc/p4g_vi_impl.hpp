@@ -79,12 +79,14 @@ struct ViRun {
 
 static int asm_setup(p4g_solver_s* s, ViRun& R);
 
-// The coarsest level of a 27-plane operator, refactored at every Newton step:
-// band LU without pivoting (PETSc's serial coarse LU factors the diagonally
-// dominant Jacobians without row exchanges; of a symmetric positive definite
-// operator, spd, it is the Cholesky factor up to scaling), then the engine's
-// dense inverse.  Bands of 64 and more (long sides across x, 3D) are factored
-// as the set-up factors them, on the host.
+// The coarsest level of a 27-plane operator, inverted anew at every Newton
+// step without pivoting (PETSc's serial coarse LU factors the diagonally
+// dominant Jacobians without row exchanges, and its Cholesky needs none).
+// Bands below 64: by blocks on the device (k_blk_factor, k_blk_inverse), with
+// the band LU's pivots.  Wider ones (long sides along x, 3D) would not fit a
+// workgroup's registers: on the host, a symmetric positive definite operator
+// (spd) densely, as the set-up does, any other by band LU, whose inverse is
+// then formed on the device.
 static int coarse_factor_band(p4g_solver_s* s, const LevelInfo& L, const double* g27, bool spd, Engine<double>& e,
                               hipStream_t st) {
     const int n = (int)L.n;

@@ -646,7 +646,7 @@ SOR3_PAIRS = {
 @pytest.mark.parametrize("name", sorted(SOR3_PAIRS))
 def test_sor3_pipelined_matches_hyperplanes(name):
     # PETSc's default level smoother on 3D grids: the pipelined strip sweeps
-    # (k_sor7_strips) update every point from the same values in the same
+    # (k_sor7) update every point from the same values in the same
     # order as the hyperplane sweeps (k_sor_plane): the same solve bit for bit
     args = SOR3_PAIRS[name]
     print("sor3 pair", name, args, flush=True)
