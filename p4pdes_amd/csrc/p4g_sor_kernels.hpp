@@ -67,7 +67,13 @@ __device__ __forceinline__ void st_tagged(u64* lo, u64* hi, double v, unsigned t
 }
 
 // accesses through a buffer descriptor: past its bytes a load gives zero and
-// a store is dropped; voff per lane, soff uniform
+// a store is dropped; voff per lane, soff uniform.  16-byte stores take no
+// uniform register offset: a store of more than 8 bytes reads its data late,
+// and an instruction right behind it that writes one of its registers needs a
+// wait state between, which the compiler leaves out where the offset is in a
+// register.  With other kernels on the GPU such stores then stored the next
+// instruction's result (the low half of a sum, an error of 1e-9 in one of ten
+// applications with five solvers at once).
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, unsigned bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
 }
@@ -85,10 +91,10 @@ __device__ __forceinline__ T2<double> buffer_ld2(__amdgpu_buffer_rsrc_t b, unsig
     const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(b, (int)voff, (int)soff, 0);
     return T2<double>{dbl_of((int)v.x, (int)v.y), dbl_of((int)v.z, (int)v.w)};
 }
-__device__ __forceinline__ void buffer_st2(__amdgpu_buffer_rsrc_t b, unsigned voff, unsigned soff, double v0, double v1) {
+__device__ __forceinline__ void buffer_st2(__amdgpu_buffer_rsrc_t b, unsigned voff, double v0, double v1) {
     const long long p = __double_as_longlong(v0), q = __double_as_longlong(v1);
     __builtin_amdgcn_raw_buffer_store_b128(
-        u32x4{(unsigned)p, (unsigned)(p >> 32), (unsigned)q, (unsigned)(q >> 32)}, b, (int)voff, (int)soff, 0);
+        u32x4{(unsigned)p, (unsigned)(p >> 32), (unsigned)q, (unsigned)(q >> 32)}, b, (int)voff, 0, 0);
 }
 // the sweep's control words and the state of its waits (uniform)
 struct SorCtl {
@@ -312,6 +318,7 @@ __global__ void __launch_bounds__(Sor2<NINE>::NT) k_sor2(Sor2Args A) {
         double h1 = 0.0, u1 = 0.0, u2 = 0.0;    // own last result; the neighbour row's last two
         auto steps = [&](int k, int oslot, int part, const Ops& P) __attribute__((always_inline)) {
             char* const op = sor_lds + G::LO + oslot * G::OB + r * 16;
+            const unsigned vs = v16 + (k * SB + part * H) * 512u;
             f64x2 keep, kres;
 #pragma unroll
             for (int e = 0; e < H; ++e) {
@@ -349,7 +356,7 @@ __global__ void __launch_bounds__(Sor2<NINE>::NT) k_sor2(Sor2Args A) {
                 kres[e & 1] = res;
                 h1 = res;
                 if (e & 1) {
-                    if (!BWD) buffer_st2(Sr, v16 + (e / 2) * 1024u, (k * SB + part * H) * 512u, keep[0], keep[1]);
+                    if (!BWD) buffer_st2(Sr, vs + (e / 2) * 1024u, keep[0], keep[1]);
                     *(f64x2*)(op + (part * H + e) / 2 * G::VS) = kres;
                 }
             }
@@ -793,7 +800,7 @@ __global__ void __launch_bounds__(64) k_sor7(Sor7Args A) {
             }
 #pragma unroll
             for (int p = 0; p < K / 2; ++p)
-                buffer_st2(Sr, v16, (tf * (K / 2) + p) * 1024u, keep[2 * p], keep[2 * p + 1]);
+                buffer_st2(Sr, v16 + tf * (K / 2) * 1024u + p * 1024u, keep[2 * p], keep[2 * p + 1]);
             if (og < ng - 1) {
                 char* const p = zout + (long)t * 1024;
                 st_tagged((u64*)(p + v8), (u64*)(p + 512 + v8), xs[K - 1], tag);

@@ -7,6 +7,7 @@ of the batches of steps and of the plane groups, 35 strips (on two XCDs), 258
 (two launches), single interior points, 3D strips whose steps just fill 64 or
 128 or go one past, and boxes longer in each direction."""
 import ctypes
+import threading
 import time
 
 import numpy as np
@@ -191,3 +192,33 @@ def test_late_neighbour_is_awaited_to_the_limit(polls):
         t = time.perf_counter() - t
     assert rc == 76 and "pipelined SOR sweep stalled" in capi.last_error()
     assert t >= 0.3e-6 * polls
+
+
+def test_sweeps_of_several_solvers_at_once():
+    # solvers on threads of their own, each with its own stream and sweep
+    # arrays: 35 strips on two XCDs, 16 on one, 3D plane groups; every result
+    # is the one that the solver gives alone
+    args = ["-fsh_dim 2 -fsh_problem zero -da_grid_x 19 -da_grid_y 2200 -pc_mg_levels 1",
+            "-fsh_dim 2 -fsh_problem zero -da_refine 9", "-fsh_dim 2 -fsh_problem zero -da_refine 9",
+            "-fsh_dim 3 -fsh_problem zero -da_refine 6", "-fsh_dim 3 -fsh_problem zero -da_grid_x 5 -da_refine 5"]
+    sessions = [capi.Session(a + " -pc_type mg") for a in args]
+    bad = []
+    try:
+        rhs = [np.random.default_rng(i).standard_normal(s.n) for i, s in enumerate(sessions)]
+        alone = [capi.Solver(s).pc_apply(b) for s, b in zip(sessions, rhs)]
+
+        def work(i):
+            for _ in range(8):
+                if not np.array_equal(capi.Solver(sessions[i]).pc_apply(rhs[i]), alone[i]):
+                    bad.append(i)
+
+        print("sweeps at once", flush=True)
+        threads = [threading.Thread(target=work, args=(i,)) for i in range(len(sessions))]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    finally:
+        for s in sessions:
+            s.close()
+    assert not bad
