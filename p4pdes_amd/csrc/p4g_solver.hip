@@ -89,7 +89,10 @@ static double now_ms() {
 static bool device_room(size_t bytes, size_t rest, long free_mb) {
     size_t avail = 0, total = 0;
     if (free_mb >= 0) avail = (size_t)free_mb << 20;
-    else if (hipMemGetInfo(&avail, &total) != hipSuccess) return true;
+    else if (hipMemGetInfo(&avail, &total) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
     return avail >= bytes + rest;
 }
 
@@ -2763,8 +2766,7 @@ static void sor_splits(p4g_solver_s* s) {
     }
 }
 
-// the working arrays of level l's pipelined SOR sweeps (1D levels, and grids
-// without interior points, have none)
+// k_sor2's LDS, more than a kernel gets unasked
 template <bool NINE>
 static int sor2_lds() {
     HIP_TRY(hipFuncSetAttribute((const void*)&k_sor2<NINE, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -2816,8 +2818,9 @@ static int sor_pipes_check(p4g_solver_s* s, const char* who) {
     return 0;
 }
 
-// level l's sweep arrays; none (hyperplane sweeps) where they leave less than
-// `rest` bytes of device memory
+// the working arrays of level l's pipelined SOR sweeps; 1D levels and grids
+// without interior points have none, nor do levels (hyperplane sweeps) whose
+// arrays would leave less than `rest` bytes of device memory
 static int sor_pipe_alloc(p4g_solver_s* s, int l, SorKind kind, size_t rest) {
     LevelInfo& L = s->lv[l];
     if (L.dim < 2 || L.var || L.mx > (1 << 20) - 256) return 0;      // (a strip is addressed in 32 bits)
